@@ -266,7 +266,7 @@ int ae_write_synthetic_ae8(const char* path, uint64_t seed);
 #define AE_KERNEL_ATTENTION 2
 #define AE_KERNEL_GEMM_ATTN_OUT 3
 #define AE_KERNEL_LN1 4
-#define AE_KERNEL_GEMM_FFN_UP 5 /* the whole fused FFN block when a pass has >= 4096 tokens */
+#define AE_KERNEL_GEMM_FFN_UP 5 /* the whole fused FFN block when a pass has more than 1024 tokens */
 #define AE_KERNEL_GEMM_FFN_DOWN 6 /* unused (count 0) when the FFN block is fused */
 #define AE_KERNEL_LN2 7
 #define AE_KERNEL_LAYER11_TAIL 8
@@ -339,14 +339,14 @@ int ae_debug_set_ffn_rows(int rows);
 /* The fused FFN kernel's GELU, process-wide (a test hook, no reference
  * counterpart): 0 (the default) evaluates it with a fast approximation whose
  * distance from the reference's f32 GELU is certified on all 2^32 inputs and
- * recomputes exactly every value whose int8 quantization or row maximum that
- * distance leaves undecided; nonzero evaluates the reference's GELU on every
+ * evaluates exactly the values that decide a row maximum and every value whose
+ * int8 quantization that distance leaves undecided; nonzero evaluates the reference's GELU on every
  * element.  Both give the same bits. */
 int ae_debug_set_ffn_exact_gelu(int exact);
 /* Counters of the fast FFN kernel's exact recomputations on the current device
  * (a test hook): *tiles = 16-column tiles of 4 rows recomputed for an undecided
- * quantized value, *rows = passes of 32 rows that recomputed elements for a row
- * maximum; reset != 0 clears them after reading. */
+ * quantized value, *rows = groups of 16 rows in which a row maximum was settled
+ * among several exactly evaluated elements; reset != 0 clears them after reading. */
 int ae_debug_ffn_repairs(uint64_t* tiles, uint64_t* rows, int reset);
 /* The certification of the fused FFN kernel's fast GELU (a test hook,
  * synchronous, a few seconds): evaluates it and the reference's GELU on all

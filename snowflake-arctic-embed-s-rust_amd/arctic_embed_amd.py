@@ -511,8 +511,8 @@ def gelu_fast_certify():
 
 def ffn_repairs(reset=False):
     """(tiles, rows): the fast FFN kernel's exact recomputations on the current device since the
-    last reset: 16-column tiles recomputed for an undecided quantized value, and 32-row passes that
-    recomputed elements for a row maximum (a test hook)."""
+    last reset: 16-column tiles recomputed for an undecided quantized value, and groups of 16 rows in
+    which a row maximum was settled among several exactly evaluated elements (a test hook)."""
     t, r = ctypes.c_uint64(0), ctypes.c_uint64(0)
     _check(_lib.ae_debug_ffn_repairs(ctypes.byref(t), ctypes.byref(r), 1 if reset else 0))
     return int(t.value), int(r.value)

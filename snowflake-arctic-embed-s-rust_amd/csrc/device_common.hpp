@@ -268,6 +268,39 @@ __device__ __forceinline__ float gelu_fast(float v) {
   return __builtin_fmaf(-fabsf(v), ph * e, fmaxf(v, 0.0f));
 }
 
+// The same for N values at once, operation by operation (bit for bit gelu_fast):
+// a dependent VALU instruction issues about 10 cycles after its source, so a
+// wave beside one other on its SIMD needs several independent chains in flight;
+// the scheduling barriers keep the compiler from serializing them again (it
+// orders the values one after the other to save registers).
+// kc: 0.3275911f * 0.70710677f in a VGPR (its instruction takes |v|, so it cannot
+// hold the constant itself, and an f32 instruction that reads an SGPR issues at
+// half the rate).  The maximum by hand: fmaxf would canonicalize v first.
+template <int N>
+__device__ __forceinline__ void gelu_fast_n(const float (&v)[N], float kc, float (&out)[N]) {
+  constexpr float kA1 = 0.5f * 0.254829592f, kA2 = 0.5f * -0.284496736f, kA3 = 0.5f * 1.421413741f,
+                  kA4 = 0.5f * -1.453152027f, kA5 = 0.5f * 1.061405429f;
+  float t[N], a[N], ph[N], m[N];
+  auto each = [&](auto f) {
+#pragma unroll
+    for (int k = 0; k < N; k++) f(k);
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  each([&](int k) { t[k] = __builtin_fmaf(fabsf(v[k]), kc, 1.0f); });
+  each([&](int k) { a[k] = v[k] * (-0.5f * 1.44269504088896340736f); });
+  each([&](int k) { t[k] = __builtin_amdgcn_rcpf(t[k]); });
+  each([&](int k) { a[k] = v[k] * a[k]; });
+  each([&](int k) { a[k] = __builtin_amdgcn_exp2f(a[k]); });
+  each([&](int k) { ph[k] = __builtin_fmaf(kA5, t[k], kA4); });
+  each([&](int k) { ph[k] = __builtin_fmaf(ph[k], t[k], kA3); });
+  each([&](int k) { ph[k] = __builtin_fmaf(ph[k], t[k], kA2); });
+  each([&](int k) { ph[k] = __builtin_fmaf(ph[k], t[k], kA1); });
+  each([&](int k) { ph[k] = t[k] * ph[k]; });
+  each([&](int k) { asm("v_max_f32 %0, 0, %1" : "=v"(m[k]) : "v"(v[k])); });
+  each([&](int k) { ph[k] = ph[k] * a[k]; });
+  each([&](int k) { out[k] = __builtin_fmaf(-fabsf(v[k]), ph[k], m[k]); });
+}
+
 // Sequential sum of f(row[j]) over one 384-float LDS row (float4-aligned), in
 // index order: 12 batches of 8 float4, each read while the previous one is added.
 template <typename F>

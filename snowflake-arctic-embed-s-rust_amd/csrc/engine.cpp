@@ -343,11 +343,6 @@ struct KernelTimer {
   }
 };
 
-// The FFN block runs as one fused kernel (aek::launch_ffn) from this many token
-// rows on: its workgroups own 32 whole rows, one per CU, so below a few
-// thousand rows the split-K GEMM pair keeps more of the GPU busy.
-constexpr int kFfnFusedMinRows = 4096;
-
 static aek::FfnArgs ffn_args(const ae_linear& up, const ae_linear& down, int m, const int8_t* a, const float* a_scale,
                              const float* res, float* out) {
   aek::FfnArgs f{};
@@ -421,21 +416,6 @@ int run_forward(ae_workspace* ws, const uint16_t* ids, const int* cu, int B, int
     p.rowmax_init2 = rowmax_init2;
     return p;
   };
-  // an N = 384 GEMM and the LayerNorm of its output: one kernel for few rows
-  // (latency-bound), else the two kernels
-  auto gemm_then_ln = [&](int gemm_kind, int ln_kind, const GemmArgs& g, int amode, const LnArgs& l) {
-    if (gemm_fuses_ln(g, amode)) {
-      KernelTimer kt(ws, st, gemm_kind);
-      launch_gemm_ln(g, amode, l, st);
-      return;
-    }
-    {
-      KernelTimer kt(ws, st, gemm_kind);
-      launch_gemm(g, amode, kEpiF32, st);
-    }
-    KernelTimer kt(ws, st, ln_kind);
-    launch_ln_quant(l, kLnSrcF32, st);
-  };
   {  // embeddings + LayerNorm + SmoothQuant (src/model.rs:549-586)
     KernelTimer kt(ws, st, AE_KERNEL_EMBED_LN);
     LnArgs p{};
@@ -487,13 +467,17 @@ int run_forward(ae_workspace* ws, const uint16_t* ids, const int* cu, int B, int
   const bool small = gemm_small_path(T);
   const float* ln2_w = nullptr;  // small: the previous layer's LN2, applied by the next QKV prologue
   const float* ln2_b = nullptr;
-  // With the fused FFN (many rows), LN2 writes its (mean, rstd) per row instead
-  // of its f32 output: the next attention-output kernel, its only reader,
-  // recomputes that output from LN2's input rows (tmp) as LN2 forms it, and the
-  // [CLS] gather of layer 11 does so for its rows.  This saves LN2's f32 store
-  // (T x 1536 bytes per layer).  The last layer of a truncated pass
+  // Many rows (every other batch): the FFN block is one kernel (launch_ffn).  It
+  // starts where the few-row path ends because a launch takes 18 us with any
+  // number of 16-row workgroups up to one per CU, while the FFN-up and FFN-down
+  // GEMMs took 16 + 30 us at 1,280 rows and 18 + 30 at 3,776 (few workgroups,
+  // 24 dependent K steps each in FFN-down).  LN2 then writes its (mean, rstd) per
+  // row instead of its f32 output: the next attention-output kernel, its only
+  // reader, recomputes that output from LN2's input rows (tmp) as LN2 forms it,
+  // and the [CLS] gather of layer 11 does so for its rows.  This saves LN2's f32
+  // store (T x 1536 bytes per layer).  The last layer of a truncated pass
   // (stop_layers) still stores it: it is the state returned.
-  const bool ln2_stats = !small && T >= kFfnFusedMinRows;
+  const bool ln2_stats = !small;
   for (int l = 0; l < ae::kLayers - 1; l++) {  // src/model.rs:593-768
     if (stop_layers >= 0 && l >= stop_layers) break;
     const DevLayer& D = E->layers[l];
@@ -555,9 +539,11 @@ int run_forward(ae_workspace* ws, const uint16_t* ids, const int* cu, int B, int
         g.res_gamma = E->layers[l - 1].ln2_w;
         g.res_beta = E->layers[l - 1].ln2_b;
       }
-      gemm_then_ln(AE_KERNEL_GEMM_ATTN_OUT, AE_KERNEL_LN1, g, kAF32QSmooth,
-                   ln_args(ws->tmp, ws->hidden, D.ln1_w, D.ln1_b, D.ffn_inter.inv_smooth, ws->act_q, ws->act_scale,
-                           ws->rowmax_g, T));
+      KernelTimer kt(ws, st, AE_KERNEL_GEMM_ATTN_OUT);  // and LN1, in the same kernel
+      launch_gemm_ln(g, kAF32QSmooth,
+                     ln_args(ws->tmp, ws->hidden, D.ln1_w, D.ln1_b, D.ffn_inter.inv_smooth, ws->act_q, ws->act_scale,
+                             nullptr, T),
+                     st);
     }
     LnArgs ln2 = ln_args(ws->tmp, ws->hidden, D.ln2_w, D.ln2_b, E->layers[l + 1].qkv_smooth, ws->act_q,
                          ws->act_scale, ws->rowmax_ctx, T);
@@ -565,25 +551,13 @@ int run_forward(ae_workspace* ws, const uint16_t* ids, const int* cu, int B, int
       ln2.stats = ws->ln2_stats;
       if (!(stop_layers >= 0 && l + 1 == stop_layers)) ln2.dst = nullptr;
     }
-    if (T >= kFfnFusedMinRows) {  // FFN-up, GELU, quantize and FFN-down in one kernel
-      {
-        KernelTimer kt(ws, st, AE_KERNEL_GEMM_FFN_UP);
-        launch_ffn(ffn_args(D.ffn_inter, D.ffn_out, T, ws->act_q, ws->act_scale, ws->hidden, ws->tmp), st, ws->side,
-                   ws->fork_ev, ws->join_ev);
-      }
-      KernelTimer kt(ws, st, AE_KERNEL_LN2);
-      launch_ln_quant(ln2, kLnSrcF32, st);
-    } else {
-      {
-        KernelTimer kt(ws, st, AE_KERNEL_GEMM_FFN_UP);
-        gemm(D.ffn_inter, T, ws->act_q, kAI8, ws->act_scale, nullptr, nullptr, nullptr, ws->g, kEpiGelu,
-             D.ffn_out.inv_smooth, ws->rowmax_g);
-      }
-      gemm_then_ln(AE_KERNEL_GEMM_FFN_DOWN, AE_KERNEL_LN2,
-                   gemm_args(D.ffn_out, T, ws->g, nullptr, ws->rowmax_g, nullptr, ws->hidden, ws->tmp, nullptr,
-                             nullptr),
-                   kAF32Q, ln2);
+    {  // FFN-up, GELU, quantize and FFN-down in one kernel
+      KernelTimer kt(ws, st, AE_KERNEL_GEMM_FFN_UP);
+      launch_ffn(ffn_args(D.ffn_inter, D.ffn_out, T, ws->act_q, ws->act_scale, ws->hidden, ws->tmp), st, ws->side,
+                 ws->fork_ev, ws->join_ev);
     }
+    KernelTimer kt(ws, st, AE_KERNEL_LN2);
+    launch_ln_quant(ln2, kLnSrcF32, st);
   }
   if (stop_layers >= 0) {
     if (small && ln2_w) {  // the state after the last layer run: its LN2, as the next QKV would apply it

@@ -9,21 +9,48 @@
 // residual hidden); the arithmetic of each step is the one of gemm.hip's
 // kEpiGelu epilogue, the row quantizer and the kAF32Q epilogue.)
 //
-// One workgroup (8 waves) owns 32 complete token rows.  The row absmax of g is
-// therefore known inside the workgroup, and the [rows, 1536] intermediate never
-// leaves the CU: the GELU values overwrite the FFN-up accumulator registers in
-// place, their int8 quantization is written to LDS, and that LDS tile is the A
-// operand of the FFN-down MFMAs.  Compared with two GEMMs this removes the f32
-// intermediate's HBM round trip (12 bytes per element: f32 write, f32 read at
-// quantize-on-load) and the second GEMM's A-quantization work.
+// A workgroup of 8 waves owns 16 NR kP complete token rows, in kP passes of
+// 16 NR rows, so the [rows, 1536] intermediate never leaves the CU.  What its
+// registers hold of it is the pre-activation v: the row maximum of |g| needs v
+// only at a few candidates, and a value whose quantization the fast GELU leaves
+// undecided is recomputed from v on the spot.  Per pass:
 //
-// Wave w computes FFN-up columns [192w, 192w+192) for all 32 rows (2 x 12 tiles
-// of v_mfma_i32_16x16x64_i8, 96 accumulator VGPRs) and FFN-down columns
-// [48w, 48w+48) (2 x 3 tiles).  Weights are the pre-swizzled fragment order of
-// gemm.hip ([K/64][N/16][64 lanes][16 B]), streamed per wave from L2.
+//  1. FFN-up.  Wave w takes the 16-column blocks w, w + 8, .. (12 of them).
+//     The weights are the MFMA's A operand and the tokens its B operand, so a
+//     lane ends with four consecutive columns of one token: the row maxima, the
+//     row scales and the quantizer's factors are one register per 16 rows, and
+//     four quantized values are one dword of the int8 row.
+//  2. Row maxima, exactly, from a few candidates (below).
+//  3. GELU and quantization into the int8 row tile in LDS.
+//
+// FFN-down then streams W2 once for all rows of the workgroup; wave w computes
+// columns [48 w, 48 w + 48).
+//
+// What bounds it (s_memtime stamps of one 32-row pass, cycles at 2.4 GHz): FFN-up
+// 13 K (590 KB of W1 through the CU's 64 B/clk vector memory path; its 8 K of MFMA
+// and VALU work hide behind it), row maxima 7 K (two barriers and the scan), GELU
+// and quantization 16 K (VALU issue: 27 instructions per value, 83 cycles per
+// wave64 value), FFN-down 8 K per 32 rows (at 16 and 32 rows per workgroup the W2
+// stream).  MFMA and VALU work of different waves do not overlap on this part.
+// The code is kept to 27-48 KB: every workgroup runs most of it once, and at 72
+// or 98 KB (all loops unrolled) it fell out of the instruction cache between
+// workgroups (first round of 64-row workgroups 67 us instead of 54).
+// Measured against the kernel before it (32- and 64-row workgroups holding g in
+// place of v, the tokens as the A operand: row state in four registers per 16
+// rows, a byte transpose per dword, 22 cycles per value of top-element tracking,
+// 40 of quantization, and an undecided value recomputed from W1): 2,048 rows 26.9
+// -> 19.2 us (16-row workgroups), 8,192 rows 32.4 -> 29.2, 32,768 rows 112 -> 107,
+// 68,270 rows 247 -> 233, 294,912 rows 987 -> 900 us (same box).
+// Tried: 12 or 16 waves in one workgroup with FFN-down interleaved by chunks of
+// 192 or 256 columns (8 or 6 more barriers per tile: 20-25 % slower), FFN-up
+// computed twice instead of holding v (152 us at 32,768 rows), the FFN-up and
+// GELU loops rolled too (indexed register moves; 12 % slower at 2,048 rows).
+//
+// Weights are the pre-swizzled fragment order of gemm.hip ([K/64][N/16][64
+// lanes][16 B]), streamed per wave from L2.
 #include <hip/hip_runtime.h>
 
-#include <type_traits>
+#include <algorithm>
 
 #include "device_common.hpp"
 #include "kernels.hpp"
@@ -32,24 +59,17 @@ namespace aek {
 
 namespace {
 constexpr int kH = 384, kF = 1536;
-constexpr int kRows = 32;                 // token rows per workgroup
-constexpr int kWaves = 8;
+constexpr int kWaves = 8, kThreads = 64 * kWaves;
 constexpr int kAPitch = kH + 16;          // LDS row pitch of the input tile (bytes)
 constexpr int kQPitch = kF + 16;          // LDS row pitch of the quantized intermediate (bytes)
 constexpr int kUpCB = kF / 16 / kWaves;   // FFN-up 16-column blocks per wave (12)
 constexpr int kDnCB = kH / 16 / kWaves;   // FFN-down 16-column blocks per wave (3)
-constexpr int kEPitch = kDnCB * 16 + 4;   // per-wave epilogue staging row pitch (words)
 constexpr int kRing = 8;                  // FFN-down K steps of weight fragments in flight
 constexpr int kUpSteps = kH / 64, kDnSteps = kF / 64;
 
-// 4 x 4 byte transpose over the lanes of a quad: lane k holds byte r = M[r][k]
-// (a column); afterwards it holds byte c = M[k][c] (a row).  Two exchanges
-// (lane k^1, then k^2), each followed by one byte select (v_perm_b32: selector
-// values 0-3 pick bytes of the second operand, 4-7 of the first).
-__device__ __forceinline__ uint32_t quad_transpose_bytes(uint32_t v, int k) {
-  const uint32_t w = __builtin_amdgcn_perm(dpp<kDppXor1>(v), v, (k & 1) ? 0x03070105u : 0x06020400u);
-  return __builtin_amdgcn_perm(dpp<kDppXor2>(w), w, (k & 2) ? 0x03020706u : 0x05040100u);
-}
+typedef float v12f __attribute__((ext_vector_type(12)));
+typedef float v4f __attribute__((ext_vector_type(4)));
+
 // a raw buffer resource over `bytes` bytes of weights (gfx9 descriptor word 3:
 // 32-bit data format) and a 16-byte load at a vector plus scalar byte offset
 __device__ __forceinline__ __amdgpu_buffer_rsrc_t weight_rsrc(const int8_t* base, int bytes) {
@@ -58,512 +78,428 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t weight_rsrc(const int8_t* base
 __device__ __forceinline__ v4i weight_load(__amdgpu_buffer_rsrc_t r, uint32_t voff, int soff) {
   return __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(r, voff, soff, 0));
 }
+// lanes of a wave mask below this one
+__device__ __forceinline__ int lanes_below(uint64_t mask) {
+  return (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(mask >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)mask, 0));
+}
 }  // namespace
 
 // Bounds of the fast path (kFast), from gelu_fast's certified bound
-// |G - G'| <= kGeluFastRel |G'| + kGeluFastAbs (device_common.hpp).  With
-// g = RN(G gs) and g' = RN(G' gs) (u = 2^-24 the unit roundoff):
-//   |g - g'| <= (kGeluFastRel + 2u)(1 + u)^2 |g'| + |gs| kGeluFastAbs (1 + u) + 2^-148
-//            <= kUpRel |g'| + k0,   k0 = kGeluFastAbs' gs_max + 2^-140,
-// gs_max = max |gs| over the lane's 12 columns.  hi(a) = fma(a, 1 + 2 kUpRel, k0)
-// is then an upper bound of |g| for any element with |g'| <= a (also covering
-// the fma's rounding).  For the quantization x = RN(g inv) against
-// x' = RN(g' inv):  |x - x'| <= (kUpRel + 2^-22) |x'| + k0 inv (1 + 2^-22) +
-// tiny; with the computed distance of |x'| to the nearest half-integer (exact
-// but for 2^-26 below 0.25) the decision threshold is
-//   th = fma(|x'|, kQRel, th0),  th0 = fma(k0 (1 + 2^-20), inv, 2^-25),
-// and x and x' round to the same int8 value whenever dist > th.
-constexpr float kUpRel = 0x1.5p-21f;             // >= (2^-21 + 2^-23)(1 + 2^-24)^2
-constexpr float kHiMul = 1.0f + 2.0f * kUpRel;
-constexpr float kAbsGs = 0x1.65p-24f;            // >= kGeluFastAbs (1 + 2^-24), rounded up
-constexpr float kQRel = 0x1.ep-21f;              // >= (kUpRel + 2^-22)(1 + 2^-20)
-constexpr float kK0Inv = 1.0f + 0x1p-20f;
+// |G - G'| <= kGeluFastRel |G'| + kGeluFastAbs (device_common.hpp), u = 2^-24 the
+// unit roundoff.  The reference quantizes x = RN(RN(G gs) inv), the kernel
+// x' = RN(G' RN(gs inv)); two roundings on either side give
+//   |x - x'| <= (kGeluFastRel + 4u)(1 + 2^-20) |x'| + kGeluFastAbs gs_max inv (1 + 2^-20) + tiny,
+// gs_max = max |gs| over all columns.  x' and x round to the same int8 value when
+// x' is farther than that from every half-integer, i.e. when
+//   |x' - round(x')| + kQRel |x'| < 0.5 - (kGeluFastAbs gs_max inv (1 + 2^-20) + 2^-24)
+// (the distance is exact; 2^-24 covers the rounding of the sums).
+constexpr float kQRel = 0x1.ep-21f;    // >= (2^-21 + 2^-22)(1 + 2^-20)
+constexpr float kQAbs = 0x1.65p-24f;   // >= kGeluFastAbs (1 + 2^-20)
+// |GELU(v)| <= max(kCapMul v - kCapSub, kCapMin) for every v: a line just above
+// the tangent at v = 2, and a constant above |GELU| to its left.  Below 0.25,
+// |GELU(v)| <= max(v, 0.17) < kCapMin; from 8 on, GELU(v) <= v is below the line;
+// the floats in between are enumerated by test_ffn_gelu_cap_on_every_float.  The
+// row maxima use the bound times |gs| (rounding is monotonic, so |g| <= it).
+constexpr float kCapMul = 1.0854f, kCapSub = 0.2158f, kCapMin = 0.44f;
+// the share of a row's largest bound from which an element is a candidate for
+// its maximum: GELU(v) exceeds that share of the bound for every v from 0.57 on
+// (it falls to 1 / kCapMul = 0.9213 for large v)
+constexpr float kCandShare = 0.92f;
 
-// repair counters (test hook ae_debug_ffn_repairs): [0] column tiles of 4 rows
-// recomputed exactly because a quantized value was undecided, [1] passes whose
-// row maxima needed more than each lane's top element
+// repair counters (test hook ae_debug_ffn_repairs): [0] 16-row x 16-column tiles
+// recomputed exactly because a quantized value was undecided, [1] groups of 16
+// rows in which a row maximum was settled among several exact values
 __device__ unsigned long long g_ffn_repairs[2];
 
-// kP passes of 32 rows per workgroup (kP = 2: 64 rows): each pass runs FFN-up,
-// its GELU, the row absmax and the quantization into rows [32 pp, 32 pp + 32) of
-// the LDS intermediate; FFN-down then streams W2 once for all 32 kP rows (590 KB
-// per workgroup through the CU's vector memory path, the phase's bound).  Pass
-// pp + 1's input rows are staged with pass pp's, and its first weight fragments
-// are loaded after pass pp's GELU loop.
+// kFast: the GELU is gelu_fast with exact repair (the same bits as the exact
+// kernel, kFast = false, whose registers hold g = GELU(v) gs in place of v).
 //
-// kFast: the GELU of the FFN-up epilogue is gelu_fast, and exactness is
-// restored where the int8 output can depend on it:
-//  * row maxima: each lane keeps, per row, its two largest |g'| (as keys with
-//    the column block in the low 4 bits, so the top one's column is known) and
-//    the top one's pre-activation; the top one is evaluated exactly
-//    (gelu_exact, skipped when every lane's top is in the GELU's exact
-//    saturated ranges), and the maximum of those is the row maximum whenever no
-//    lane's second value can reach it (hi(second) < max).  Otherwise (rare: a
-//    near tie inside one lane) every element whose hi reaches the maximum is
-//    recomputed exactly and folded in;
-//  * quantization: q = round(g' inv) where |x'| is farther than th from every
-//    half-integer; otherwise the wave recomputes that 16-column tile exactly
-//    (rows' int8 inputs still in LDS . the column of W1, int32 dot products,
-//    then the reference's epilogue and gelu_exact) and overwrites its bytes.
-// The result is bit-identical to the exact kernel.
-template <int kP, bool kFast>
-__global__ __launch_bounds__(512, 2) void ffn_fused_kernel(FfnArgs p) {
-  constexpr int kT = kRows * kP;  // token rows per workgroup
-  __shared__ __attribute__((aligned(16))) int8_t sA[kP][kRows * kAPitch];
-  __shared__ __attribute__((aligned(16))) int8_t sQ[kT * kQPitch];
-  __shared__ __attribute__((aligned(16))) float sMax[kT][kWaves];  // per-wave row absmax of g
-  // kFast: per-wave upper bound (f32 bits) of |g| over the row's elements other than each lane's top one
-  __shared__ __attribute__((aligned(16))) uint32_t sU[kFast ? kT : 1][kWaves];
-  // kFast: row maxima of the rare recomputation (f32 bits; zero unless it ran).  A
-  // separate array: sMax and sU stay unchanged after a pass's barrier, so every
-  // wave reads the same values when it decides whether the recomputation (and
-  // its barrier) runs
-  __shared__ uint32_t sMax2[kFast ? kT : 1];
+// Row maxima (kFast): FFN-up keeps, per lane, row and column block, the largest
+// bound B = max(kCapMul v - kCapSub, kCapMin) |gs| of its four columns, and from
+// those U, the row's largest.  Every element whose bound reaches kCandShare U,
+// the top one among them, is evaluated exactly; the largest, M1, is the row
+// maximum if M1 >= kCandShare U, because no other element can exceed that.
+// Otherwise (rows whose largest v is below 0.57) a second scan evaluates every
+// element whose bound reaches M1.  The candidates of a wave (a few) go to a list
+// in LDS first, so that one gelu_exact serves them all.
+template <int NR, int kP, bool kFast>
+__global__ __launch_bounds__(kThreads, 2) void ffn_kernel(FfnArgs p) {
+  constexpr int RP = 16 * NR, R = RP * kP;  // token rows per pass and per workgroup
+  __shared__ __attribute__((aligned(16))) int8_t sA[R * kAPitch];
+  // the quantized intermediate; before a pass's quantization its rows hold the waves' candidate lists
+  __shared__ __attribute__((aligned(16))) int8_t sQ[R * kQPitch];
+  constexpr int kListCap = RP * kQPitch / kWaves / 8;  // (v, column | row << 16) per wave
+  __shared__ __attribute__((aligned(16))) float sWs[kF], sB[kF], sGs[kF];
+  __shared__ __attribute__((aligned(16))) float sU[R][kWaves];  // per-wave row maxima of the bound (exact kernel: of |g|)
+  __shared__ float sSa[R], sMax[R];
+  __shared__ uint32_t sM[2][R];  // row maxima of |g| over the first scan's elements and the second's (f32 bits)
+  __shared__ int sCnt[kP], s_full[kP];  // candidates of a pass's first scan; a wave's exceeded its list
+  __shared__ uint32_t s_gmax;
   __shared__ uint64_t s_tab[32];
-  // the FFN-down epilogue's per-wave staging tiles (kRows rows at a time): their
-  // own array at kP = 1, the intermediate's space at kP = 2 (free once FFN-down
-  // has read it; 53 KB of 99 KB)
-  constexpr int kEWords = kRows * kEPitch;
-  __shared__ __attribute__((aligned(16))) int sE1[kP == 1 ? kWaves * kEWords : 4];
-  static_assert(kP == 1 || (size_t)kWaves * kEWords * 4 <= sizeof(sQ), "staging fits the intermediate");
-  // (wave via readfirstlane: known uniform, so the weight fragments' offsets are
-  // scalars; as a vector value the 72 offsets of a pass sat in VGPRs all kernel long)
-  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int fr = lane & 15, fq = lane >> 4;  // MFMA: operand row / output column; k group / output row quad
-  const int m0 = blockIdx.x * kT;
+  // (wave via readfirstlane: known uniform, so the weight fragments' offsets are scalars)
+  int tid = threadIdx.x;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  int lane = tid & 63, fr = lane & 15, fq = lane >> 4;  // fr: token of the 16-row block, fq: k group and column quad
+  const int m0 = blockIdx.x * R;
 
-  // input tiles: kP x 32 rows x 384 int8 (rows past M repeat row M-1; never stored)
-  for (int c = tid; c < kT * (kH / 16); c += 512) {
-    const int row = c / (kH / 16), c16 = c - row * (kH / 16);
-    const int grow = min(m0 + row, p.M - 1);
-    *reinterpret_cast<v4i*>(&sA[row / kRows][(row % kRows) * kAPitch + c16 * 16]) =
-        __builtin_nontemporal_load(reinterpret_cast<const v4i*>(p.A + (size_t)grow * kH + c16 * 16));
-  }
-  exp_tab_fill(s_tab, tid);  // ordered before the GELUs by the input tiles' barrier
-
-  // ---- FFN-up and its GELU epilogue, software-pipelined by column block ----
-  // acc[i][j] = rows 16i.., columns (cb1 + j)*16..  Column block j is finished
-  // (all six K steps) one iteration before its GELU, and its weight fragments
-  // are loaded two iterations before that, so the matrix cores and the weight
-  // stream of block j + 1 run while the VALU evaluates the GELUs of block j.
-  // Weight fragments through buffer resources: the fragment's offset is a scalar
-  // (wave-uniform) and the lane's 16 bytes one VGPR shared by every load, so the
-  // loads hold no 64-bit vector addresses (the 64-row fast kernel spilled them).
-  const int cb1 = wave * kUpCB;
-  const __amdgpu_buffer_rsrc_t w1r = weight_rsrc(p.w1, kF * kH);
+  // weight fragments through buffer resources: the fragment's offset is a scalar
+  // and the lane's 16 bytes one VGPR shared by every load.  Opaque copies of the
+  // bases: the offsets are formed next to their loads, not hoisted and held
+  const __amdgpu_buffer_rsrc_t w1r = weight_rsrc(p.w1, kF * kH), w2r = weight_rsrc(p.w2, kF * kH);
   const uint32_t lane16 = (uint32_t)lane * 16u;
-  auto load_col = [&](int j, v4i* dst) {  // the six K steps of column block j
-    // an opaque copy of the base per call: the offsets are formed next to their
-    // loads (scalar adds), not all hoisted and held in SGPRs (which spilled)
-    int base = (cb1 + j) * 1024;
+
+  // input rows (rows past M repeat row M-1; never stored)
+  constexpr int kLd = (R * (kH / 16) + kThreads - 1) / kThreads;
+  v4i an[kLd];
+#pragma unroll
+  for (int i = 0; i < kLd; i++) {
+    const int c = min(tid + kThreads * i, R * (kH / 16) - 1), row = c / (kH / 16), c16 = c - row * (kH / 16);
+    an[i] = __builtin_nontemporal_load(reinterpret_cast<const v4i*>(p.A + (size_t)min(m0 + row, p.M - 1) * kH + c16 * 16));
+  }
+  v4i w1[2][kUpSteps];  // column blocks j and j + 1
+  auto load_w1 = [&](int j, v4i (&dst)[kUpSteps]) {
+    int base = (j * kWaves + wave) * 1024;
     asm volatile("" : "+s"(base));
 #pragma unroll
     for (int kt = 0; kt < kUpSteps; kt++) dst[kt] = weight_load(w1r, lane16, base + kt * (kF / 16) * 1024);
   };
-  v4i acc[2][kUpCB];
-  v4i bq[2][kUpSteps];  // fragments of column blocks j + 1 (then j + 3) and j + 2
-  load_col(0, bq[0]);
-  load_col(1, bq[1]);
-  const ExpTabLds tb{s_tab};  // wave-uniform from here to the end of the GELU loops
-  auto row_absmax = [&](int row) {
-    const float4 a = *reinterpret_cast<const float4*>(&sMax[row][0]);
-    const float4 b = *reinterpret_cast<const float4*>(&sMax[row][4]);
-    return fmaxf(fmaxf(fmaxf(a.x, a.y), fmaxf(a.z, a.w)), fmaxf(fmaxf(b.x, b.y), fmaxf(b.z, b.w)));
-  };
-  // this lane's row scales (rows 16i + 4fq + r of a pass), the next pass's loaded
-  // at the end of this pass's GELU loop
-  float sa[2][4], sa_next[2][4];
-  auto load_sa = [&](int r0, float (&dst)[2][4]) {
+  load_w1(0, w1[0]);
+  load_w1(1, w1[1]);
+  // the column operands
+  float gmx = 0.0f;
+  for (int c = tid; c < kF / 4; c += kThreads) {
+    reinterpret_cast<float4*>(sWs)[c] = reinterpret_cast<const float4*>(p.w1_scale)[c];
+    reinterpret_cast<float4*>(sB)[c] = reinterpret_cast<const float4*>(p.b1)[c];
+    const float4 g = reinterpret_cast<const float4*>(p.g_smooth)[c];
+    reinterpret_cast<float4*>(sGs)[c] = g;
+    gmx = fmaxf(fmaxf(fmaxf(gmx, fabsf(g.x)), fmaxf(fabsf(g.y), fabsf(g.z))), fabsf(g.w));
+  }
+  if (tid < R) {
+    sSa[tid] = p.a_scale[min(m0 + tid, p.M - 1)];
+    sM[0][tid] = __float_as_uint(1e-8f);
+    sM[1][tid] = 0u;
+  }
+  if (tid < kP) sCnt[tid] = 0, s_full[tid] = 0;
+  if (tid == 0) s_gmax = 0u;
+  exp_tab_fill(s_tab, tid);
 #pragma unroll
-    for (int i = 0; i < 2; i++)
-#pragma unroll
-      for (int r = 0; r < 4; r++) dst[i][r] = p.a_scale[min(m0 + r0 + i * 16 + fq * 4 + r, p.M - 1)];
-  };
-  load_sa(0, sa);
-  if constexpr (kFast)
-    for (int t = tid; t < kT; t += 512) sMax2[t] = 0u;
-  __syncthreads();  // the input tiles are in LDS
-#pragma unroll
-  for (int pp = 0; pp < kP; pp++) {
-    const int8_t* sAp = sA[pp];
-    const int r0 = kRows * pp;  // this pass's first row in the tile
-    // the per-column operands are loaded again in every pass: opaque copies of
-    // their pointers keep the compiler from hoisting the 36 loads out of the
-    // pass loop (and holding 36 more registers through the GELUs)
-    const float *w1s = p.w1_scale, *b1 = p.b1, *gsm = p.g_smooth;
-    if constexpr (kP > 1) asm volatile("" : "+s"(w1s), "+s"(b1), "+s"(gsm));
-    auto mma_col = [&](int j, const v4i* bf) {
-#pragma unroll
-      for (int i = 0; i < 2; i++) acc[i][j] = v4i{0, 0, 0, 0};
-#pragma unroll
-      for (int kt = 0; kt < kUpSteps; kt++) {
-        v4i af[2];
-#pragma unroll
-        for (int i = 0; i < 2; i++)
-          af[i] = *reinterpret_cast<const v4i*>(&sAp[(i * 16 + fr) * kAPitch + kt * 64 + fq * 16]);
-#pragma unroll
-        for (int i = 0; i < 2; i++) acc[i][j] = __builtin_amdgcn_mfma_i32_16x16x64_i8(af[i], bf[kt], acc[i][j], 0, 0, 0);
-      }
-    };
-    // kFast: the exact g of this lane's rows 16i + 4fq + r (r < 4) of column (cb1 + j)*16 + fr:
-    // the 16 x 16 FFN-up tile recomputed by its six MFMAs (A fragments from the pass's int8 input
-    // tile in LDS, W1 fragments in one round trip from L2; the same int32 sums as in the pass),
-    // then the reference's epilogue and gelu_exact.  Wave-uniform (i, j).
-    auto exact_tile = [&](int i, int j, float (&g)[4], auto serial) {
-      v4i wf[kUpSteps];
-      load_col(j, wf);
-      v4i t = v4i{0, 0, 0, 0};
-#pragma unroll
-      for (int kt = 0; kt < kUpSteps; kt++) {
-        const v4i af = *reinterpret_cast<const v4i*>(&sAp[(i * 16 + fr) * kAPitch + kt * 64 + fq * 16]);
-        t = __builtin_amdgcn_mfma_i32_16x16x64_i8(af, wf[kt], t, 0, 0, 0);
-      }
-      const int col = (cb1 + j) * 16 + fr;
-      const float ws = w1s[col], bb = b1[col], gs = gsm[col];
-#pragma unroll
-      for (int r = 0; r < 4; r++) {
-        const float sar = i ? sa[1][r] : sa[0][r];
-        g[r] = gelu_exact(fmaf((float)t[r], sar * ws, bb), tb) * gs;
-        // where registers are short (beside the pass's 96 values), one exact GELU at a time;
-        // else the four chains overlap (the repair is latency-bound)
-        if constexpr (decltype(serial)::value) asm volatile("" : "+v"(g[r]));
-      }
-    };
-    mma_col(0, bq[0]);
-    load_col(2, bq[0]);
+  for (int i = 0; i < kLd; i++) {
+    const int c = tid + kThreads * i, row = c / (kH / 16), c16 = c - row * (kH / 16);
+    if (R * (kH / 16) % kThreads == 0 || c < R * (kH / 16)) *reinterpret_cast<v4i*>(&sA[row * kAPitch + c16 * 16]) = an[i];
+  }
+  __syncthreads();
+  if constexpr (kFast) {
+    gmx = row16_max(gmx);
+    if (fr == 0) atomicMax(&s_gmax, __float_as_uint(gmx));  // read after the first row-maximum barrier
+  }
+  const ExpTabLds tb{s_tab};
+  // (constants that an f32 instruction would otherwise read from an SGPR, at half its rate)
+  float kc = 0.3275911f * 0.70710677f, kcap = kCapMul, kq = kQRel;
+  asm volatile("" : "+v"(kc), "+v"(kcap), "+v"(kq));
+  // opaque per phase: addresses formed from them are not kept from one phase to the next (spills)
+  auto opaque_ids = [&]() { asm volatile("" : "+v"(tid), "+v"(lane), "+v"(fr), "+v"(fq)); };
 
-    // GELU epilogue: g = GELU(fma(f32(acc), sa*ws, b)) * inv_smooth, in place.
-    // This lane holds rows r0 + 16i + 4fq + r (i < 2, r < 4) of column (cb1 + j)*16 + fr.
-    float mx[2][4];
-    uint32_t t1[2][4], t2[2][4];  // kFast: the two largest keys (|g'| bits, low 4 bits = j) per row
-    float vt[2][4];               // kFast: the pre-activation of the t1 element
-    float gs_max = 0.0f;          // kFast: max |inv_smooth| over this lane's columns
+#pragma unroll 1
+  for (int pp = 0; pp < kP; pp++) {
+    const int r0 = RP * pp;  // this pass's first row in the tile
+    opaque_ids();
+    float sa[NR];
 #pragma unroll
-    for (int i = 0; i < 2; i++)
+    for (int i = 0; i < NR; i++) sa[i] = sSa[r0 + i * 16 + fr];
+
+    // ---- FFN-up: v = fma(f32(acc), sa * ws, b) and its bound ----
+    // (vectors over the column blocks: the scans index them in rolled loops)
+    v12f v[NR][4], bm[NR];
+    float mx[NR];
 #pragma unroll
-      for (int r = 0; r < 4; r++) {
-        mx[i][r] = 1e-8f;  // max_abs starts at 1e-8 (src/simd_math.rs:1295-1312)
-        t1[i][r] = t2[i][r] = 0u;
-        vt[i][r] = 0.0f;
+    for (int i = 0; i < NR; i++) mx[i] = 0.0f;
+#pragma unroll
+    for (int j = 0; j < kUpCB; j++) {
+      const int col = (j * kWaves + wave) * 16 + fq * 4;  // this lane's four columns
+      v4i acc[NR];
+#pragma unroll
+      for (int i = 0; i < NR; i++) acc[i] = v4i{0, 0, 0, 0};
+#pragma unroll
+      for (int kt = 0; kt < kUpSteps; kt++)
+#pragma unroll
+        for (int i = 0; i < NR; i++) {
+          const v4i t = *reinterpret_cast<const v4i*>(&sA[(r0 + i * 16 + fr) * kAPitch + kt * 64 + fq * 16]);
+          acc[i] = __builtin_amdgcn_mfma_i32_16x16x64_i8(w1[j & 1][kt], t, acc[i], 0, 0, 0);
+        }
+      if (j + 2 < kUpCB) load_w1(j + 2, w1[j & 1]);
+      const v4f ws = *reinterpret_cast<const v4f*>(&sWs[col]);
+      const v4f bb = *reinterpret_cast<const v4f*>(&sB[col]);
+      const v4f gs = *reinterpret_cast<const v4f*>(&sGs[col]);
+      const float cap0 = kCapMin * fmaxf(fmaxf(fabsf(gs[0]), fabsf(gs[1])), fmaxf(fabsf(gs[2]), fabsf(gs[3])));
+#pragma unroll
+      for (int i = 0; i < NR; i++) {
+        float u[4];
+#pragma unroll
+        for (int r = 0; r < 4; r++) {
+          float x = fmaf((float)acc[i][r], sa[i] * ws[r], bb[r]);
+          if constexpr (kFast) {
+            // in program order: else the int32 sums of later blocks are held beside their operands
+            asm volatile("" : "+v"(x));
+            v[i][r][j] = x;
+            u[r] = fmaf(x, kcap, -kCapSub) * fabsf(gs[r]);
+          } else {
+            x = gelu_exact(x, tb) * gs[r];
+            asm volatile("" : "+v"(x));
+            v[i][r][j] = x;
+            u[r] = fabsf(x);
+          }
+        }
+        // (ignores a NaN, as `if a > max_abs`)
+        float m = fmaxf(fmaxf(fmaxf(kFast ? cap0 : 0.0f, u[0]), fmaxf(u[1], u[2])), u[3]);
+        asm volatile("" : "+v"(m));
+        bm[i][j] = m;
+        mx[i] = fmaxf(mx[i], m);
       }
-    // the column operands (w1_scale, b1, inv_smooth) one block ahead: block
-    // j + 1's are issued at the top of block j, ahead of its weight loads, so
-    // that the GELU of a block does not wait for its own operand loads
-    float cop[3];
-    auto load_cop = [&](int j) {
-      const int col = (cb1 + j) * 16 + fr;
-      cop[0] = w1s[col];
-      cop[1] = b1[col];
-      cop[2] = gsm[col];
-    };
-    load_cop(0);
+    }
+    opaque_ids();
+    // ---- row maxima: over this wave's columns, then over the waves through LDS ----
+#pragma unroll
+    for (int i = 0; i < NR; i++) {
+      mx[i] = fmaxf(mx[i], __shfl_xor(mx[i], 16, 64));
+      mx[i] = fmaxf(mx[i], __shfl_xor(mx[i], 32, 64));
+      if (fq == 0) sU[r0 + i * 16 + fr][wave] = mx[i];
+    }
+    __syncthreads();
+    float M[NR], thr[NR];
+#pragma unroll
+    for (int i = 0; i < NR; i++) {
+      const float4* u4 = reinterpret_cast<const float4*>(&sU[r0 + i * 16 + fr][0]);
+      const float4 a = u4[0], b = u4[1];
+      const float U = fmaxf(fmaxf(fmaxf(a.x, a.y), fmaxf(a.z, a.w)), fmaxf(fmaxf(b.x, b.y), fmaxf(b.z, b.w)));
+      M[i] = fmaxf(U, 1e-8f);  // max_abs starts at 1e-8 (src/simd_math.rs:1295-1312)
+      thr[i] = kCandShare * U;
+    }
+    float gs_max = 0.0f;
+    if constexpr (kFast) {
+      gs_max = __uint_as_float(s_gmax);
+      {  // first scan: candidates to the wave's list, then one gelu_exact for up to 64 of them
+        // (two arrays: as pairs, every v would sit in a register pair of its own)
+        float* lv = reinterpret_cast<float*>(sQ + r0 * kQPitch) + wave * 2 * kListCap;
+        uint32_t* lid = reinterpret_cast<uint32_t*>(lv) + kListCap;
+        int n = 0;  // (wave-uniform)
+        bool full = false;
+#pragma unroll 1
+        for (int j = 0; j < kUpCB; j++) {
+          const int col = (j * kWaves + wave) * 16 + fq * 4;
+#pragma unroll
+          for (int i = 0; i < NR; i++) {
+            if (__builtin_amdgcn_ballot_w64(bm[i][j] >= thr[i]) == 0) continue;  // wave-uniform
+            const v4f gs = *reinterpret_cast<const v4f*>(&sGs[col]);
+#pragma unroll
+            for (int r = 0; r < 4; r++) {
+              const float x = v[i][r][j];
+              const bool c = fmaxf(fmaf(x, kcap, -kCapSub), kCapMin) * fabsf(gs[r]) >= thr[i];
+              const uint64_t m = __builtin_amdgcn_ballot_w64(c);
+              if (m == 0) continue;
+              if (n + __builtin_popcountll(m) <= kListCap) {
+                if (c) {
+                  const int k = n + lanes_below(m);
+                  lv[k] = x;
+                  lid[k] = (uint32_t)(col + r) | (uint32_t)(r0 + i * 16 + fr) << 16;
+                }
+                n += __builtin_popcountll(m);
+              } else {
+                full = true;
+              }
+            }
+          }
+        }
+        wave_lds_sync();
+        for (int k = 0; k < n; k += 64) {
+          const int e = min(k + lane, n - 1);
+          const uint32_t id = lid[e];
+          const float g = fabsf(gelu_exact(lv[e], tb) * sGs[id & 0xffffu]);
+          if (k + lane < n && g > 0.0f) atomicMax(&sM[0][id >> 16], __float_as_uint(g));  // a NaN is ignored
+        }
+        if (lane == 0) {
+          if (n > 0) atomicAdd(&sCnt[pp], n);
+          if (full) s_full[pp] = 1;
+        }
+      }
+      __syncthreads();
+      bool open = s_full[pp] != 0;  // the same in every wave: each reads all rows' U and M1, which no longer change
+#pragma unroll
+      for (int i = 0; i < NR; i++) {
+        M[i] = __uint_as_float(sM[0][r0 + i * 16 + fr]);
+        open = open || !(M[i] >= thr[i] * (1.0f + 0x1p-20f));
+      }
+      if (__builtin_amdgcn_ballot_w64(open) != 0) {  // second scan
+#pragma unroll 1
+        for (int j = 0; j < kUpCB; j++) {
+          const int col = (j * kWaves + wave) * 16 + fq * 4;
+#pragma unroll
+          for (int i = 0; i < NR; i++) {
+            if (__builtin_amdgcn_ballot_w64(bm[i][j] >= M[i]) == 0) continue;
+            v4f x = v4f{v[i][0][j], v[i][1][j], v[i][2][j], v[i][3][j]}, g = *reinterpret_cast<const v4f*>(&sGs[col]);
+            float top = 0.0f;
+#pragma unroll 1
+            for (int r = 0; r < 4; r++) {  // element 0 evaluated, then the four rotated
+              top = nanless_max(top, fabsf(gelu_exact(x[0], tb) * g[0]));
+              x = v4f{x[1], x[2], x[3], x[0]};
+              g = v4f{g[1], g[2], g[3], g[0]};
+            }
+            atomicMax(&sM[1][r0 + i * 16 + fr], __float_as_uint(top));
+          }
+        }
+        __syncthreads();
+#pragma unroll
+        for (int i = 0; i < NR; i++) M[i] = fmaxf(M[i], __uint_as_float(sM[1][r0 + i * 16 + fr]));
+      }
+      if (tid == 0 && sCnt[pp] > RP) atomicAdd(&g_ffn_repairs[1], (unsigned long long)NR);
+    }
+    // the next pass's first weight blocks, behind the GELUs
+    if (kP > 1 && pp + 1 < kP) {
+      load_w1(0, w1[0]);
+      load_w1(1, w1[1]);
+    }
+
+    // ---- GELU and quantization into the LDS tile ----
+    opaque_ids();
+    if (wave == 0 && fq == 0) {
+#pragma unroll
+      for (int i = 0; i < NR; i++) sMax[r0 + i * 16 + fr] = M[i];  // for the epilogue
+    }
+    float inv[NR], lim[NR];
+#pragma unroll
+    for (int i = 0; i < NR; i++) {
+      inv[i] = 127.0f / M[i];
+      lim[i] = fmaxf(0.5f - fmaf(gs_max * kQAbs, inv[i], 0x1p-24f), 0.0f);
+    }
 #pragma unroll
     for (int j = 0; j < kUpCB; j++) {
       // waves w and w + 4 share a SIMD; alternating their priority per column block
       // keeps them level, so neither waits long at the barrier after the loop
       if ((j ^ (wave >> 2)) & 1) __builtin_amdgcn_s_setprio(1);
       else __builtin_amdgcn_s_setprio(0);
-      const float ws = cop[0], bb = cop[1], gs = cop[2];
-      if (j + 1 < kUpCB) load_cop(j + 1);
-      if (j + 1 < kUpCB) {
-        mma_col(j + 1, bq[(j + 1) & 1]);
-        if (j + 3 < kUpCB) load_col(j + 3, bq[(j + 1) & 1]);
-      }
-      if constexpr (kFast) gs_max = fmaxf(gs_max, fabsf(gs));
+      const int col = (j * kWaves + wave) * 16;
+      uint32_t pk[NR];
+      if constexpr (kFast) {
+        const v4f gs = *reinterpret_cast<const v4f*>(&sGs[col + fq * 4]);
+        bool bad[NR], any = false;
+        constexpr int N = 4 * NR;
+        float vv[N], x[N], t[N], d[N], gi[N];
 #pragma unroll
-      for (int i = 0; i < 2; i++)
+        for (int k = 0; k < N; k++) vv[k] = v[k >> 2][k & 3][j];
+        gelu_fast_n<N>(vv, kc, x);
+        auto each = [&](auto f) {
 #pragma unroll
-        for (int r = 0; r < 4; r++) {
-          const float v = fmaf((float)acc[i][j][r], sa[i][r] * ws, bb);
-          if constexpr (kFast) {
-            float g = gelu_fast(v) * gs;
-            asm volatile("" : "+v"(g));  // in program order, as below
-            const uint32_t key = (__float_as_uint(g) & 0x7ffffff0u) | (uint32_t)j;
-            const bool top = key > t1[i][r];
-            uint32_t m2;
-            asm("v_med3_u32 %0, %1, %2, %3" : "=v"(m2) : "v"(key), "v"(t1[i][r]), "v"(t2[i][r]));
-            t2[i][r] = m2;
-            t1[i][r] = max(t1[i][r], key);
-            vt[i][r] = top ? v : vt[i][r];
-            // the tracking state in program order too (else the compiler sinks the
-            // selects and holds every element's v and compare mask: spills)
-            asm volatile("" : "+v"(t1[i][r]), "+v"(t2[i][r]), "+v"(vt[i][r]));
-            acc[i][j][r] = __float_as_int(g);
-          } else {
-            float g = gelu_exact(v, tb) * gs;
-            // g is materialized here, in program order: without this the compiler
-            // sinks the GELU tails towards their later uses and keeps every
-            // head's double-precision temporaries live (hundreds of spills)
-            asm volatile("" : "+v"(g));
-            acc[i][j][r] = __float_as_int(g);
-            mx[i][r] = nanless_max(mx[i][r], fabsf(g));
+          for (int k = 0; k < N; k++) f(k);
+          __builtin_amdgcn_sched_barrier(0);
+        };
+        each([&](int k) { gi[k] = gs[k & 3] * inv[k >> 2]; });
+        each([&](int k) { x[k] = x[k] * gi[k]; });
+        each([&](int k) { t[k] = x[k] + 0x1.8p23f; });  // round to nearest: the low byte of t is q
+        each([&](int k) { d[k] = t[k] - 0x1.8p23f; });
+        each([&](int k) { d[k] = x[k] - d[k]; });
+        each([&](int k) { d[k] = fmaf(fabsf(x[k]), kq, fabsf(d[k])); });
+#pragma unroll
+        for (int i = 0; i < NR; i++) {
+          uint32_t worst = 0;
+#pragma unroll
+          for (int r = 0; r < 4; r++) worst = max(worst, __float_as_uint(d[4 * i + r]));  // (as u32: a NaN is the largest)
+          auto tb4 = [&](int r) { return __float_as_uint(t[4 * i + r]); };
+          pk[i] = __builtin_amdgcn_perm(__builtin_amdgcn_perm(tb4(3), tb4(2), 0x0c0c0400u),
+                                        __builtin_amdgcn_perm(tb4(1), tb4(0), 0x0c0c0400u), 0x05040100u);
+          bad[i] = worst >= __float_as_uint(lim[i]);
+          any = any || bad[i];
+        }
+        if (__builtin_expect(__builtin_amdgcn_ballot_w64(any) != 0, 0)) {  // rare: the tiles' exact values
+#pragma unroll
+          for (int i = 0; i < NR; i++) {
+            if (__builtin_amdgcn_ballot_w64(bad[i]) == 0) continue;
+            if (lane == 0) atomicAdd(&g_ffn_repairs[0], 1ull);
+            v4f x = v4f{v[i][0][j], v[i][1][j], v[i][2][j], v[i][3][j]}, g = gs;
+            uint32_t w = 0;
+#pragma unroll 1
+            for (int r = 0; r < 4; r++) {  // element 0 evaluated, then the four rotated
+              const int q = qround_bounded(gelu_exact(x[0], tb) * g[0] * inv[i]);
+              w = (w >> 8) | ((uint32_t)q << 24);
+              x = v4f{x[1], x[2], x[3], x[0]};
+              g = v4f{g[1], g[2], g[3], g[0]};
+            }
+            pk[i] = w;
           }
         }
+      } else {
+#pragma unroll
+        for (int i = 0; i < NR; i++)
+          pk[i] = pack4(qround_bounded(v[i][0][j] * inv[i]), qround_bounded(v[i][1][j] * inv[i]),
+                        qround_bounded(v[i][2][j] * inv[i]), qround_bounded(v[i][3][j] * inv[i]));
+      }
+#pragma unroll
+      for (int i = 0; i < NR; i++)
+        *reinterpret_cast<uint32_t*>(&sQ[(r0 + i * 16 + fr) * kQPitch + col + fq * 4]) = pk[i];
     }
     __builtin_amdgcn_s_setprio(0);
-    // the next pass's first weight blocks and row scales, behind the absmax and
-    // quantization (kFast: after the row-maximum check, whose rare recomputation
-    // would otherwise hold them too)
-    auto load_next = [&]() {
-      if (pp + 1 < kP) {
-        load_col(0, bq[0]);
-        load_col(1, bq[1]);
-        load_sa(r0 + kRows, sa_next);
-      }
-    };
-    if constexpr (!kFast) load_next();
-    // kFast: k0 (see kUpRel) and, per row, the exact |g| of the lane's top element and the upper
-    // bound of its others
-    float k0 = 0.0f;
-    uint32_t ub[2][4];
-    if constexpr (kFast) {
-      k0 = fmaf(gs_max, kAbsGs, 0x1p-140f);
-#pragma unroll
-      for (int i = 0; i < 2; i++)
-#pragma unroll
-        for (int r = 0; r < 4; r++) {
-          const float v = vt[i][r];
-          const float gst = gsm[(cb1 + (int)(t1[i][r] & 15u)) * 16 + fr];
-          const bool sat = v >= kGeluSatPos || (v <= kGeluSatNeg && v >= -3.40282347e38f);
-          float G = v >= kGeluSatPos ? v : 0.0f;  // the saturated values (gelu_exact's, by enumeration)
-          if (__builtin_amdgcn_ballot_w64(!sat) != 0) G = gelu_exact(v, tb);  // wave-uniform
-          mx[i][r] = nanless_max(1e-8f, fabsf(G * gst));
-          ub[i][r] = __float_as_uint(fmaf(__uint_as_float(t2[i][r] | 15u), kHiMul, k0)) & 0x7fffffffu;
-        }
-    }
-    // row absmax: over the 16 lanes of this row quad (no NaN: nanless_max above),
-    // then over the 8 waves via LDS
-#pragma unroll
-    for (int i = 0; i < 2; i++)
-#pragma unroll
-      for (int r = 0; r < 4; r++) {
-        mx[i][r] = row16_max(mx[i][r]);
-        if constexpr (kFast) ub[i][r] = row16_max_u32(ub[i][r]);
-      }
-    if (fr == 0) {
-#pragma unroll
-      for (int i = 0; i < 2; i++)
-#pragma unroll
-        for (int r = 0; r < 4; r++) {
-          sMax[r0 + i * 16 + fq * 4 + r][wave] = mx[i][r];
-          if constexpr (kFast) sU[r0 + i * 16 + fq * 4 + r][wave] = ub[i][r];
-        }
-    }
-    __syncthreads();
-
-    // ---- quantize: q = round(g * (127 / max_abs)) into the LDS tile ----
-    // A lane's 4 values of one tile are 4 rows of one column; a quad byte
-    // transpose turns them into 4 columns of one row, written as one dword.
-    const int qk = fr & 3;
-    if constexpr (!kFast) {
-#pragma unroll
-      for (int i = 0; i < 2; i++) {
-        float inv_scale[4];
-#pragma unroll
-        for (int r = 0; r < 4; r++) inv_scale[r] = 127.0f / row_absmax(r0 + i * 16 + fq * 4 + r);
-        int8_t* dst = &sQ[(r0 + i * 16 + fq * 4 + qk) * kQPitch + cb1 * 16 + (fr & 12)];
-#pragma unroll
-        for (int j = 0; j < kUpCB; j++) {
-          const uint32_t col4 = pack4(qround_bounded(__int_as_float(acc[i][j][0]) * inv_scale[0]),
-                                      qround_bounded(__int_as_float(acc[i][j][1]) * inv_scale[1]),
-                                      qround_bounded(__int_as_float(acc[i][j][2]) * inv_scale[2]),
-                                      qround_bounded(__int_as_float(acc[i][j][3]) * inv_scale[3]));
-          *reinterpret_cast<uint32_t*>(dst + j * 16) = quad_transpose_bytes(col4, qk);
-        }
-      }
-    } else {
-      // the row maxima, and whether some row's bound reaches its maximum (every wave's
-      // lanes cover all 32 rows of the pass, so all waves take the same branch)
-      float M[2][4];
-      bool reach = false;
-#pragma unroll
-      for (int i = 0; i < 2; i++)
-#pragma unroll
-        for (int r = 0; r < 4; r++) {
-          const int row = r0 + i * 16 + fq * 4 + r;
-          M[i][r] = row_absmax(row);
-          const uint4 u0 = *reinterpret_cast<const uint4*>(&sU[row][0]);
-          const uint4 u1 = *reinterpret_cast<const uint4*>(&sU[row][4]);
-          const uint32_t u = max(max(max(u0.x, u0.y), max(u0.z, u0.w)), max(max(u1.x, u1.y), max(u1.z, u1.w)));
-          reach = reach || u >= __float_as_uint(M[i][r]);
-        }
-      if (__builtin_amdgcn_ballot_w64(reach) != 0) {  // rare: exact values of every element that can reach it
-        uint32_t tiles = 0;
-#pragma unroll
-        for (int i = 0; i < 2; i++)
-#pragma unroll
-          for (int j = 0; j < kUpCB; j++) {
-            bool c = false;
-#pragma unroll
-            for (int r = 0; r < 4; r++) {
-              const uint32_t hi =
-                  __float_as_uint(fmaf(fabsf(__int_as_float(acc[i][j][r])), kHiMul, k0)) & 0x7fffffffu;
-              c = c || hi >= __float_as_uint(M[i][r]);
-            }
-            if (__builtin_amdgcn_ballot_w64(c) != 0) tiles |= 1u << (i * kUpCB + j);
-          }
-        if (lane == 0 && wave == 0) atomicAdd(&g_ffn_repairs[1], 1ull);
-        while (tiles != 0) {  // wave-uniform
-          const int t = __builtin_ctz(tiles);
-          tiles &= tiles - 1;
-          const int i = t >= kUpCB ? 1 : 0, j = t - i * kUpCB;
-          float g[4];
-          exact_tile(i, j, g, std::true_type{});
-#pragma unroll
-          for (int r = 0; r < 4; r++)
-            if (!__builtin_isnan(g[r])) atomicMax(&sMax2[r0 + i * 16 + fq * 4 + r], __float_as_uint(fabsf(g[r])));
-        }
-        __syncthreads();
-#pragma unroll
-        for (int i = 0; i < 2; i++)
-#pragma unroll
-          for (int r = 0; r < 4; r++) M[i][r] = fmaxf(M[i][r], __uint_as_float(sMax2[r0 + i * 16 + fq * 4 + r]));
-      }
-      float inv_scale[2][4], th0[2][4];
-#pragma unroll
-      for (int i = 0; i < 2; i++)
-#pragma unroll
-        for (int r = 0; r < 4; r++) {
-          inv_scale[i][r] = 127.0f / M[i][r];
-          th0[i][r] = fmaf(k0 * kK0Inv, inv_scale[i][r], 0x1p-25f);
-        }
-      uint32_t undecided = 0;  // wave-uniform: column tiles (i, j) with a value too close to a rounding boundary
-#pragma unroll
-      for (int i = 0; i < 2; i++) {
-        int8_t* dst = &sQ[(r0 + i * 16 + fq * 4 + qk) * kQPitch + cb1 * 16 + (fr & 12)];
-#pragma unroll
-        for (int j = 0; j < kUpCB; j++) {
-          int q[4];
-          bool ok = true;
-#pragma unroll
-          for (int r = 0; r < 4; r++) {
-            const float x = __int_as_float(acc[i][j][r]) * inv_scale[i][r];
-            q[r] = qround_bounded(x);
-            const float dist = fabsf(__builtin_amdgcn_fractf(fabsf(x)) - 0.5f);
-            ok = ok && dist > fmaf(fabsf(x), kQRel, th0[i][r]);
-          }
-          if (__builtin_amdgcn_ballot_w64(!ok) != 0) undecided |= 1u << (i * kUpCB + j);
-          *reinterpret_cast<uint32_t*>(dst + j * 16) = quad_transpose_bytes(pack4(q[0], q[1], q[2], q[3]), qk);
-        }
-      }
-      // (issued here, the next pass's operands are not held through the quantization)
-      load_next();
-      if (undecided != 0) {
-        wave_lds_sync();  // this wave's dword stores land before the bytes that replace them
-        if (lane == 0) atomicAdd(&g_ffn_repairs[0], (unsigned long long)__builtin_popcount(undecided));
-        while (undecided != 0) {  // wave-uniform
-          const int t = __builtin_ctz(undecided);
-          undecided &= undecided - 1;
-          const int i = t >= kUpCB ? 1 : 0, j = t - i * kUpCB;
-          float g[4];
-          exact_tile(i, j, g, std::false_type{});
-#pragma unroll
-          for (int r = 0; r < 4; r++) {
-            const float inv = i ? inv_scale[1][r] : inv_scale[0][r];
-            sQ[(r0 + i * 16 + fq * 4 + r) * kQPitch + (cb1 + j) * 16 + fr] = (int8_t)qround_bounded(g[r] * inv);
-          }
-        }
-      }
-    }
-    if (pp + 1 < kP) {
-#pragma unroll
-      for (int i = 0; i < 2; i++)
-#pragma unroll
-        for (int r = 0; r < 4; r++) sa[i][r] = sa_next[i][r];
-    }
   }
 
-  // ---- FFN-down: acc2[i][j] = rows 16i.., columns (3w + j)*16.., K = 1536 ----
-  const int cb2 = wave * kDnCB;
-  const __amdgpu_buffer_rsrc_t w2r = weight_rsrc(p.w2, kF * kH);
-  auto load_b2 = [&](int kt, v4i* dst) {
-    int base = (kt * (kH / 16) + cb2) * 1024;  // (opaque, as in load_col)
+  // ---- FFN-down: acc2[i][n] = rows 16i.., columns 48 w + 16 n.., K = 1536 ----
+  opaque_ids();
+  constexpr int kRB = NR * kP;  // 16-row blocks
+  const int dcol = wave * kDnCB * 16;
+  auto load_w2 = [&](int kt, v4i (&dst)[kDnCB]) {
+    int base = (kt * (kH / 16)) * 1024 + dcol * 64;
     asm volatile("" : "+s"(base));
 #pragma unroll
-    for (int j = 0; j < kDnCB; j++) dst[j] = weight_load(w2r, lane16, base + j * 1024);
+    for (int n = 0; n < kDnCB; n++) dst[n] = weight_load(w2r, lane16, base + n * 1024);
   };
   v4i ring[kRing][kDnCB];
 #pragma unroll
-  for (int s = 0; s < kRing; s++) load_b2(s, ring[s]);
-  // the epilogue's residual float4s (all kP halves), loaded now so that HBM latency hides behind FFN-down
-  constexpr int kF4 = kDnCB * 4;              // float4 columns of one wave row (12)
-  constexpr int kEpiIt = kRows * kF4 / 64;    // float4s per lane and 32 rows (6)
-  float4 res4[kP][kEpiIt];
+  for (int s = 0; s < kRing; s++) load_w2(s, ring[s]);
+  // the epilogue's operands, loaded now so that the residual's HBM latency hides behind FFN-down
+  v4f res[kRB][kDnCB];
 #pragma unroll
-  for (int h = 0; h < kP; h++)
+  for (int i = 0; i < kRB; i++)
 #pragma unroll
-    for (int k = 0; k < kEpiIt; k++) {
-      const int idx = lane + 64 * k, rr = kRows * h + idx / kF4, c4 = idx % kF4;
-      const v4i r = __builtin_nontemporal_load(
-          reinterpret_cast<const v4i*>(p.res + (size_t)min(m0 + rr, p.M - 1) * kH + cb2 * 16 + c4 * 4));
-      res4[h][k] = make_float4(__int_as_float(r.x), __int_as_float(r.y), __int_as_float(r.z), __int_as_float(r.w));
-    }
+    for (int n = 0; n < kDnCB; n++)
+      res[i][n] = __builtin_nontemporal_load(
+          reinterpret_cast<const v4f*>(p.res + (size_t)min(m0 + i * 16 + fr, p.M - 1) * kH + dcol + n * 16 + fq * 4));
   __syncthreads();  // sQ complete
-  constexpr int kRB = kT / 16;  // 16-row blocks
   v4i acc2[kRB][kDnCB];
 #pragma unroll
   for (int i = 0; i < kRB; i++)
 #pragma unroll
-    for (int j = 0; j < kDnCB; j++) acc2[i][j] = v4i{0, 0, 0, 0};
+    for (int n = 0; n < kDnCB; n++) acc2[i][n] = v4i{0, 0, 0, 0};
 #pragma unroll
   for (int kt = 0; kt < kDnSteps; kt++) {  // fully unrolled ring of kRing steps
-    v4i af[kRB];
+    v4i q[kRB];
 #pragma unroll
-    for (int i = 0; i < kRB; i++) af[i] = *reinterpret_cast<const v4i*>(&sQ[(i * 16 + fr) * kQPitch + kt * 64 + fq * 16]);
+    for (int i = 0; i < kRB; i++) q[i] = *reinterpret_cast<const v4i*>(&sQ[(i * 16 + fr) * kQPitch + kt * 64 + fq * 16]);
 #pragma unroll
-    for (int j = 0; j < kDnCB; j++)
+    for (int n = 0; n < kDnCB; n++)
 #pragma unroll
       for (int i = 0; i < kRB; i++)
-        acc2[i][j] = __builtin_amdgcn_mfma_i32_16x16x64_i8(af[i], ring[kt % kRing][j], acc2[i][j], 0, 0, 0);
-    if (kt + kRing < kDnSteps) load_b2(kt + kRing, ring[kt % kRing]);
+        acc2[i][n] = __builtin_amdgcn_mfma_i32_16x16x64_i8(ring[kt % kRing][n], q[i], acc2[i][n], 0, 0, 0);
+    if (kt + kRing < kDnSteps) load_w2(kt + kRing, ring[kt % kRing]);
   }
 
-  // ---- epilogue of FFN-down through this wave's LDS tile, whole float4s per lane, 32 rows at a time ----
-  if constexpr (kP > 1) __syncthreads();  // every wave is done with sQ, whose space the staging reuses
-  int* E = (kP == 1 ? sE1 : reinterpret_cast<int*>(sQ)) + wave * kEWords;
+  // ---- epilogue: out = fma(f32(acc), s * ws2, b2 + res), whole float4s per lane ----
+  v4f ws2[kDnCB], b2[kDnCB];
 #pragma unroll
-  for (int h = 0; h < kP; h++) {
-    if (h > 0) wave_lds_sync();  // the previous half's reads are done
+  for (int n = 0; n < kDnCB; n++) {
+    ws2[n] = *reinterpret_cast<const v4f*>(p.w2_scale + dcol + n * 16 + fq * 4);
+    b2[n] = *reinterpret_cast<const v4f*>(p.b2 + dcol + n * 16 + fq * 4);
+  }
 #pragma unroll
-    for (int i = 0; i < 2; i++)
+  for (int i = 0; i < kRB; i++) {
+    const float s = sMax[i * 16 + fr] / 127.0f;  // scale = max_abs / 127.0
+    const int row = m0 + i * 16 + fr;
 #pragma unroll
-      for (int j = 0; j < kDnCB; j++)
+    for (int n = 0; n < kDnCB; n++) {
+      v4f o;
 #pragma unroll
-        for (int r = 0; r < 4; r++) E[(i * 16 + fq * 4 + r) * kEPitch + j * 16 + fr] = acc2[2 * h + i][j][r];
-    wave_lds_sync();
-#pragma unroll
-    for (int k = 0; k < kEpiIt; k++) {
-      const int idx = lane + 64 * k, er = idx / kF4, c4 = idx - er * kF4, rr = kRows * h + er;
-      const int row = m0 + rr;
-      const bool ok = row < p.M;
-      const int col = cb2 * 16 + c4 * 4;
-      float mrow = row_absmax(rr);
-      if constexpr (kFast) mrow = fmaxf(mrow, __uint_as_float(sMax2[rr]));
-      const float s = mrow / 127.0f;  // scale = max_abs / 127.0
-      const int4 a4 = *reinterpret_cast<const int4*>(&E[er * kEPitch + c4 * 4]);
-      const float4 ws4 = *reinterpret_cast<const float4*>(p.w2_scale + col);
-      float4 b4 = *reinterpret_cast<const float4*>(p.b2 + col);
-      const float4 r4 = res4[h][k];
-      b4.x = b4.x + r4.x; b4.y = b4.y + r4.y; b4.z = b4.z + r4.z; b4.w = b4.w + r4.w;
-      float4 v;
-      v.x = fmaf((float)a4.x, s * ws4.x, b4.x);
-      v.y = fmaf((float)a4.y, s * ws4.y, b4.y);
-      v.z = fmaf((float)a4.z, s * ws4.z, b4.z);
-      v.w = fmaf((float)a4.w, s * ws4.w, b4.w);
-      if (ok)  // streaming store: keeps the weights resident in L2
-        __builtin_nontemporal_store(v4i{__float_as_int(v.x), __float_as_int(v.y), __float_as_int(v.z), __float_as_int(v.w)},
-                                    reinterpret_cast<v4i*>(p.out + (size_t)row * kH + col));
+      for (int r = 0; r < 4; r++) o[r] = fmaf((float)acc2[i][n][r], s * ws2[n][r], b2[n][r] + res[i][n][r]);
+      if (row < p.M)  // streaming store: keeps the weights resident in L2
+        __builtin_nontemporal_store(o, reinterpret_cast<v4f*>(p.out + (size_t)row * kH + dcol + n * 16 + fq * 4));
     }
   }
 }
 
-// 64-row workgroups stream W2 once per 64 rows instead of twice, at about 1.87x
-// the time of a 32-row one (measured at C5).  With one workgroup per CU, a
-// launch takes about as many workgroup times as it has rounds of workgroups over
-// the CUs, so launch_ffn picks, in 32-row workgroup times, the cheapest of: all
-// rows in 32-row workgroups, all in 64-row ones, or k full rounds of 64-row
-// workgroups followed by a second launch of 32-row ones for the remaining rows
-// (its last, partial round then holds the short workgroups).
 static int g_ffn_rows = 0;  // 0 by the batch, 32, 64, or -m: the mixed plan with m rows first (test hook)
 void set_ffn_rows(int rows) { g_ffn_rows = rows; }
 int ffn_rows() { return g_ffn_rows; }
@@ -626,55 +562,69 @@ hipError_t ffn_repair_counts(unsigned long long counts[2], bool reset) {
   return e;
 }
 
-template <int kP>
-static void launch_ffn_rows(const FfnArgs& p, unsigned grid, hipStream_t st) {
+template <int NR, int kP>
+static void launch_ffn_rows(const FfnArgs& p, hipStream_t st) {
+  constexpr int R = 16 * NR * kP;
+  const dim3 grid((unsigned)((p.M + R - 1) / R));
   if (p.fast_gelu && !g_ffn_exact_gelu)
-    hipLaunchKernelGGL((ffn_fused_kernel<kP, true>), dim3(grid), dim3(512), 0, st, p);
+    hipLaunchKernelGGL((ffn_kernel<NR, kP, true>), grid, dim3(kThreads), 0, st, p);
   else
-    hipLaunchKernelGGL((ffn_fused_kernel<kP, false>), dim3(grid), dim3(512), 0, st, p);
+    hipLaunchKernelGGL((ffn_kernel<NR, kP, false>), grid, dim3(kThreads), 0, st, p);
+}
+static void launch_ffn_tile(const FfnArgs& p, int rows, hipStream_t st) {
+  if (rows == 16) launch_ffn_rows<1, 1>(p, st);
+  else if (rows == 32) launch_ffn_rows<2, 1>(p, st);
+  else launch_ffn_rows<2, 2>(p, st);
 }
 
+// With one workgroup per CU a launch takes about as many workgroup times as it
+// has rounds of workgroups over the CUs.  Times in hundredths of a 16-row
+// workgroup's (18 to 21 us): a 32-row one 140 (25 to 29 us), a 64-row one 255 (54
+// us for one round, 107 for two, 900 for 18).  The plan is the cheapest of: all
+// rows in 16-, 32- or 64-row workgroups, or k full rounds of 64-row ones and then
+// a second launch for the remaining rows, whose last, partial round then holds
+// short workgroups (68,270 rows: 233 us, against 245 in 64-row and 251 in 32-row
+// workgroups).
 void launch_ffn(const FfnArgs& p, hipStream_t st, hipStream_t side, hipEvent_t fork, hipEvent_t join) {
   if (p.M <= 0) return;
   const long cus = device_cu_count();
   auto rounds = [&](long rows, long tile) { return ((rows + tile - 1) / tile + cus - 1) / cus; };
-  constexpr long kT64 = 187;  // a 64-row workgroup's time, in hundredths of a 32-row one
-  long best = 100 * rounds(p.M, 32), best_k = -1;  // -1: all 32-row, 0: all 64-row, k: mixed
-  if (100 * rounds(p.M, 32) > kT64 * rounds(p.M, 64)) best = kT64 * rounds(p.M, 64), best_k = 0;
+  constexpr long kT16 = 100, kT32 = 140, kT64 = 255, kFirst64 = 15, kLaunch = 10;
+  auto short_tile = [&](long rows) { return kT16 * rounds(rows, 16) <= kT32 * rounds(rows, 32) ? 16 : 32; };
+  auto short_time = [&](long rows) { return std::min(kT16 * rounds(rows, 16), kT32 * rounds(rows, 32)); };
+  int tile = short_tile(p.M), tail = 0;
+  long best = short_time(p.M), m64 = 0;
+  if (kT64 * rounds(p.M, 64) + kFirst64 < best) best = kT64 * rounds(p.M, 64) + kFirst64, tile = 64;
   for (long k = 1; 64 * cus * k < p.M; k++) {
-    const long t = kT64 * k + 100 * rounds(p.M - 64 * cus * k, 32) + 10;  // + a second launch
-    if (t < best) best = t, best_k = k;
+    const long rem = p.M - 64 * cus * k, t = kT64 * k + kFirst64 + short_time(rem) + kLaunch;
+    if (t < best) best = t, m64 = 64 * cus * k, tail = short_tile(rem);
   }
-  if (g_ffn_rows == 32) best_k = -1;
-  if (g_ffn_rows == 64) best_k = 0;
-  int m64 = (int)(64 * cus * (best_k > 0 ? best_k : 0));
+  if (g_ffn_rows > 0) tile = g_ffn_rows, m64 = 0;
   if (g_ffn_rows < 0) {  // forced mixed plan (m64 rows in 64-row workgroups, when there are more)
-    m64 = -g_ffn_rows;
-    best_k = m64 < p.M ? 1 : 0;
+    m64 = -g_ffn_rows < p.M ? -g_ffn_rows : 0;
+    tile = 64, tail = 32;
   }
-  if (best_k < 0) {
-    launch_ffn_rows<1>(p, (unsigned)((p.M + 31) / 32), st);
-  } else if (best_k == 0) {
-    launch_ffn_rows<2>(p, (unsigned)((p.M + 63) / 64), st);
+  if (m64 == 0) {
+    launch_ffn_tile(p, tile, st);
+    return;
+  }
+  FfnArgs a = p, b = p;
+  a.M = (int)m64;
+  b.M = (int)(p.M - m64);
+  b.A = p.A + m64 * kH;
+  b.a_scale = p.a_scale + m64;
+  b.res = p.res + m64 * kH;
+  b.out = p.out + m64 * kH;
+  if (side && fork && join) {
+    (void)hipEventRecord(fork, st);
+    (void)hipStreamWaitEvent(side, fork, 0);
+    launch_ffn_tile(b, tail, side);
+    (void)hipEventRecord(join, side);
+    launch_ffn_tile(a, 64, st);
+    (void)hipStreamWaitEvent(st, join, 0);
   } else {
-    FfnArgs a = p, b = p;
-    a.M = m64;
-    b.M = p.M - m64;
-    b.A = p.A + (size_t)m64 * kH;
-    b.a_scale = p.a_scale + m64;
-    b.res = p.res + (size_t)m64 * kH;
-    b.out = p.out + (size_t)m64 * kH;
-    if (side && fork && join) {
-      (void)hipEventRecord(fork, st);
-      (void)hipStreamWaitEvent(side, fork, 0);
-      launch_ffn_rows<1>(b, (unsigned)((b.M + 31) / 32), side);
-      (void)hipEventRecord(join, side);
-      launch_ffn_rows<2>(a, (unsigned)(m64 / 64), st);
-      (void)hipStreamWaitEvent(st, join, 0);
-    } else {
-      launch_ffn_rows<2>(a, (unsigned)(m64 / 64), st);
-      launch_ffn_rows<1>(b, (unsigned)((b.M + 31) / 32), st);
-    }
+    launch_ffn_tile(a, 64, st);
+    launch_ffn_tile(b, tail, st);
   }
 }
 

@@ -66,16 +66,17 @@ struct FfnArgs {
   // g_smooth entry finite (else the exact-GELU kernel runs)
   bool fast_gelu = false;
 };
-// side (optional, with fork and join events): a second stream on which the mixed
-// plan's 32-row launch runs beside the 64-row one (forked after the work queued
-// on st, joined before st continues), so its partial round of workgroups fills
-// CUs as the 64-row rounds free them instead of running alone at the end
+// side (optional, with fork and join events): a second stream on which a mixed
+// plan's launch of short workgroups runs beside the 64-row one (forked after the
+// work queued on st, joined before st continues), so its partial round of
+// workgroups fills CUs as the 64-row rounds free them instead of running alone
+// at the end
 void launch_ffn(const FfnArgs& p, hipStream_t st, hipStream_t side = nullptr, hipEvent_t fork = nullptr,
                 hipEvent_t join = nullptr);
 // test hooks: the exact-GELU kernel for every launch (process-wide); the fast
 // kernel's repair counters on the current device ([0] column tiles recomputed for
-// an undecided quantized value, [1] passes that recomputed elements for a row
-// maximum), optionally reset
+// an undecided quantized value, [1] groups of 16 rows in which a row maximum was
+// settled among several exact values), optionally reset
 void set_ffn_exact_gelu(bool exact);
 bool ffn_exact_gelu();
 hipError_t ffn_repair_counts(unsigned long long counts[2], bool reset);

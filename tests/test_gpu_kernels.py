@@ -395,6 +395,58 @@ def test_ffn_fast_and_exact_gelu_kernels_agree(torch_gpu):
     assert np.array_equal(bits(outs[0][:300]), bits(ref))
 
 
+@pytest.mark.parametrize("m", [1, 15, 16, 17, 47, 1025, 4096, 4097, 8193])
+def test_ffn_fused_by_the_batch_bit_exact(torch_gpu, m):
+    """The fused FFN with the workgroup height that the launch picks: 16 rows up to 4,096 of them
+    (partial last tiles included), 32 from there on."""
+    torch = torch_gpu
+    w1, ws1, b1, s1 = linear_inputs(1536, 384, 51)
+    w2, ws2, b2, s2 = linear_inputs(384, 1536, 52)
+    rng = np.random.default_rng(m)
+    a = rng.integers(-127, 128, (m, 384), dtype=np.int8)
+    sa = rng.uniform(0.001, 0.1, m).astype(f32)
+    res = rng.normal(0, 1, (m, 384)).astype(f32)
+    up, down = ae.Linear(w1, ws1, b1, s1), ae.Linear(w2, ws2, b2, s2)
+    a_d, sa_d, res_d = dev(torch, a), dev(torch, sa), dev(torch, res)
+    out_d = torch.full((m, 384), float("nan"), dtype=torch.float32, device="cuda")
+    up.ffn(down, m, a_d.data_ptr(), sa_d.data_ptr(), res_d.data_ptr(), out_d.data_ptr())
+    torch.cuda.synchronize()
+    ref = _ffn_ref(a, sa, w1, ws1, b1, w2, ws2, b2, s2, res)
+    assert np.array_equal(bits(out_d.cpu().numpy()), bits(ref))
+
+
+@pytest.mark.parametrize("m", [5, 70])
+def test_ffn_row_maximum_candidates(torch_gpu, ffn_rows, m):
+    """Row maxima that the fused FFN's first candidate scan cannot settle: rows whose largest
+    pre-activation is small (GELU far below its bound, a large inv_smooth on a negative column, every
+    column alike so that the candidates overflow a wave's list) and infinite or NaN row scales."""
+    torch = torch_gpu
+    w1, ws1, b1, s1 = linear_inputs(1536, 384, 61)
+    w2, ws2, b2, s2 = linear_inputs(384, 1536, 62)
+    rng = np.random.default_rng(63)
+    a = rng.integers(-127, 128, (m, 384), dtype=np.int8)
+    sa = rng.uniform(1e-5, 1e-3, m).astype(f32)  # |v| up to about 0.3
+    res = rng.normal(0, 1, (m, 384)).astype(f32)
+    sa[0] = 0.0                       # v = b1 alone
+    sa[1], sa[2] = np.inf, np.nan
+    s2[7] = 40.0                      # a negative GELU may be the row maximum
+    w1[7], b1[7] = 0, -0.75
+    outs = []
+    for flat in (False, True):
+        if flat:  # every column the same value: all of them candidates
+            w1, b1, s2 = np.zeros_like(w1), np.full_like(b1, 0.3), np.ones_like(s2)
+        up, down = ae.Linear(w1, ws1, b1, s1), ae.Linear(w2, ws2, b2, s2)
+        a_d, sa_d, res_d = dev(torch, a), dev(torch, sa), dev(torch, res)
+        out_d = torch.full((m, 384), float("nan"), dtype=torch.float32, device="cuda")
+        up.ffn(down, m, a_d.data_ptr(), sa_d.data_ptr(), res_d.data_ptr(), out_d.data_ptr())
+        torch.cuda.synchronize()
+        outs.append((out_d.cpu().numpy(), _ffn_ref(a, sa, w1, ws1, b1, w2, ws2, b2, s2, res)))
+    for got, ref in outs:
+        nan = np.isnan(ref)
+        assert np.array_equal(nan, np.isnan(got))
+        assert np.array_equal(bits(got)[~nan], bits(ref)[~nan])
+
+
 @pytest.mark.parametrize("m", [1, 31, 33, 100])
 def test_layernorm_quant_bit_exact(torch_gpu, m):
     torch = torch_gpu

@@ -422,3 +422,20 @@ def test_one_activation_step_breaks_the_cosine_gate(oracle_model, layer):
         e = oracle_model.forward_cls_perturbed(ids, layer, row, col).astype(np.float64)
         cos = float(np.dot(e, base) / (np.linalg.norm(e) * np.linalg.norm(base)))
         assert cos < 0.99999 or np.abs(e - base).max() > 1e-4, (row, col, cos)
+
+
+def test_ffn_gelu_cap_on_every_float():
+    """The fused FFN kernel takes max(1.0854 v - 0.2158, 0.44) as an upper bound of |GELU(v)| for
+    its row maxima (ffn.hip): checked on every float of [0.25, 8) and on samples outside, where
+    |GELU(v)| <= max(v, 0.17) or GELU(v) <= v settles it."""
+    def cap(v):  # the kernel's fma rounds once; the f64 product is exact and the sum's error far below the margin
+        return np.maximum((v.astype(np.float64) * np.float32(1.0854) - np.float64(np.float32(0.2158))).astype(np.float32),
+                          np.float32(0.44))
+    lo, hi = (int(np.float32(x).view(np.uint32)) for x in (0.25, 8.0))
+    for first in range(lo, hi, 1 << 22):
+        v = np.arange(first, min(first + (1 << 22), hi), dtype=np.uint32).view(np.float32)
+        assert np.all(orc.gelu(v) * np.float32(1 + 2.0 ** -20) <= cap(v))
+    v = np.concatenate([np.arange(lo - (1 << 20), lo, dtype=np.uint32).view(np.float32),
+                        np.arange(hi, hi + (1 << 20), dtype=np.uint32).view(np.float32)])
+    v = np.concatenate([v, -np.linspace(0, 8, 1 << 20, dtype=np.float32), np.float32([1e10, 3e38, -1e10, 0.0])])
+    assert np.all(np.abs(orc.gelu(v)) <= cap(v))
