@@ -1,6 +1,7 @@
 // attention.hip -- varlen multi-head attention (head_dim 32) and the layer-11
 // [CLS]-only attention, both in the reference's exact scalar evaluation order.
 #include <hip/hip_runtime.h>
+#include <type_traits>
 
 #include <mutex>
 
@@ -213,6 +214,67 @@ __device__ __forceinline__ void add_blocks(float (&acc)[4], const v16f& pr) {
     for (int i = 0; i < 4; i++) acc[i] = acc[i] + pr[4 * blk + i];
 }
 
+// The item of a workgroup of the latency form for a batch of at most kHalfMaxSegs
+// segments, found from cu_seqlens by the workgroup itself where the plan kernel
+// would cost a launch.  Returns false for a surplus workgroup.
+//
+// tps > 0 (16-query tiles of the longest segment; all workgroups are resident at
+// once, so their order does not matter): workgroup (segment, tile, head), heads
+// fastest, which spreads every batch evenly over the CUs (dealt by (segment, head)
+// to XCDs instead, four XCDs get two of a row's 12 heads and the others one: 320
+// keys 16.4 us, against 13.0).  The bounds are two scalar loads, or known (len1).
+//
+// tps = 0, the plan's dealing in short, for XCD x = blockIdx % 8 and its slot
+// blockIdx / 8: segments longest first (lane b holds segment b), the 12 heads of
+// the one of rank r to XCDs (12 r + h) % 8, so XCD x has two of its heads when
+// (x < 4) == (r even) and one otherwise; a slot counts through its XCD's tiles in
+// that order.
+constexpr int kHalfMaxSegs = 16;
+__device__ __forceinline__ bool half_item(const AttnArgs& p, int tps, int& h, int4& rec) {
+  const int lmax = p.s_pitch - 4;
+  if (tps > 0) {
+    const int u = blockIdx.x / 12, b = u / tps, q0 = 16 * (u - b * tps);
+    h = blockIdx.x - 12 * u;
+    int s0 = 0, len = p.len1;
+    if (p.len1 <= 0) {
+      s0 = p.cu[b];
+      len = p.cu[b + 1] - s0;
+    }
+    len = min(len, lmax);
+    rec = make_int4(s0, len, q0, len - q0);
+    return true;
+  }
+  const int x = blockIdx.x & 7, slot = blockIdx.x >> 3, lane = threadIdx.x & 63;
+  const int s0 = p.cu[min(lane, p.B)], s1 = p.cu[min(lane + 1, p.B)];  // (lanes past the last segment: length 0)
+  const int L = max(0, min(s1 - s0, lmax)), key = (L << 6) - lane;
+  int rank = 0;
+#pragma unroll
+  for (int j = 0; j < kHalfMaxSegs; j++) rank += __builtin_amdgcn_readlane(key, j) > key ? 1 : 0;
+  // lane r: the segment of rank r, its tiles on this XCD and their inclusive prefix over the ranks (one DPP row)
+  const int seg = __builtin_amdgcn_ds_permute(4 * (lane < kHalfMaxSegs ? rank : lane), (L << 6) | lane);
+  const int tiles = ((seg >> 6) + 15) >> 4;
+  const bool two = (x < 4) == ((lane & 1) == 0);
+  const int mine = two ? 2 * tiles : tiles;
+  int incl = mine;
+  incl += __builtin_amdgcn_update_dpp(0, incl, 0x111, 0xf, 0xf, true);  // row_shr:1, 2, 4, 8
+  incl += __builtin_amdgcn_update_dpp(0, incl, 0x112, 0xf, 0xf, true);
+  incl += __builtin_amdgcn_update_dpp(0, incl, 0x114, 0xf, 0xf, true);
+  incl += __builtin_amdgcn_update_dpp(0, incl, 0x118, 0xf, 0xf, true);
+  const uint64_t owner = __ballot(lane < kHalfMaxSegs && slot < incl);
+  if (owner == 0) return false;
+  const int r = __builtin_ctzll(owner);
+  const int e = __builtin_amdgcn_readlane(seg, r), n = __builtin_amdgcn_readlane(tiles, r);
+  const int len = e >> 6;
+  int k = slot - __builtin_amdgcn_readlane(incl - mine, r);
+  h = (x + 4 * (r & 1)) & 7;
+  if (k >= n) {
+    k -= n;
+    h += 8;
+  }
+  rec = make_int4(__builtin_amdgcn_readlane(s0, e & 63), len, 16 * k, len - 16 * k);
+  return true;
+}
+
 // dynamic LDS: S[kAttnQ][pitch] scores -> exps, per tile: pitch = round16(L) + 4
 // (at most the launch's s_pitch, or kAttnLongL + 4 in the short-row launch)
 // The tiles of one (sequence, head) share that head's K and V: the plan deals
@@ -225,20 +287,38 @@ __device__ __forceinline__ void add_blocks(float (&acc)[4], const v16f& pr) {
 // back-to-back MFMAs before their adds), 160 VGPRs.  Otherwise one MFMA result
 // at a time with scalar operands, 92 VGPRs: for short rows, where the score
 // tile leaves room for more waves than the wide variant's registers do.
-template <bool kWide>
-__global__ __launch_bounds__(256) void attention_kernel(AttnArgs p, int list_records, int list) {
+//
+// kHalf > 0 (wide only; the latency form): tiles of 16 queries with half the LDS,
+// for batches whose 32-query tiles leave CUs idle (launch_attention), 116 VGPRs.
+// kHalf = 1: each item of the plan is taken by two workgroups; kHalf = 2: the tiles
+// come from half_item.
+//
+// kWaves = 8 for the smallest batches: the score and exp phases of a tile are
+// split over twice the waves (the in-order sums of a tile occupy one wave, or two,
+// either way).
+template <bool kWide, int kHalf, int kWaves>
+__global__ __launch_bounds__(64 * kWaves) void attention_kernel(AttnArgs p, int list_records, int list) {
   extern __shared__ __attribute__((aligned(16))) float smem[];
-  __shared__ float s_maxw[4][kAttnQ];
+  __shared__ float s_maxw[kWaves][kAttnQ];
   __shared__ float s_max[kAttnQ], s_inv[kAttnQ];
   __shared__ uint64_t s_tab[32];
   int h;
   int4 rec;
-  if (!plan_item(reinterpret_cast<const int4*>(p.plan) + (size_t)list * list_records, h, rec)) return;  // surplus
-  const int nq = rec.w;
-  if (nq == 0) return;
+  if constexpr (kHalf == 2) {
+    if (!half_item(p, /*tps=*/list_records, h, rec)) return;  // surplus
+  } else {
+    // workgroups x, x + 8, .. run on XCD x: with kHalf every second one takes an item's other half
+    const int slot = blockIdx.x >> 3, half = kHalf ? slot & 1 : 0;
+    if (!plan_item(reinterpret_cast<const int4*>(p.plan) + (size_t)list * list_records, kHalf ? slot >> 1 : slot, h, rec))
+      return;
+    rec.z += 16 * half;
+    rec.w -= 16 * half;
+  }
+  const int nq = kHalf ? min(rec.w, 16) : rec.w;
+  if (nq <= 0) return;
   const int s0 = rec.x, L = rec.y, q0 = rec.z;  // L <= s_pitch - 4 (the plan clamps it)
   const int pitch = ((L + 15) & ~15) + 4;        // this tile's score row pitch
-  const int nqh = (nq + 15) >> 4;  // query halves with at least one query
+  const int nqh = kHalf ? 1 : (nq + 15) >> 4;  // query halves with at least one query
   float* S = smem;                 // [kAttnQ][pitch]
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);  // uniform: per-wave loop bounds stay scalar
@@ -271,7 +351,7 @@ __global__ __launch_bounds__(256) void attention_kernel(AttnArgs p, int list_rec
   for (int qh = 0; qh < 2; qh++) load_dims(qkv + (size_t)min(q0 + 16 * qh + lr, L - 1) * HQKV, qf[qh]);
 
   // phase 1: scores (dot32_f32 scalar order) and the row max.  Wave w takes the
-  // 16-key blocks kb = w, w+4, ... with both query halves; A = K block, B = Q
+  // 16-key blocks kb = w, w + kWaves, ... with both query halves; A = K block, B = Q
   // half, so lane l ends with the scores of query 16qh + lr for keys
   // 16kb + 4lg + i.  K fragments come straight from global memory (L2), one
   // block ahead, into ping-pong registers (rows clamped to the segment).
@@ -327,12 +407,12 @@ __global__ __launch_bounds__(256) void attention_kernel(AttnArgs p, int list_rec
   {
     float ka[8], kb8[8];
     if (wave < nkb) load_kf(wave, ka);
-    for (int kb = wave; kb < nkb; kb += 8) {  // wave-uniform
-      load_kf(kb + 4, kb8);
+    for (int kb = wave; kb < nkb; kb += 2 * kWaves) {  // wave-uniform
+      load_kf(kb + kWaves, kb8);
       score_block(kb, ka);
-      if (kb + 4 >= nkb) break;
-      load_kf(kb + 8, ka);
-      score_block(kb + 4, kb8);
+      if (kb + kWaves >= nkb) break;
+      load_kf(kb + 2 * kWaves, ka);
+      score_block(kb + kWaves, kb8);
     }
   }
   // PV set-up (phase 6), and the V fragments of its first three key groups and
@@ -378,8 +458,12 @@ __global__ __launch_bounds__(256) void attention_kernel(AttnArgs p, int list_rec
     if (lane < 16) s_maxw[wave][16 * qh + lane] = m;
   }
   __syncthreads();
-  if (tid < kAttnQ)
-    s_max[tid] = fmaxf(fmaxf(s_maxw[0][tid], s_maxw[1][tid]), fmaxf(s_maxw[2][tid], s_maxw[3][tid]));
+  if (tid < kAttnQ) {
+    float m = s_maxw[0][tid];
+#pragma unroll
+    for (int w = 1; w < kWaves; w++) m = fmaxf(m, s_maxw[w][tid]);
+    s_max[tid] = m;
+  }
   __syncthreads();
 
   // phase 3: e_t = expf(s_t - max) over the nq x ceil(L/4) float4s of the tile,
@@ -392,14 +476,15 @@ __global__ __launch_bounds__(256) void attention_kernel(AttnArgs p, int list_rec
     const float rcols = 1.0f / (float)cols4;
     const int units = nq * cols4;
     // two float4 units per lane and step (eight independent exps in flight);
-    // wave-uniform trip count (expf_libm needs all lanes)
-    for (int u0 = 0; u0 < units; u0 += 512) {
-      float* e[2];
-      float4 v[2];
-      float m[2];
+    // wave-uniform trip count (expf_libm needs all lanes).  kHalf: one unit in a
+    // last step of at most one per lane.
+    auto exps = [&](int u0, auto n) {
+      float* e[n];
+      float4 v[n];
+      float m[n];
 #pragma unroll
-      for (int k = 0; k < 2; k++) {
-        const int u = min(u0 + 256 * k + tid, units - 1);
+      for (int k = 0; k < n; k++) {
+        const int u = min(u0 + 64 * kWaves * k + tid, units - 1);
         const int q = (int)(((float)u + 0.5f) * rcols);
         const int c4 = u - q * cols4;
         e[k] = &S[q * pitch + 4 * c4];
@@ -407,16 +492,19 @@ __global__ __launch_bounds__(256) void attention_kernel(AttnArgs p, int list_rec
         m[k] = s_max[q];
       }
 #pragma unroll
-      for (int k = 0; k < 2; k++) {
+      for (int k = 0; k < n; k++) {
         v[k].x = expf_libm(v[k].x - m[k], tb);
         v[k].y = expf_libm(v[k].y - m[k], tb);
         v[k].z = expf_libm(v[k].z - m[k], tb);
         v[k].w = expf_libm(v[k].w - m[k], tb);
       }
 #pragma unroll
-      for (int k = 0; k < 2; k++)
-        if (u0 + 256 * k + tid < units) *reinterpret_cast<float4*>(e[k]) = v[k];
-    }
+      for (int k = 0; k < n; k++)
+        if (u0 + 64 * kWaves * k + tid < units) *reinterpret_cast<float4*>(e[k]) = v[k];
+    };
+    int u0 = 0;
+    for (; u0 + (kHalf ? 64 * kWaves : 0) < units; u0 += 128 * kWaves) exps(u0, std::integral_constant<int, 2>{});
+    if (kHalf && u0 < units) exps(u0, std::integral_constant<int, 1>{});
   }
   __syncthreads();
   // phase 4: in-order denominator, one lane per query
@@ -601,34 +689,33 @@ __global__ __launch_bounds__(256) void attention_kernel(AttnArgs p, int list_rec
 }
 
 // ---------------------------------------------------------------------------
-// Latency form, for batches of few tiles (a single sequence, the latency entry
-// points): one workgroup of 8 waves per (sequence, 8 queries, head), with the
-// arithmetic of attention_kernel<true> in the same order, laid out for a short
-// critical path rather than for throughput:
+// One sequence of at most kLatL tokens (the latency entry points): one workgroup
+// of 8 waves per (8 queries, head), with the arithmetic of attention_kernel<true>
+// in the same order, laid out for a short critical path rather than for
+// throughput (128 keys 6.6 us, attention_kernel's 16-query tiles 7.4; two rows
+// of 128: 11 / 7.6):
 //  * every global load (the Q operands, the K operands of the wave's key
-//    blocks, the head's V rows into LDS) is issued at the start;
-//  * scores: wave w takes the 16-key blocks w, w + 8, ...: MFMA products and
-//    in-order adds exactly as attention_kernel<true>'s phase 1;
+//    block, the head's V rows into LDS) is issued at the start;
+//  * scores: wave w takes the 16-key block w: MFMA products and in-order adds
+//    exactly as attention_kernel<true>'s phase 1;
 //  * exp and the in-order denominator as there;
 //  * p_t = e_t * inv in place (the reference's `s[i] * inv`), then PV on the
 //    VALU, one output (query, dim) per thread: p_t * v_t,d rounded, added in
 //    key order from LDS.
-// dynamic LDS: S[16][s_pitch] scores -> exps, then V[s_pitch - 4][32]
 // ---------------------------------------------------------------------------
+constexpr int kLatL = 128;  // keys: one 16-key block per wave
 constexpr int kLatQ = 8;  // queries per workgroup (MFMA rows 8-15 repeat a query and are not used)
 
-__global__ __launch_bounds__(512) void attention_lat_kernel(AttnArgs p, int tiles_per_seq) {
-  extern __shared__ __attribute__((aligned(16))) float smem[];
+__global__ __launch_bounds__(512) void attention_lat_kernel(AttnArgs p) {
   __shared__ float s_maxw[8][kLatQ];
   __shared__ float s_max[kLatQ], s_inv[kLatQ];
   __shared__ uint64_t s_tab[32];
-  const int pitch = p.s_pitch, lmax = pitch - 4;
-  float* S = smem;                   // [kLatQ][pitch]
-  float* sV = smem + kLatQ * pitch;  // [lmax][32]
-  const int h = blockIdx.x % 12, bt = blockIdx.x / 12, b = bt / tiles_per_seq;
-  const int q0 = (bt - b * tiles_per_seq) * kLatQ;
-  // a single segment whose bounds the host knows (p.len1 > 0): no cu_seqlens load
-  const int s0 = p.len1 > 0 ? 0 : p.cu[b], L = min(p.len1 > 0 ? p.len1 : p.cu[b + 1] - s0, lmax);
+  constexpr int pitch = kLatL + 4;
+  __shared__ __attribute__((aligned(16))) float S[kLatQ * pitch];  // scores -> exps -> probabilities
+  __shared__ __attribute__((aligned(16))) float sV[kLatL * 32];
+  const int h = blockIdx.x % 12, q0 = blockIdx.x / 12 * kLatQ;
+  // bounds that the host knows (p.len1 > 0): no cu_seqlens load
+  const int s0 = p.len1 > 0 ? 0 : p.cu[0], L = min(p.len1 > 0 ? p.len1 : p.cu[1] - s0, min(p.s_pitch - 4, kLatL));
   if (q0 >= L) return;  // workgroup-uniform
   const int nq = min(kLatQ, L - q0);
   const int tid = threadIdx.x, lane = tid & 63;
@@ -651,12 +738,12 @@ __global__ __launch_bounds__(512) void attention_lat_kernel(AttnArgs p, int tile
   // arrived, which waits for V only (the memory counter drains in issue order),
   // so the V and Q/K latencies overlap.  Float4 f = tid + 512 i is key f / 8,
   // dims 4 (f % 8) .. +3.  Every load up to the stores is unconditional (lanes
-  // past the segment load its last float4 and store nothing; K blocks past it
+  // past the segment load its last float4 and store it again; K blocks past it
   // load row L - 1 and are not used) and a scheduling barrier separates the
   // loads from the stores: otherwise the compiler sank each V load to its store
   // and waited for it there, one at a time (or, with a load under a per-lane
   // branch, kept the array in scratch memory).
-  constexpr int kVF = 8;  // float4s per thread at 512 keys
+  constexpr int kVF = 8 * kLatL / 512;  // float4s per thread
   typedef float f4 __attribute__((ext_vector_type(4)));
   f4 vr[kVF];
 #pragma unroll
@@ -666,10 +753,8 @@ __global__ __launch_bounds__(512) void attention_lat_kernel(AttnArgs p, int tile
   }
   float qf[8];  // query q0 + lr (rows past the segment, and lr >= kLatQ, clamped)
   load_dims(qkv + (size_t)min(q0 + min(lr, kLatQ - 1), L - 1) * HQKV, qf);
-  const int nkb = (L + 15) >> 4;  // <= 32: at most 4 blocks per wave
-  float kf[4][8];
-#pragma unroll
-  for (int j = 0; j < 4; j++) load_dims(qkv + H + (size_t)min(16 * (wave + 8 * j) + lr, L - 1) * HQKV, kf[j]);
+  float kf[8];
+  load_dims(qkv + H + (size_t)min(16 * wave + lr, L - 1) * HQKV, kf);
   __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
   for (int i = 0; i < kVF; i++)  // lanes past the segment rewrite its last float4
@@ -678,33 +763,29 @@ __global__ __launch_bounds__(512) void attention_lat_kernel(AttnArgs p, int tile
   // scores of query lr for keys 16kb + 4lg + i (dot32_f32 order) and the row max;
   // keys >= L repeat key L - 1 (clamped rows) and cannot change the max
   float m = -INFINITY;
+  if (16 * wave < L) {  // wave-uniform
+    float acc[4];
 #pragma unroll
-  for (int j = 0; j < 4; j++) {
-    const int kb = wave + 8 * j;
-    if (kb < nkb) {  // wave-uniform
-      float acc[4];
+    for (int c = 0; c < 2; c++) {
+      v16f pr[4];
 #pragma unroll
-      for (int c = 0; c < 2; c++) {
-        v16f pr[4];
+      for (int u = 0; u < 4; u++) pr[u] = mfma_products(kf[4 * c + u], qf[4 * c + u]);
 #pragma unroll
-        for (int u = 0; u < 4; u++) pr[u] = mfma_products(kf[j][4 * c + u], qf[4 * c + u]);
+      for (int blk = 0; blk < 4; blk++)  // dims 16c + 4blk + u, in order
 #pragma unroll
-        for (int blk = 0; blk < 4; blk++)  // dims 16c + 4blk + u, in order
+        for (int u = 0; u < 4; u++)
 #pragma unroll
-          for (int u = 0; u < 4; u++)
-#pragma unroll
-            for (int i = 0; i < 4; i++)
-              acc[i] = (c == 0 && blk == 0 && u == 0) ? pr[0][i] : acc[i] + pr[u][4 * blk + i];
-      }
-      float4 sc;
-      sc.x = acc[0] * kInvSqrtD;
-      sc.y = acc[1] * kInvSqrtD;
-      sc.z = acc[2] * kInvSqrtD;
-      sc.w = acc[3] * kInvSqrtD;
-      if (lr < kLatQ) {
-        *reinterpret_cast<float4*>(&S[lr * pitch + 16 * kb + 4 * lg]) = sc;  // < round16(L) <= lmax
-        m = fmaxf(fmaxf(m, fmaxf(sc.x, sc.y)), fmaxf(sc.z, sc.w));
-      }
+          for (int i = 0; i < 4; i++)
+            acc[i] = (c == 0 && blk == 0 && u == 0) ? pr[0][i] : acc[i] + pr[u][4 * blk + i];
+    }
+    float4 sc;
+    sc.x = acc[0] * kInvSqrtD;
+    sc.y = acc[1] * kInvSqrtD;
+    sc.z = acc[2] * kInvSqrtD;
+    sc.w = acc[3] * kInvSqrtD;
+    if (lr < kLatQ) {
+      *reinterpret_cast<float4*>(&S[lr * pitch + 16 * wave + 4 * lg]) = sc;
+      m = fmaxf(fmaxf(m, fmaxf(sc.x, sc.y)), fmaxf(sc.z, sc.w));
     }
   }
   m = fmaxf(m, __shfl_xor(m, 16, 64));
@@ -724,8 +805,8 @@ __global__ __launch_bounds__(512) void attention_lat_kernel(AttnArgs p, int tile
     const int cols4 = (L + 3) >> 2;
     const float rcols = 1.0f / (float)cols4;  // q = floor((u + 0.5) / cols4): exact for u < 2^13
     const int units = nq * cols4;
-    for (int u0 = 0; u0 < units; u0 += 512) {  // uniform trip count (expf_libm needs all lanes)
-      const int u = min(u0 + tid, units - 1);
+    if (64 * wave < units) {  // wave-uniform (expf_libm needs all lanes); one float4 per lane
+      const int u = min(tid, units - 1);
       const int q = (int)(((float)u + 0.5f) * rcols);
       float* e = &S[q * pitch + 4 * (u - q * cols4)];
       float4 v = *reinterpret_cast<const float4*>(e);
@@ -734,7 +815,7 @@ __global__ __launch_bounds__(512) void attention_lat_kernel(AttnArgs p, int tile
       v.y = expf_libm(v.y - mq, tb);
       v.z = expf_libm(v.z - mq, tb);
       v.w = expf_libm(v.w - mq, tb);
-      if (u0 + tid < units) *reinterpret_cast<float4*>(e) = v;
+      if (tid < units) *reinterpret_cast<float4*>(e) = v;
     }
   }
   __syncthreads();
@@ -779,14 +860,14 @@ __global__ __launch_bounds__(512) void attention_lat_kernel(AttnArgs p, int tile
     s_inv[tid] = inv;
   }
   __syncthreads();
-  // p_t = e_t * inv in place (the reference's normalization), one float4 per thread and step
+  // p_t = e_t * inv in place (the reference's normalization), one float4 per thread
   {
     const int cols4 = (L + 3) >> 2;
     const float rcols = 1.0f / (float)cols4;
     const int units = nq * cols4;
-    for (int u = tid; u < units; u += 512) {
-      const int q = (int)(((float)u + 0.5f) * rcols);
-      float4* e = reinterpret_cast<float4*>(&S[q * pitch + 4 * (u - q * cols4)]);
+    if (tid < units) {
+      const int q = (int)(((float)tid + 0.5f) * rcols);
+      float4* e = reinterpret_cast<float4*>(&S[q * pitch + 4 * (tid - q * cols4)]);
       const float inv = s_inv[q];
       float4 v = *e;
       v.x = v.x * inv; v.y = v.y * inv; v.z = v.z * inv; v.w = v.w * inv;
@@ -1057,19 +1138,15 @@ int attention_pitch(int max_len) {
 }
 
 __global__ __launch_bounds__(256) void cls_attention_kernel(ClsArgs p);
-__global__ __launch_bounds__(512) void attention_lat_kernel(AttnArgs p, int tiles_per_seq);
 
 // allow > 64 KiB of dynamic LDS for the tiled kernel on the current device; called
 // at engine open and by the stand-alone operator, never inside a stream capture
 void init_attention_kernels() {
   const int lds = (int)attention_lds_bytes(attention_pitch(512));
-  (void)hipFuncSetAttribute(reinterpret_cast<const void*>(attention_kernel<true>),
+  (void)hipFuncSetAttribute(reinterpret_cast<const void*>(attention_kernel<true, 0, 4>),
                             hipFuncAttributeMaxDynamicSharedMemorySize, lds);
-  (void)hipFuncSetAttribute(reinterpret_cast<const void*>(attention_kernel<false>),
+  (void)hipFuncSetAttribute(reinterpret_cast<const void*>(attention_kernel<false, 0, 4>),
                             hipFuncAttributeMaxDynamicSharedMemorySize, lds);
-  (void)hipFuncSetAttribute(reinterpret_cast<const void*>(attention_lat_kernel),
-                            hipFuncAttributeMaxDynamicSharedMemorySize,
-                            (int)(sizeof(float) * (16 * (size_t)attention_pitch(512) + 32 * 512)));
 }
 
 // The wide variant (3 workgroups per CU by registers) is faster from rows of
@@ -1087,23 +1164,55 @@ void launch_attention_plan(const AttnArgs& p, hipStream_t st, int split, int max
                      reinterpret_cast<int4*>(p.plan));
 }
 
-// The latency form serves batches of at most this many 32-query tiles
-// (B * ceil(longest / 32)): below it the tiled kernel leaves most CUs idle and
-// its time is the critical path of one workgroup.
-constexpr int kLatMaxTiles = 16;
-static int g_attention_form = 0;  // 0 by the batch, 1 tiled / rows only, 2 latency form only
+// Batches whose 32-query tiles leave CUs idle or end on a long critical path take
+// the latency form's 16-query tiles.  Kernel times in us, 16-query against
+// 32-query tiles (against the two launches by length where those apply; these
+// need the plan kernel's 12 to 19 us first, once per pass): one row of 256
+// keys 11.0 / 14.2, 512: 22.6 / 24.8; 2 x 512: 29.3 / 31.1, 8 x 128: 12.0 / 12.2,
+// 12 x 128: 16.4 / 14.9, 3 x 384: 26.9 / 25.9, 16 x 96: 14.7 / 12.7, so up to kHalfMaxT
+// tokens.  Batches of mixed lengths (16 to 512 keys), whose long rows are the
+// critical path: 1,782 tokens 31.5 / 45.7, 2,843: 44 / 60.6, 5,470: 84 / 91,
+// 9,420: 146 / 146, 13,773: 217 / 210; 128 rows of 64 with one of 512 (8,704) 50 /
+// 54, so up to kHalfMaxMixedT tokens.
+constexpr int kHalfMaxT = 1024, kHalfMaxMixedT = 9000;
+// 16-query tiles (counting the longest row's for every row) whose workgroups, 12
+// per tile, are resident at once at 4 per CU
+constexpr int kHalfResidentTiles = 80;
+// and at 2 per CU with 8 waves each: eight waves against four, 2 x 80 keys 6.2 /
+// 6.7, one row of 320: 12.8 / 13.6, 512 (32 tiles): 22.6 / 23.1; 3 x 256 (48 tiles): 20.4 / 16.8
+constexpr int kHalfWaves8Tiles = 42;
+static int g_attention_form = 0;  // 0 by the batch, 1 tiled (32 queries) / register rows only, 2 latency form only
 void set_attention_form(int form) { g_attention_form = form; }
 int attention_form() { return g_attention_form; }
 
 void launch_attention(const AttnArgs& p, int T, hipStream_t st, bool plan) {
   if (T <= 0 || p.B <= 0) return;
   const int max_len = p.s_pitch - 4;  // round16 of the longest sequence
-  const bool lat = g_attention_form == 2 ||
-                   (g_attention_form == 0 && max_len > 64 && (size_t)p.B * ((max_len + 31) / 32) <= kLatMaxTiles);
-  if (lat) {
-    const int tps = (max_len + kLatQ - 1) / kLatQ;
-    const size_t lds = sizeof(float) * ((size_t)kLatQ * p.s_pitch + (size_t)max_len * 32);
-    hipLaunchKernelGGL(attention_lat_kernel, dim3(p.B * tps * 12), dim3(512), lds, st, p, tps);
+  const bool mixed = 2 * (size_t)max_len * p.B > 3 * (size_t)T;  // the longest row over 1.5 times the mean
+  const bool half = g_attention_form == 2 || (g_attention_form == 0 && max_len > 64 && T <= (mixed ? kHalfMaxMixedT : kHalfMaxT));
+  const int max_tiles = attention_max_tiles(p.B, T);
+  const int records = (int)attention_plan_list_records(p.B, T);
+  if (g_attention_form != 1 && p.B == 1 && max_len > 64 && max_len <= kLatL) {
+    hipLaunchKernelGGL(attention_lat_kernel, dim3(12 * ((max_len + kLatQ - 1) / kLatQ)), dim3(512), 0, st, p);
+    return;
+  }
+  if (half) {
+    const size_t lds = attention_lds_bytes(p.s_pitch) / 2;
+    if (p.B <= kHalfMaxSegs) {
+      const int tps = (max_len + 15) / 16, tiles = p.B * tps;
+      if (tiles <= kHalfWaves8Tiles) {
+        hipLaunchKernelGGL((attention_kernel<true, 2, 8>), dim3(12 * tiles), dim3(512), lds, st, p, tps, 0);
+      } else if (tiles <= kHalfResidentTiles) {
+        hipLaunchKernelGGL((attention_kernel<true, 2, 4>), dim3(12 * tiles), dim3(256), lds, st, p, tps, 0);
+      } else {  // the most tiles an XCD gets: half as many again as the batch has, plus half a segment's
+        const int slots = (3 * ((T + 15 * p.B) / 16) + tps) / 2 + 1;
+        hipLaunchKernelGGL((attention_kernel<true, 2, 4>), dim3(8 * slots), dim3(256), lds, st, p, 0, 0);
+      }
+      return;
+    }
+    if (plan) launch_attention_plan(p, st, 0, max_tiles);
+    hipLaunchKernelGGL((attention_kernel<true, 1, 4>), dim3(2 * 8 * attention_plan_cap(max_tiles)), dim3(256), lds, st, p,
+                       records, 0);
     return;
   }
   if (max_len <= 32) {
@@ -1120,16 +1229,14 @@ void launch_attention(const AttnArgs& p, int T, hipStream_t st, bool plan) {
   // three workgroups per CU.  The grids are sized for the worst case; the
   // surplus workgroups leave after one scalar load (plan_item).
   const bool split = max_len > kAttnLongL && T <= kSplitMaxMean * p.B;
-  const int max_tiles = attention_max_tiles(p.B, T);
   if (plan) launch_attention_plan(p, st, split ? 1 : 0, max_tiles);
   const bool wide = T > kWideMinMeanLen * p.B;
-  const int records = (int)attention_plan_list_records(p.B, T);
   const dim3 grid(8 * attention_plan_cap(max_tiles));
   auto launch = [&](int list, size_t lds) {
     if (wide)
-      hipLaunchKernelGGL(attention_kernel<true>, grid, dim3(256), lds, st, p, records, list);
+      hipLaunchKernelGGL((attention_kernel<true, 0, 4>), grid, dim3(256), lds, st, p, records, list);
     else
-      hipLaunchKernelGGL(attention_kernel<false>, grid, dim3(256), lds, st, p, records, list);
+      hipLaunchKernelGGL((attention_kernel<false, 0, 4>), grid, dim3(256), lds, st, p, records, list);
   };
   if (split) {
     launch(0, attention_lds_bytes(kAttnLongL + 4));

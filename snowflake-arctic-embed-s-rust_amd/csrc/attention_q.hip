@@ -201,7 +201,7 @@ __global__ __launch_bounds__(256) void sme_attention_kernel(AttnArgs p, SmeArgs 
   __shared__ uint64_t s_tab[32];
   int h, b;
   int4 rec;
-  if (!plan_item(reinterpret_cast<const int4*>(p.plan), h, b, rec)) return;  // a surplus workgroup (list 0)
+  if (!plan_item(reinterpret_cast<const int4*>(p.plan), blockIdx.x >> 3, h, b, rec)) return;  // a surplus workgroup (list 0)
   const int nq = rec.w;
   const int s0 = rec.x, L = rec.y, q0 = rec.z;
   // per_seq: sequences under 16 tokens take the exact attention (forward_cls,

@@ -346,13 +346,12 @@ __device__ __forceinline__ int xcd_contiguous(int p, int n) {
 
 // The attention kernels' workgroup -> item map over one list of a tile plan
 // (attention_plan_kernel): workgroup p runs on XCD x = p mod 8 (the hardware's
-// round-robin dispatch) and takes item p / 8 of XCD x's list, whose count and
-// first item are int2 x of the list's header.  The surplus workgroups of the
+// round-robin dispatch) and takes item i (p / 8, or what the kernel makes of it)
+// of XCD x's list, whose count and first item are int2 x of the list's header.  The surplus workgroups of the
 // worst-case grid come last on every XCD and leave after the header load:
 // false for those.  rec = {s0, L, q0, nq}.
-__device__ __forceinline__ bool plan_item(const int4* list, int& h, int& seg, int4& rec) {
+__device__ __forceinline__ bool plan_item(const int4* list, int i, int& h, int& seg, int4& rec) {
   const int2 hx = reinterpret_cast<const int2*>(list)[blockIdx.x & 7];
-  const int i = blockIdx.x >> 3;
   if (i >= hx.x) return false;
   rec = list[kPlanHdr + hx.y + i];
   h = rec.z >> 16;
@@ -361,9 +360,9 @@ __device__ __forceinline__ bool plan_item(const int4* list, int& h, int& seg, in
   rec.w &= 0xff;
   return true;
 }
-__device__ __forceinline__ bool plan_item(const int4* list, int& h, int4& rec) {
+__device__ __forceinline__ bool plan_item(const int4* list, int i, int& h, int4& rec) {
   int seg;
-  return plan_item(list, h, seg, rec);
+  return plan_item(list, i, h, seg, rec);
 }
 
 // index of the segment containing token t: largest b with cu[b] <= t (cu has B+1 entries)

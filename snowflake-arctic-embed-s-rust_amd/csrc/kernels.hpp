@@ -176,7 +176,7 @@ struct AttnArgs {
   uint32_t* rowmax;        // [T] or null
   int s_pitch;             // score row pitch: attention_pitch(max sequence length)
   int skip_from = 0;       // attention_rows_kernel: segments of at least this many tokens are left out (0: none)
-  int len1 = 0;            // B == 1 and cu_seqlens = {0, len1} known on the host: the latency form skips its load
+  int len1 = 0;            // B == 1 and cu_seqlens = {0, len1} known on the host: the latency form needs no load
 };
 int attention_pitch(int max_len);
 size_t attention_lds_bytes(int s_pitch);
@@ -206,7 +206,7 @@ hipError_t noalloc_plan_scratch(int** plan);
 void launch_attention(const AttnArgs& p, int T, hipStream_t st, bool plan = true);
 // split = 1: rows of more than 384 keys in the plan's second list
 void launch_attention_plan(const AttnArgs& p, hipStream_t st, int split, int max_tiles);
-// exact-attention kernel choice for later launches: 0 by the batch, 1 tiled /
+// exact-attention kernel choice for later launches: 0 by the batch, 1 tiled (32 queries) /
 // register rows only, 2 the latency form only (a test hook; same bits)
 void set_attention_form(int form);
 int attention_form();  // the current setting

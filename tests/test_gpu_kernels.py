@@ -511,13 +511,13 @@ def test_gelu_bit_exact_over_float_sample(torch_gpu):
     assert np.array_equal(bits(y)[~nan], bits(ref)[~nan])
 
 
-# exact attention has five code paths, chosen by the batch's shape: the latency
-# form (at most 16 tiles of 32 queries, longest > 64), register-resident rows
-# (longest <= 32, <= 64), else the tiled kernel with the wide (mean > 48) or the
-# narrow operand layout; these length sets reach each.  The tiled kernel runs the
-# rows of more than 400 keys in a launch of their own when the batch's mean
-# length is at most 448 ("tiled_long": both sides of 400, with short rows;
-# "tiled_long_mean410"), else every row in one launch ("tiled_long32")
+# exact attention has five code paths: register-resident rows (longest <= 32, <= 64),
+# the latency form for small batches and mixed ones (LATENCY_LENS below), else the tiled
+# kernel with the wide (mean > 48) or the narrow operand layout, which runs the rows
+# of more than 400 keys in a launch of their own when the batch's mean length is at
+# most 448 ("tiled_long": both sides of 400, with short rows; "tiled_long_mean410"), else
+# every row in one launch ("tiled_long32").  test_attention_latency_form_choices takes
+# the "tiled" sets, which are small, through the tiled kernel
 ATTN_LENS = {"tiled_wide": [1, 2, 17, 31, 32, 33, 64, 65, 130, 512, 3],
              "tiled_long": [384, 385, 17, 400, 401, 408, 409, 431, 1, 449, 480, 500, 511, 512, 24, 25, 200],
              "tiled_long_mean410": [512, 500, 450, 400, 385, 512, 480, 449, 33, 384],
@@ -556,6 +556,45 @@ def test_attention_bit_exact(torch_gpu, attention_form, lens):
     torch.cuda.synchronize()
     ref = orc.attention(qkv, cu)
     assert np.array_equal(bits(ctx_d.cpu().numpy()), bits(ref))
+
+
+# the latency form's choices: up to 16 segments its workgroups find their items (up to
+# 42 tiles of 16 queries with eight waves, up to 80 all resident at once, else longest
+# first), from 17 on the plan's, one row of up to 128 has a kernel of its own; by the batch up to 1,024 tokens, or 9,000 where the longest row is over
+# 1.5 times the mean.  Each set takes the latency form and the 32-query tiles.
+LATENCY_LENS = {"one_65": [65], "one_129": [129], "one_497": [497],
+                "two": [81, 17], "tiles_42": [336, 335], "tiles_44": [337, 340],
+                "resident_80_tiles": [256, 241, 255, 250, 242],
+                "longest_first": [16, 257, 1, 512, 512, 15, 31, 33, 48, 512, 49, 500, 2, 64, 65],
+                "segments_16": [96, 95, 97] + [15, 16, 17, 31, 32, 33, 47, 48, 49, 63, 64, 65, 1],
+                "segments_17": [96, 95, 97] + [15, 16, 17, 31, 32, 33, 47, 48, 49, 63, 64, 65, 1, 2],
+                "even_1024": [128] * 8, "even_1025": [128] * 7 + [129],
+                "mixed_9000": [512] * 4 + [200] * 34 + [152], "mixed_9001": [512] * 4 + [200] * 34 + [153],
+                **{k: v for k, v in ATTN_LENS.items() if k.startswith("tiled")}}
+
+
+@pytest.mark.parametrize("form", [0, 1, 2], ids=["by_shape", "tiles32", "latency_form"])
+@pytest.mark.parametrize("lens", list(LATENCY_LENS.values()), ids=list(LATENCY_LENS))
+def test_attention_latency_form_choices(torch_gpu, form, lens):
+    """Bit-exact on both sides of each of the latency form's limits, through the operator that
+    finds the longest row itself and through the one that is given a bound (512 here)."""
+    torch = torch_gpu
+    cu = np.concatenate([[0], np.cumsum(lens)]).astype(np.int32)
+    T = int(cu[-1])
+    rng = np.random.default_rng(len(lens) + T)
+    qkv = rng.normal(0, 1.0, (T, 1152)).astype(f32)
+    qkv_d, cu_d = dev(torch, qkv), dev(torch, cu)
+    ctx_d = torch.full((2, T, 384), float("nan"), dtype=torch.float32, device="cuda")
+    print("attention form", form, "segments", len(lens), "tokens", T, flush=True)
+    ae.set_attention_form(form)
+    try:
+        ae.attention_varlen(qkv_d.data_ptr(), cu_d.data_ptr(), len(lens), T, ctx_d[0].data_ptr())
+        ae.attention_varlen_noalloc(qkv_d.data_ptr(), cu_d.data_ptr(), len(lens), T, 512, ctx_d[1].data_ptr())
+        torch.cuda.synchronize()
+    finally:
+        ae.set_attention_form(0)
+    ref = bits(orc.attention(qkv, cu))
+    assert np.array_equal(bits(ctx_d[0].cpu().numpy()), ref) and np.array_equal(bits(ctx_d[1].cpu().numpy()), ref)
 
 
 @pytest.mark.parametrize("lens", [[1, 2, 7, 8, 9, 15, 16, 17, 31, 32, 33], [5, 40, 97, 300, 1, 512, 63],
