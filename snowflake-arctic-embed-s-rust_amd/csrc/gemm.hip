@@ -761,6 +761,22 @@ __global__ __launch_bounds__(512) void gemm_small_kernel(GemmArgs p, LnArgs ln, 
       epos(k, er, ec4);
       resv[k] = *reinterpret_cast<const float4*>(p.res + (size_t)min(m0 + er, p.M - 1) * p.N + col0 + ec4 * 4);
     }
+    if constexpr (LN) {
+      if (p.res_stats) {  // the residual is the LayerNorm of these rows, recomputed as that LayerNorm forms it
+#pragma unroll
+        for (int k = 0; k < kEk; k++) {
+          int er, ec4;
+          epos(k, er, ec4);
+          const float2 st = p.res_stats[min(m0 + er, p.M - 1)];
+          const float4 g = *reinterpret_cast<const float4*>(p.res_gamma + col0 + ec4 * 4);
+          const float4 b = *reinterpret_cast<const float4*>(p.res_beta + col0 + ec4 * 4);
+          resv[k].x = (resv[k].x - st.x) * st.y * g.x + b.x;
+          resv[k].y = (resv[k].y - st.x) * st.y * g.y + b.y;
+          resv[k].z = (resv[k].z - st.x) * st.y * g.z + b.z;
+          resv[k].w = (resv[k].w - st.x) * st.y * g.w + b.w;
+        }
+      }
+    }
   }
 
   // the A tile into LDS: int8 A as loaded, f32 A quantized as astore does above,
@@ -1090,15 +1106,28 @@ static bool small_gemm(const GemmArgs& p) { return p.M <= kSmallM && p.K <= kSma
 // the 8 waves of 16 x 48 workgroups (gemm_small_kernel KS = 8)
 constexpr int kSplitMinK = 1024;
 
-// ln != null: N = 384, kEpiF32, small_gemm(p); the epilogue applies *ln to each
-// output row and p.out is not written
+// The attention output GEMM with LN1 (kAF32QSmooth, N = K = 384) takes
+// gemm_small_kernel's 16-row workgroups of 8 waves while one per compute unit
+// covers the rows.  Both forms are latency chains there (quantize, six K steps,
+// two in-order sums of 384), and gemm_ln_rows_kernel's 32-row workgroups of 4
+// waves take twice as long for theirs on half the compute units: in passes of
+// 1,280, 2,844 and 4,096 rows it took 7.5, 7.2 and 6.7 us more per layer (771 ->
+// 689, 1,111 -> 1,032, 1,701 -> 1,627 us per pass).  With more rows the second
+// workgroup per CU waits for registers: 5,200 rows 1,023 -> 1,029, 8,000 rows
+// 1,789 -> 1,781.
+static bool ln_rows16(const GemmArgs& p) { return small_gemm(p) || (p.M + 15) / 16 <= device_cu_count(); }
+
+// ln != null: N = 384, kEpiF32, K <= kSmallMaxK, ln_rows16(p); the epilogue
+// applies *ln to each output row and p.out is not written
 template <int AM, int EM>
 static void launch_variant(GemmArgs p, hipStream_t st, const LnArgs* ln = nullptr) {
   const int mt16 = (p.M + 15) / 16;
+  if (ln) {
+    hipLaunchKernelGGL((gemm_small_kernel<AM, kEpiF32, true, 1>), dim3(mt16), dim3(512), 0, st, p, *ln, PreArgs{});
+    return;
+  }
   if (small_gemm(p)) {
-    if (ln) {
-      hipLaunchKernelGGL((gemm_small_kernel<AM, kEpiF32, true, 1>), dim3(mt16), dim3(512), 0, st, p, *ln, PreArgs{});
-    } else if (EM == kEpiF32 && p.K >= kSplitMinK && p.K % 512 == 0) {
+    if (EM == kEpiF32 && p.K >= kSplitMinK && p.K % 512 == 0) {
       if (AM != kAI8 && mt16 * (p.N / 48) < 256)  // 8-row tiles: half the f32 A per workgroup, twice the workgroups
         hipLaunchKernelGGL((gemm_small_kernel<AM, kEpiF32, false, 8, 8>), dim3(((p.M + 7) / 8) * (p.N / 48)),
                            dim3(512), 0, st, p, LnArgs{}, PreArgs{});
@@ -1165,7 +1194,7 @@ void launch_gemm_ln(const GemmArgs& p, int amode, const LnArgs& ln, hipStream_t 
     launch_ln_quant(l, kLnSrcF32, st);
     return;
   }
-  if (!small_gemm(p)) {  // many rows: kAF32QSmooth, N = K = 384, with residual
+  if (!ln_rows16(p)) {  // many rows: kAF32QSmooth, N = K = 384, with residual
     hipLaunchKernelGGL(gemm_ln_rows_kernel, dim3((p.M + kLrRows - 1) / kLrRows), dim3(256), 0, st, p, ln);
     return;
   }

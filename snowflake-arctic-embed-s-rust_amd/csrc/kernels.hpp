@@ -32,8 +32,7 @@ struct GemmArgs {
   const float* g_smooth;      // kEpiGelu: next layer inv_smooth [N]
   uint32_t* g_rowmax;         // kEpiGelu: [M], pre-set to bits(1e-8f)
   int col_fast;               // set by launch_gemm: workgroup order (column tile fastest)
-  // gemm_ln_rows_kernel only (launch_gemm_ln's many-rows path; the caller sets
-  // them only there): res holds a LayerNorm's input rows, and the residual is
+  // launch_gemm_ln only, in a call that gemm_fuses_ln holds for: res holds a LayerNorm's input rows, and the residual is
   // that LayerNorm's output, recomputed as ((res - mean) * rstd) * res_gamma +
   // res_beta from its (mean, rstd) per row
   const float2* res_stats = nullptr;

@@ -193,6 +193,34 @@ def test_gemm_then_layernorm_bit_exact(torch_gpu, m):
     assert np.array_equal(bits(sc_d.cpu().numpy()), bits(rsc))
 
 
+@pytest.mark.parametrize("m", [1025, 4095, 4096, 4097])
+def test_gemm_then_layernorm_tile_heights(torch_gpu, m):
+    """The same on both sides of the rule for the tile height (16 rows while one workgroup per
+    compute unit covers them, 32 beyond), with partial last tiles, the output in the residual's place."""
+    torch = torch_gpu
+    n = k = 384
+    w, ws, b, s = linear_inputs(n, k, 12)
+    rng = np.random.default_rng(m)
+    x, res = rng.normal(0, 1.5, (m, k)).astype(f32), rng.normal(0, 1, (m, n)).astype(f32)
+    gamma, beta = (1 + rng.normal(0, 0.05, n)).astype(f32), rng.normal(0, 0.02, n).astype(f32)
+    ln_s = (rng.uniform(0.5, 2.0, n) ** -1).astype(f32)
+    rowmax = np.maximum(np.abs(x * s).max(1), f32(1e-8)).astype(f32)
+    lin = ae.Linear(w, ws, b, s)
+    x_d, rm_d, res_d = dev(torch, x), dev(torch, rowmax.view(np.uint32).astype(np.int32)), dev(torch, res)
+    s_d, g_d, b_d, ls_d = dev(torch, s), dev(torch, gamma), dev(torch, beta), dev(torch, ln_s)
+    q_d = torch.zeros((m, n), dtype=torch.int8, device="cuda")
+    sc_d = torch.zeros(m, dtype=torch.float32, device="cuda")
+    lin.gemm_ln(m, x_d.data_ptr(), rm_d.data_ptr(), s_d.data_ptr(), res_d.data_ptr(), g_d.data_ptr(), b_d.data_ptr(),
+                ls_d.data_ptr(), res_d.data_ptr(), q_d.data_ptr(), sc_d.data_ptr())
+    torch.cuda.synchronize()
+    lin.close()
+    q, sc = orc.smooth_quant_rows(x, s)
+    ry, rq, rsc = orc.ln_quant_rows(orc.gemm(q, sc, w, ws, b, res), gamma, beta, ln_s)
+    assert np.array_equal(bits(res_d.cpu().numpy()), bits(ry))
+    assert np.array_equal(q_d.cpu().numpy(), rq)
+    assert np.array_equal(bits(sc_d.cpu().numpy()), bits(rsc))
+
+
 @pytest.mark.parametrize("m", [1, 45, 130])
 def test_gemm_gelu_epilogue_bit_exact(torch_gpu, m):
     """FFN-up GEMM with the GELU * inv_smooth epilogue and the row absmax."""
