@@ -488,7 +488,7 @@ int run_forward(ae_workspace* ws, const uint16_t* ids, const int* cu, int B, int
                                           nullptr),
                                 ln_args(ws->tmp, ws->hidden, ln2_w, ln2_b, D.qkv_smooth, nullptr, nullptr,
                                         ws->rowmax_ctx, T, ws->rowmax_g),
-                                kEpiF32, st);
+                                st);
       } else {
         GemmArgs g = gemm_args(D.qkv, T, ws->act_q, ws->act_scale, nullptr, nullptr, nullptr, ws->qkv, nullptr, nullptr);
         // Q is read once by the attention; K and V many times: only K and V
@@ -519,7 +519,7 @@ int run_forward(ae_workspace* ws, const uint16_t* ids, const int* cu, int B, int
                            pre,
                            ln_args(nullptr, ws->tmp, D.ln1_w, D.ln1_b, D.ffn_inter.inv_smooth, nullptr, nullptr,
                                    nullptr, T),
-                           kEpiGelu, st);
+                           st);
       }
       {  // residual LN1(h) in tmp, written in place
         KernelTimer kt(ws, st, AE_KERNEL_GEMM_FFN_DOWN);
@@ -577,7 +577,7 @@ int run_forward(ae_workspace* ws, const uint16_t* ids, const int* cu, int B, int
     launch_gemm_ln_prologue(gemm_args(D.kv_only, T, ws->tmp, nullptr, nullptr, nullptr, nullptr, kv, nullptr, nullptr),
                             ln_args(ws->tmp, ws->hidden, ln2_w, ln2_b, D.qkv_smooth, ws->act_q, ws->act_scale, nullptr,
                                     T),
-                            kEpiF32, st);
+                            st);
   } else {
     gemm(D.kv_only, T, ws->act_q, kAI8, ws->act_scale, nullptr, nullptr, nullptr, kv, kEpiF32, nullptr, nullptr);
   }
@@ -612,7 +612,7 @@ int run_forward(ae_workspace* ws, const uint16_t* ids, const int* cu, int B, int
                        pre,
                        ln_args(nullptr, ws->tmp_c, D.ln1_w, D.ln1_b, D.ffn_inter.inv_smooth, nullptr, nullptr, nullptr,
                                B),
-                       kEpiGelu, st);
+                       st);
     gemm(D.ffn_out, B, ws->g_c, kAF32Q, nullptr, ws->rowmax_g_c, nullptr, ws->tmp_c, ws->tmp_c, kEpiF32, nullptr,
          nullptr);
     launch_final_ln_l2(B, ws->tmp_c, D.ln2_w, D.ln2_b, out, st);

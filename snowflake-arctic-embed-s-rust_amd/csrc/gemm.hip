@@ -29,6 +29,7 @@
 #include <atomic>
 
 #include <algorithm>
+#include <type_traits>
 
 #include "device_common.hpp"
 #include "kernels.hpp"
@@ -602,8 +603,8 @@ __global__ __launch_bounds__(256, 3) void gemm_ln_rows_kernel(GemmArgs p, LnArgs
 // LayerNorm + SmoothQuant of `ln` to its 16 output rows, reference
 // src/simd_math.rs:208-247, and p.out is not written); KS = 2: 192 columns;
 // KS = 8: 48 columns (a workgroup streams an eighth of the weights of the
-// KS = 1 form), for long K and for a LayerNorm prologue (four times the
-// workgroups of KS = 2, each normalizing its 16 rows).
+// KS = 1 form), for long K.  A LayerNorm prologue takes the KS that fills the
+// compute units in one round (launch_gemm_ln_prologue).
 // ---------------------------------------------------------------------------
 constexpr int kSmallMaxK = 1536;
 constexpr int kSmallPitch = kSmallMaxK + 16;  // LDS bytes per A row: conflict-free fragment reads
@@ -617,7 +618,7 @@ __global__ __launch_bounds__(512) void gemm_small_kernel(GemmArgs p, LnArgs ln, 
   constexpr int RPW = 16 / KS, kPos = RPW * kF4, kEk = (kPos + 63) / 64;  // epilogue rows / float4s per wave
   constexpr int kRing = KS == 1 ? 6 : 3;  // B ring depth (K steps in flight per wave)
   constexpr bool kLnIn = AM == kALn || AM == kAPreLn;  // a LayerNorm in front of the GEMM
-  static_assert(KS == 1 || KS == 2 || KS == 8, "K splits");
+  static_assert(KS == 1 || KS == 2 || KS == 4 || KS == 8, "K splits");
   static_assert(RT == 16 || (RT == 8 && KS == 8 && !LN && AM != kALn && AM != kAPreLn), "8-row tiles: KS = 8 only");
   static_assert(!LN || (KS == 1 && EM == kEpiF32), "fused LayerNorm: 16 rows x 384 columns");
   static_assert(!kLnIn || !LN, "LayerNorm prologue or epilogue");
@@ -1167,22 +1168,38 @@ bool gemm_fuses_ln(const GemmArgs& p, int amode) {
 
 bool gemm_small_path(int m) { return m > 0 && m <= kSmallM; }
 
-void launch_gemm_ln_prologue(const GemmArgs& p, const LnArgs& ln, int emode, hipStream_t st) {
+// A workgroup with a LayerNorm in front (up to 216 VGPRs, 8 waves) has a compute
+// unit to itself, and most of its time is that LayerNorm, whatever its columns.
+// So the K split is the largest whose workgroups still run in one round: 48
+// columns each up to 160 rows (N = 1152), 96 up to 336, 192 up to 672, then 384.
+// Passes with 48 / 96 / 192 / 384 columns: 128 rows 411 / 412 / 416 / 427 us,
+// 256 rows 523 / 472 / 476 / 485, 512 rows 737 / 673 / 625 / 635, 1,024 rows
+// 1,132 / 962 / 907 / 861 (48 columns throughout before: the QKV kernel of a
+// 509-token document took 19.3 us in three rounds).
+void launch_gemm_ln_prologue(const GemmArgs& p, const LnArgs& ln, hipStream_t st) {
   if (p.M <= 0 || p.M > kSmallM || p.K != 384) return;
-  const dim3 grid(((p.M + 15) / 16) * (p.N / 48));
-  if (emode == kEpiGelu)
-    hipLaunchKernelGGL((gemm_small_kernel<kALn, kEpiGelu, false, 8>), grid, dim3(512), 0, st, p, ln, PreArgs{});
-  else
-    hipLaunchKernelGGL((gemm_small_kernel<kALn, kEpiF32, false, 8>), grid, dim3(512), 0, st, p, ln, PreArgs{});
+  const int mt = (p.M + 15) / 16, cus = device_cu_count();
+  auto run = [&](auto ks) {
+    hipLaunchKernelGGL((gemm_small_kernel<kALn, kEpiF32, false, ks>), dim3(mt * (p.N / (384 / ks))), dim3(512), 0, st,
+                       p, ln, PreArgs{});
+  };
+  if (mt * (p.N / 48) <= cus) run(std::integral_constant<int, 8>{});
+  else if (mt * (p.N / 96) <= cus) run(std::integral_constant<int, 4>{});
+  else if (mt * (p.N / 192) <= cus) run(std::integral_constant<int, 2>{});
+  else run(std::integral_constant<int, 1>{});
 }
 
-void launch_gemm_pre_ln(const GemmArgs& p, const PreArgs& pre, const LnArgs& ln, int emode, hipStream_t st) {
+void launch_gemm_pre_ln(const GemmArgs& p, const PreArgs& pre, const LnArgs& ln, hipStream_t st) {
   if (p.M <= 0 || p.M > kSmallM || p.K != 384) return;
-  const dim3 grid(((p.M + 15) / 16) * (p.N / 192));
-  if (emode == kEpiGelu)
-    hipLaunchKernelGGL((gemm_small_kernel<kAPreLn, kEpiGelu, false, 2>), grid, dim3(512), 0, st, p, ln, pre);
+  // 192 columns per workgroup while these run in one round (512 rows at N =
+  // 1536), 384 beyond
+  const int mt = (p.M + 15) / 16;
+  if (mt * (p.N / 192) <= device_cu_count())
+    hipLaunchKernelGGL((gemm_small_kernel<kAPreLn, kEpiGelu, false, 2>), dim3(mt * (p.N / 192)), dim3(512), 0, st, p,
+                       ln, pre);
   else
-    hipLaunchKernelGGL((gemm_small_kernel<kAPreLn, kEpiF32, false, 2>), grid, dim3(512), 0, st, p, ln, pre);
+    hipLaunchKernelGGL((gemm_small_kernel<kAPreLn, kEpiGelu, false, 1>), dim3(mt * (p.N / 384)), dim3(512), 0, st, p,
+                       ln, pre);
 }
 
 void launch_gemm_ln(const GemmArgs& p, int amode, const LnArgs& ln, hipStream_t st) {

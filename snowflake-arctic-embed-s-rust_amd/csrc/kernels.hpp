@@ -142,7 +142,7 @@ bool gemm_fuses_ln(const GemmArgs& p, int amode);
 // workgroup's prologue; the workgroups of the first column tile also store the
 // LayerNorm's outputs (ln.dst, and ln.q / ln.scale / ln.rowmax_init* when set).
 // ln.dst must not alias p.A.
-void launch_gemm_ln_prologue(const GemmArgs& p, const LnArgs& ln, int emode, hipStream_t st);
+void launch_gemm_ln_prologue(const GemmArgs& p, const LnArgs& ln, hipStream_t st);
 // The GEMM in front of such a LayerNorm (kAPreLn): x = fma(f32(q(A) . W^T), sa * ws,
 // bias + res) with A [M,384] f32 quantized on load as kAF32QSmooth does (sa =
 // max_abs / 127 from a_rowmax), W [384,384] pre-swizzled.
@@ -158,7 +158,7 @@ struct PreArgs {
 // Few rows: launch_gemm_ln_prologue with the LayerNorm's input rows computed in
 // every workgroup by `pre` (the attention-output GEMM in front of LN1, then the
 // FFN-up GEMM): one kernel instead of two.  ln.dst must not alias pre.res or pre.A.
-void launch_gemm_pre_ln(const GemmArgs& p, const PreArgs& pre, const LnArgs& ln, int emode, hipStream_t st);
+void launch_gemm_pre_ln(const GemmArgs& p, const PreArgs& pre, const LnArgs& ln, hipStream_t st);
 // whether launch_gemm takes the few-rows kernels for m rows (and the prologue form applies)
 bool gemm_small_path(int m);
 

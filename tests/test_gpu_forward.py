@@ -377,6 +377,23 @@ def test_layer_prefix_state(engine, ws, oracle_model, layers):
     assert np.array_equal(h, rh) and np.array_equal(q, rq) and np.array_equal(sc, rsc)
 
 
+@pytest.mark.parametrize("total", [160, 161, 336, 337, 512, 513, 672, 673, 1024])
+def test_layer_prefix_state_few_row_column_splits(engine, oracle_model, total):
+    """The few-row kernels with a LayerNorm in front, on both sides of each change of the columns per
+    workgroup (QKV: 48 up to 160 rows, 96 up to 336, 192 up to 672, 384 beyond; FFN-up: 192 up to
+    512 rows, 384 beyond): state after two layers bit-exact against the oracle."""
+    rng = np.random.default_rng(total)
+    lens = [total] if total <= 300 else [300, total - 300] if total <= 812 else [300, 300, total - 600]
+    seqs = [np.concatenate([[101], rng.integers(1000, 30522, n - 2), [102]]).astype(np.uint16) for n in lens]
+    w = engine.workspace(total + 512, len(lens))
+    try:
+        h, q, sc = engine.forward_prefix(w, seqs, 2)
+    finally:
+        w.close()
+    rh, rq, rsc = oracle_model.run_prefix(seqs, 2)
+    assert np.array_equal(h, rh) and np.array_equal(q, rq) and np.array_equal(sc, rsc)
+
+
 @pytest.mark.parametrize("n,lo,hi,layers", [(8, 300, 512, 1), (10, 400, 512, 2)], ids=["T~3k", "T~4.6k"])
 def test_layer_prefix_state_many_rows(engine, oracle_model, n, lo, hi, layers):
     """The many-row kernels (past the few-row path's 1,024 rows): the attention output GEMM fused
