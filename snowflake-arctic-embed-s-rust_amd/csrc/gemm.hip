@@ -1107,6 +1107,20 @@ static bool small_gemm(const GemmArgs& p) { return p.M <= kSmallM && p.K <= kSma
 // the 8 waves of 16 x 48 workgroups (gemm_small_kernel KS = 8)
 constexpr int kSplitMinK = 1024;
 
+// int8 A with more rows than kSmallM (kEpiF32) keeps the 16-row workgroups while
+// these are the faster: their whole A tile is in flight at once, where
+// gemm_w8a8_kernel's K loop is a chain of 6 or 24 steps of 64 behind a barrier
+// each on a few 64 x 192 tiles.  K = 384: one round of them, three per compute
+// unit (N = 1152: 1,280 rows 6.6 -> 5.2 us, 2,048 rows 7.1 -> 6.4, but 2,843 rows
+// 8.2 -> 8.9; N = 1536: 1,536 rows 7.0 -> 6.4, 2,048 rows 7.5 -> 8.1).  K = 1536:
+// four rounds (N = 384: 1,280 rows 17.9 -> 6.8 us, 2,843 rows 18.0 -> 11.8, 5,500
+// rows 21.4 -> 18.6, but 8,192 rows 22.3 -> 26.0).
+static bool int8_rows16(const GemmArgs& p) {
+  const long mt = (p.M + 15) / 16, cus = device_cu_count();
+  if (p.K == 384) return mt * (p.N / 192) <= 3 * cus;
+  return p.K >= kSplitMinK && p.K <= kSmallMaxK && p.K % 512 == 0 && mt * (p.N / 48) <= 4 * 3 * cus;
+}
+
 // The attention output GEMM with LN1 (kAF32QSmooth, N = K = 384) takes
 // gemm_small_kernel's 16-row workgroups of 8 waves while one per compute unit
 // covers the rows.  Both forms are latency chains there (quantize, six K steps,
@@ -1127,7 +1141,7 @@ static void launch_variant(GemmArgs p, hipStream_t st, const LnArgs* ln = nullpt
     hipLaunchKernelGGL((gemm_small_kernel<AM, kEpiF32, true, 1>), dim3(mt16), dim3(512), 0, st, p, *ln, PreArgs{});
     return;
   }
-  if (small_gemm(p)) {
+  if (small_gemm(p) || (AM == kAI8 && EM == kEpiF32 && int8_rows16(p))) {
     if (EM == kEpiF32 && p.K >= kSplitMinK && p.K % 512 == 0) {
       if (AM != kAI8 && mt16 * (p.N / 48) < 256)  // 8-row tiles: half the f32 A per workgroup, twice the workgroups
         hipLaunchKernelGGL((gemm_small_kernel<AM, kEpiF32, false, 8, 8>), dim3(((p.M + 7) / 8) * (p.N / 48)),

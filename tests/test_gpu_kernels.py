@@ -110,6 +110,30 @@ def test_gemm_row_stationary_tiles(torch_gpu, m, n):
     assert np.all(np.isfinite(out))
 
 
+@pytest.mark.parametrize("m,n,k", [(1025, 384, 384), (2048, 1152, 384), (2049, 1152, 384), (1537, 1536, 384),
+                                   (1025, 384, 1536), (6144, 384, 1536), (6145, 384, 1536), (1100, 768, 1024)])
+@pytest.mark.parametrize("with_res", [False, True])
+def test_gemm_int8_tile_heights(torch_gpu, m, n, k, with_res):
+    """Both sides of the rule that keeps 16-row workgroups beyond 1,024 rows, with partial last tiles;
+    the first, last and 48 random rows bit for bit."""
+    torch = torch_gpu
+    w, ws, b, s = linear_inputs(n, k, n + k + m)
+    rng = np.random.default_rng(m)
+    a, sa = rng.integers(-127, 128, (m, k), dtype=np.int8), rng.uniform(0.01, 0.1, m).astype(f32)
+    res = rng.normal(0, 1, (m, n)).astype(f32) if with_res else None
+    lin = ae.Linear(w, ws, b, s)
+    a_d, sa_d = dev(torch, a), dev(torch, sa)
+    res_d = dev(torch, res) if with_res else None
+    out_d = torch.full((m, n), float("nan"), dtype=torch.float32, device="cuda")
+    lin.gemm(m, a_d.data_ptr(), sa_d.data_ptr(), res_d.data_ptr() if with_res else None, out_d.data_ptr())
+    torch.cuda.synchronize()
+    lin.close()
+    rows = np.unique(np.r_[0:16, m - 17:m, rng.integers(0, m, 48)])
+    out = out_d.cpu().numpy()
+    assert not np.isnan(out).any()
+    assert np.array_equal(bits(out[rows]), bits(orc.gemm(a[rows], sa[rows], w, ws, b, res[rows] if with_res else None)))
+
+
 def test_gemm_extreme_accumulators(torch_gpu):
     torch = torch_gpu
     n, k, m = 384, 1536, 3
