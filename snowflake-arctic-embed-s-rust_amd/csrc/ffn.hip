@@ -122,8 +122,16 @@ __device__ unsigned long long g_ffn_repairs[2];
 // Otherwise (rows whose largest v is below 0.57) a second scan evaluates every
 // element whose bound reaches M1.  The candidates of a wave (a few) go to a list
 // in LDS first, so that one gelu_exact serves them all.
-template <int NR, int kP, bool kFast>
-__global__ __launch_bounds__(kThreads, 2) void ffn_kernel(FfnArgs p) {
+//
+// kLn (16-row workgroups): the LayerNorm + SmoothQuant of the output rows (`ln`,
+// with ln_quant_kernel's arithmetic in its order) follows in the same kernel,
+// its 32 threads per row and in-order sums working on the rows in sQ's space.
+// As a launch of its own it took 7.1 us at 1,280 rows and 7.9 at 3,769, most of
+// it the launch and the rows' way through memory: passes of 1,280 rows 651 -> 616
+// us, 2,844 rows 1,031 -> 993, 4,096 rows 1,622 -> 1,579.
+template <int NR, int kP, bool kFast, bool kLn = false>
+__global__ __launch_bounds__(kThreads, 2) void ffn_kernel(FfnArgs p, LnArgs ln) {
+  static_assert(!kLn || NR * kP == 1, "LayerNorm of 16 rows by 512 threads");
   constexpr int RP = 16 * NR, R = RP * kP;  // token rows per pass and per workgroup
   __shared__ __attribute__((aligned(16))) int8_t sA[R * kAPitch];
   // the quantized intermediate; before a pass's quantization its rows hold the waves' candidate lists
@@ -459,6 +467,19 @@ __global__ __launch_bounds__(kThreads, 2) void ffn_kernel(FfnArgs p) {
     for (int n = 0; n < kDnCB; n++)
       res[i][n] = __builtin_nontemporal_load(
           reinterpret_cast<const v4f*>(p.res + (size_t)min(m0 + i * 16 + fr, p.M - 1) * kH + dcol + n * 16 + fq * 4));
+  // kLn: thread t takes float4 columns t % 32 + 32 i of row t / 32
+  constexpr int kLnPitch = 388;  // floats
+  static_assert(16 * kLnPitch * 4 <= 16 * kQPitch, "the LayerNorm's rows fit in sQ");
+  v4f lg[3], lb[3], lsm[3];
+  if constexpr (kLn) {
+#pragma unroll
+    for (int i = 0; i < 3; i++) {
+      const int c = ((tid & 31) + 32 * i) * 4;
+      lg[i] = *reinterpret_cast<const v4f*>(ln.gamma + c);
+      lb[i] = *reinterpret_cast<const v4f*>(ln.beta + c);
+      lsm[i] = *reinterpret_cast<const v4f*>(ln.smooth + c);
+    }
+  }
   __syncthreads();  // sQ complete
   v4i acc2[kRB][kDnCB];
 #pragma unroll
@@ -485,6 +506,8 @@ __global__ __launch_bounds__(kThreads, 2) void ffn_kernel(FfnArgs p) {
     ws2[n] = *reinterpret_cast<const v4f*>(p.w2_scale + dcol + n * 16 + fq * 4);
     b2[n] = *reinterpret_cast<const v4f*>(p.b2 + dcol + n * 16 + fq * 4);
   }
+  float* T = reinterpret_cast<float*>(sQ);  // kLn: the output rows [16][kLnPitch]
+  if constexpr (kLn) __syncthreads();       // every wave's FFN-down is done with sQ
 #pragma unroll
   for (int i = 0; i < kRB; i++) {
     const float s = sMax[i * 16 + fr] / 127.0f;  // scale = max_abs / 127.0
@@ -496,6 +519,51 @@ __global__ __launch_bounds__(kThreads, 2) void ffn_kernel(FfnArgs p) {
       for (int r = 0; r < 4; r++) o[r] = fmaf((float)acc2[i][n][r], s * ws2[n][r], b2[n][r] + res[i][n][r]);
       if (row < p.M)  // streaming store: keeps the weights resident in L2
         __builtin_nontemporal_store(o, reinterpret_cast<v4f*>(p.out + (size_t)row * kH + dcol + n * 16 + fq * 4));
+      if constexpr (kLn) *reinterpret_cast<v4f*>(&T[fr * kLnPitch + dcol + n * 16 + fq * 4]) = o;
+    }
+  }
+  if constexpr (kLn) {
+    __shared__ float s_stat[2][16];
+    const int rr = tid >> 5, sub = tid & 31, row = m0 + rr;
+    __syncthreads();
+    v4f x[3];
+#pragma unroll
+    for (int i = 0; i < 3; i++) x[i] = *reinterpret_cast<const v4f*>(&T[rr * kLnPitch + (sub + 32 * i) * 4]);
+    if (tid < 16) s_stat[0][tid] = lds_row_sum(&T[tid * kLnPitch], [](float v) { return v; }) / 384.0f;
+    __syncthreads();  // (and every read of the rows is done)
+    const float mean = s_stat[0][rr];
+#pragma unroll
+    for (int i = 0; i < 3; i++) {
+      const v4f d = x[i] - mean;
+      *reinterpret_cast<v4f*>(&T[rr * kLnPitch + (sub + 32 * i) * 4]) = d * d;
+    }
+    __syncthreads();
+    if (tid < 16)
+      s_stat[1][tid] = 1.0f / sqrtf(lds_row_sum(&T[tid * kLnPitch], [](float v) { return v; }) / 384.0f + 1e-12f);
+    __syncthreads();
+    const float rstd = s_stat[1][rr];
+    float amax = 0.0f;
+#pragma unroll
+    for (int i = 0; i < 3; i++) {
+      const v4f y = (x[i] - mean) * rstd * lg[i] + lb[i];
+      if (ln.dst && row < p.M) *reinterpret_cast<v4f*>(ln.dst + (size_t)row * kH + (sub + 32 * i) * 4) = y;
+      x[i] = y * lsm[i];
+#pragma unroll
+      for (int r = 0; r < 4; r++) amax = nanless_max(amax, fabsf(x[i][r]));
+    }
+    amax = lanes32_max(amax);  // amax is never NaN: fmaxf is nanless_max here
+    const float max_abs = nanless_max(1e-8f, amax), inv_scale = 127.0f / max_abs;
+    if (row < p.M) {
+#pragma unroll
+      for (int i = 0; i < 3; i++)
+        *reinterpret_cast<uint32_t*>(ln.q + (size_t)row * kH + (sub + 32 * i) * 4) =
+            pack4(qround(x[i][0] * inv_scale), qround(x[i][1] * inv_scale), qround(x[i][2] * inv_scale),
+                  qround(x[i][3] * inv_scale));
+      if (sub == 0) {
+        ln.scale[row] = max_abs / 127.0f;
+        if (ln.stats) ln.stats[row] = make_float2(mean, rstd);
+        if (ln.rowmax_init) ln.rowmax_init[row] = __float_as_uint(1e-8f);
+      }
     }
   }
 }
@@ -562,14 +630,14 @@ hipError_t ffn_repair_counts(unsigned long long counts[2], bool reset) {
   return e;
 }
 
-template <int NR, int kP>
-static void launch_ffn_rows(const FfnArgs& p, hipStream_t st) {
+template <int NR, int kP, bool kLn = false>
+static void launch_ffn_rows(const FfnArgs& p, hipStream_t st, const LnArgs& ln = LnArgs{}) {
   constexpr int R = 16 * NR * kP;
   const dim3 grid((unsigned)((p.M + R - 1) / R));
   if (p.fast_gelu && !g_ffn_exact_gelu)
-    hipLaunchKernelGGL((ffn_kernel<NR, kP, true>), grid, dim3(kThreads), 0, st, p);
+    hipLaunchKernelGGL((ffn_kernel<NR, kP, true, kLn>), grid, dim3(kThreads), 0, st, p, ln);
   else
-    hipLaunchKernelGGL((ffn_kernel<NR, kP, false>), grid, dim3(kThreads), 0, st, p);
+    hipLaunchKernelGGL((ffn_kernel<NR, kP, false, kLn>), grid, dim3(kThreads), 0, st, p, ln);
 }
 static void launch_ffn_tile(const FfnArgs& p, int rows, hipStream_t st) {
   if (rows == 16) launch_ffn_rows<1, 1>(p, st);
@@ -585,8 +653,12 @@ static void launch_ffn_tile(const FfnArgs& p, int rows, hipStream_t st) {
 // a second launch for the remaining rows, whose last, partial round then holds
 // short workgroups (68,270 rows: 233 us, against 245 in 64-row and 251 in 32-row
 // workgroups).
-void launch_ffn(const FfnArgs& p, hipStream_t st, hipStream_t side, hipEvent_t fork, hipEvent_t join) {
-  if (p.M <= 0) return;
+struct FfnPlan {
+  int tile;   // rows per workgroup, all rows (m64 = 0)
+  long m64;   // the mixed plan: rows in 64-row workgroups,
+  int tail;   // rows per workgroup of the others
+};
+static FfnPlan ffn_plan(const FfnArgs& p) {
   const long cus = device_cu_count();
   auto rounds = [&](long rows, long tile) { return ((rows + tile - 1) / tile + cus - 1) / cus; };
   constexpr long kT16 = 100, kT32 = 140, kT64 = 255, kFirst64 = 15, kLaunch = 10;
@@ -604,8 +676,23 @@ void launch_ffn(const FfnArgs& p, hipStream_t st, hipStream_t side, hipEvent_t f
     m64 = -g_ffn_rows < p.M ? -g_ffn_rows : 0;
     tile = 64, tail = 32;
   }
+  return {tile, m64, tail};
+}
+
+// in one round of 16-row workgroups, which all end on the LayerNorm's in-order sums together
+bool ffn_fuses_ln(const FfnArgs& p) {
+  const FfnPlan plan = ffn_plan(p);
+  return p.M > 0 && plan.m64 == 0 && plan.tile == 16;
+}
+
+void launch_ffn(const FfnArgs& p, hipStream_t st, hipStream_t side, hipEvent_t fork, hipEvent_t join, const LnArgs* ln) {
+  if (p.M <= 0) return;
+  const FfnPlan plan = ffn_plan(p);
+  const long m64 = plan.m64;
+  const int tail = plan.tail;
   if (m64 == 0) {
-    launch_ffn_tile(p, tile, st);
+    if (ln && plan.tile == 16) launch_ffn_rows<1, 1, true>(p, st, *ln);
+    else launch_ffn_tile(p, plan.tile, st);
     return;
   }
   FfnArgs a = p, b = p;

@@ -411,6 +411,27 @@ def test_layer_prefix_state_many_rows(engine, oracle_model, n, lo, hi, layers):
     assert np.array_equal(h, rh) and np.array_equal(q, rq) and np.array_equal(sc, rsc)
 
 
+@pytest.mark.parametrize("exact", [False, True], ids=["fast", "exact"])
+@pytest.mark.parametrize("total", [1025, 4096, 4097])
+def test_layer_prefix_state_ffn_with_layernorm(engine, oracle_model, total, exact):
+    """LN2 in the FFN's kernel (one round of 16-row workgroups, with a partial last one) and behind it
+    (beyond), the last layer storing its f32 rows and the first only their statistics: state after one
+    and two layers bit-exact against the oracle."""
+    rng = np.random.default_rng(total)
+    lens = [total // 9] * 8 + [total - 8 * (total // 9)]
+    seqs = [np.concatenate([[101], rng.integers(1000, 30522, n - 2), [102]]).astype(np.uint16) for n in lens]
+    w = engine.workspace(total, len(lens))
+    try:
+        ae.set_ffn_exact_gelu(exact)
+        for layers in (1, 2):
+            h, q, sc = engine.forward_prefix(w, seqs, layers)
+            rh, rq, rsc = oracle_model.run_prefix(seqs, layers)
+            assert np.array_equal(h, rh) and np.array_equal(q, rq) and np.array_equal(sc, rsc)
+    finally:
+        ae.set_ffn_exact_gelu(False)
+        w.close()
+
+
 def test_graph_replay_matches_eager(engine, oracle_model, torch_gpu):
     """Repeated forward passes replay a captured hipGraph: every replay, interleaved with
     eager passes of other shapes and host synchronizations, equals the eager result."""
