@@ -392,7 +392,7 @@ __global__ __launch_bounds__(256, 2) void gemm_astat_kernel(GemmArgs p) {
 // LN1 (reference src/model.rs:695-724: smooth_quantize_row of ctx,
 // gemm_int8_fused(attn_out, residual hidden), then layernorm_smooth_quantize_row,
 // src/simd_math.rs:208-247).
-// A workgroup of 4 waves owns 32 complete rows (wave w: columns 96w..96w+95),
+// A workgroup of 4 or 8 waves owns 32 complete rows (wave w: its 96 or 48 columns),
 // so the GEMM's output rows stay in LDS for the LayerNorm instead of going to
 // HBM and back.  The arithmetic is gemm_w8a8_kernel's kAF32QSmooth / kEpiF32
 // and ln_quant_kernel's, in the same order.  ln.dst may alias p.res: a
@@ -401,8 +401,10 @@ __global__ __launch_bounds__(256, 2) void gemm_astat_kernel(GemmArgs p) {
 constexpr int kLrRows = 32;
 constexpr int kLrPitch = 388;  // LDS floats per row of the output tile
 
-__global__ __launch_bounds__(256, 3) void gemm_ln_rows_kernel(GemmArgs p, LnArgs ln) {
-  constexpr int kCB = 6, kRing = 3, kSteps = 6, NB = 384 / 16;
+template <int kWaves>
+__global__ __launch_bounds__(64 * kWaves, kWaves == 4 ? 3 : 4) void gemm_ln_rows_kernel(GemmArgs p, LnArgs ln) {
+  constexpr int kCB = 24 / kWaves, kRing = 3, kSteps = 6, NB = 384 / 16;
+  constexpr int kLpr = 64 * kWaves / kLrRows, kF4 = 96 / kLpr;  // lanes and float4s per lane of a row
   static_assert(kLrRows * kAsPitch <= kLrRows * kLrPitch * 4, "the A tile lives in the row tile's space");
   // the int8 A tile during the K loop; then the int32 accumulators, the f32
   // output rows and their squared deviations (3 workgroups fit a CU's LDS)
@@ -419,9 +421,9 @@ __global__ __launch_bounds__(256, 3) void gemm_ln_rows_kernel(GemmArgs p, LnArgs
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int fr = lane & 15, fq = lane >> 4;
   const int m0 = blockIdx.x * kLrRows;
-  // row rl of the tile, float4 columns sub + 8 i (i < 12): the A quantization,
+  // row rl of the tile, float4 columns sub + kLpr i (i < kF4): the A quantization,
   // the epilogue and the LayerNorm all use this mapping
-  const int rl = tid >> 3, sub = tid & 7, row = m0 + rl;
+  const int rl = tid / kLpr, sub = tid % kLpr, row = m0 + rl;
   const bool valid = row < p.M;
   const int rrow = valid ? row : p.M - 1;
 
@@ -429,9 +431,9 @@ __global__ __launch_bounds__(256, 3) void gemm_ln_rows_kernel(GemmArgs p, LnArgs
   // its max, the first kRing K steps of W, w_scale and bias; the residual row
   // after the K loop
   const float* xr = reinterpret_cast<const float*>(p.A) + (size_t)rrow * 384;
-  float4 xa[12];
+  float4 xa[kF4];
 #pragma unroll
-  for (int i = 0; i < 12; i++) xa[i] = *reinterpret_cast<const float4*>(xr + (sub + 8 * i) * 4);
+  for (int i = 0; i < kF4; i++) xa[i] = *reinterpret_cast<const float4*>(xr + (sub + kLpr * i) * 4);
   const float amax_a = __uint_as_float(p.a_rowmax[rrow]);
   const int8_t* wbase = p.w + (size_t)lane * 16;
   v4i ring[kRing][kCB];
@@ -452,8 +454,8 @@ __global__ __launch_bounds__(256, 3) void gemm_ln_rows_kernel(GemmArgs p, LnArgs
   {  // A quantized as kAF32QSmooth: q = round((x * inv_smooth[j]) * (127 / max_abs))
     const float inv = 127.0f / amax_a;  // inv_scale = 127.0 / max_abs
 #pragma unroll
-    for (int i = 0; i < 12; i++) {
-      const int c = (sub + 8 * i) * 4;
+    for (int i = 0; i < kF4; i++) {
+      const int c = (sub + kLpr * i) * 4;
       const float4 sm = *reinterpret_cast<const float4*>(p.a_smooth + c);
       const float4 v = make_float4(xa[i].x * sm.x, xa[i].y * sm.y, xa[i].z * sm.z, xa[i].w * sm.w);
       *reinterpret_cast<uint32_t*>(&sA[rl * kAsPitch + c]) =
@@ -479,18 +481,18 @@ __global__ __launch_bounds__(256, 3) void gemm_ln_rows_kernel(GemmArgs p, LnArgs
         acc[i][j] = __builtin_amdgcn_mfma_i32_16x16x64_i8(af[i], ring[kt % kRing][j], acc[i][j], 0, 0, 0);
     if (kt + kRing < kSteps) wload(kt + kRing, ring[kt % kRing]);
   }
-  float4 res[12];
+  float4 res[kF4];
   const float* rr = p.res + (size_t)rrow * 384;
 #pragma unroll
-  for (int i = 0; i < 12; i++) {
-    const v4i r = __builtin_nontemporal_load(reinterpret_cast<const v4i*>(rr + (sub + 8 * i) * 4));
+  for (int i = 0; i < kF4; i++) {
+    const v4i r = __builtin_nontemporal_load(reinterpret_cast<const v4i*>(rr + (sub + kLpr * i) * 4));
     res[i] = make_float4(__int_as_float(r.x), __int_as_float(r.y), __int_as_float(r.z), __int_as_float(r.w));
   }
   if (p.res_stats) {  // the residual is the LayerNorm of these rows, recomputed as that LayerNorm forms it
     const float2 st = p.res_stats[rrow];
 #pragma unroll
-    for (int i = 0; i < 12; i++) {
-      const int c = (sub + 8 * i) * 4;
+    for (int i = 0; i < kF4; i++) {
+      const int c = (sub + kLpr * i) * 4;
       const float4 g = *reinterpret_cast<const float4*>(&sRg[c]);
       const float4 bt = *reinterpret_cast<const float4*>(&sRb[c]);
       res[i].x = (res[i].x - st.x) * st.y * g.x + bt.x;
@@ -500,22 +502,22 @@ __global__ __launch_bounds__(256, 3) void gemm_ln_rows_kernel(GemmArgs p, LnArgs
     }
   }
   __syncthreads();  // every wave's K loop is done with the A tile
-  // accumulators into the row tile (lane: rows 16 i + 4 fq + r of column 96 w + 16 j + fr)
+  // accumulators into the row tile (lane: rows 16 i + 4 fq + r of column 16 kCB w + 16 j + fr)
   int* T32 = reinterpret_cast<int*>(sT);
 #pragma unroll
   for (int i = 0; i < 2; i++)
 #pragma unroll
     for (int j = 0; j < kCB; j++)
 #pragma unroll
-      for (int r = 0; r < 4; r++) T32[(i * 16 + fq * 4 + r) * kLrPitch + wave * 96 + j * 16 + fr] = acc[i][j][r];
+      for (int r = 0; r < 4; r++) T32[(i * 16 + fq * 4 + r) * kLrPitch + wave * 16 * kCB + j * 16 + fr] = acc[i][j][r];
   __syncthreads();
 
   // epilogue: out = fma(f32(acc), sa * ws, bias + res), kept in registers and in the tile
   const float sa = amax_a / 127.0f;  // scale = max_abs / 127.0
-  float4 xv[12];
+  float4 xv[kF4];
 #pragma unroll
-  for (int i = 0; i < 12; i++) {
-    const int c = (sub + 8 * i) * 4;
+  for (int i = 0; i < kF4; i++) {
+    const int c = (sub + kLpr * i) * 4;
     const int4 a4 = *reinterpret_cast<const int4*>(&T32[rl * kLrPitch + c]);
     const float4 ws4 = *reinterpret_cast<const float4*>(&sWs[c]);
     float4 b4 = *reinterpret_cast<const float4*>(&sB[c]);
@@ -531,15 +533,15 @@ __global__ __launch_bounds__(256, 3) void gemm_ln_rows_kernel(GemmArgs p, LnArgs
   __syncthreads();
 
   // LayerNorm + SmoothQuant of the 32 rows (as ln_quant_kernel): one lane per
-  // row takes the in-order sums, 8 threads per row the rest
+  // row takes the in-order sums, kLpr threads per row the rest
   if (tid < kLrRows) s_mean[tid] = lds_row_sum(&sT[tid * kLrPitch], [](float v) { return v; }) / 384.0f;
   __syncthreads();
   const float mean = s_mean[rl];
 #pragma unroll
-  for (int i = 0; i < 12; i++) {
+  for (int i = 0; i < kF4; i++) {
     float4 d = xv[i];
     d.x = d.x - mean; d.y = d.y - mean; d.z = d.z - mean; d.w = d.w - mean;
-    *reinterpret_cast<float4*>(&sT[rl * kLrPitch + (sub + 8 * i) * 4]) = make_float4(d.x * d.x, d.y * d.y, d.z * d.z, d.w * d.w);
+    *reinterpret_cast<float4*>(&sT[rl * kLrPitch + (sub + kLpr * i) * 4]) = make_float4(d.x * d.x, d.y * d.y, d.z * d.z, d.w * d.w);
   }
   __syncthreads();
   if (tid < kLrRows) {
@@ -549,10 +551,10 @@ __global__ __launch_bounds__(256, 3) void gemm_ln_rows_kernel(GemmArgs p, LnArgs
   __syncthreads();
   const float rstd = s_rstd[rl];
   float amax = 0.0f;
-  float4 ys[12];
+  float4 ys[kF4];
 #pragma unroll
-  for (int i = 0; i < 12; i++) {
-    const int c = (sub + 8 * i) * 4;
+  for (int i = 0; i < kF4; i++) {
+    const int c = (sub + kLpr * i) * 4;
     const float4 g = *reinterpret_cast<const float4*>(ln.gamma + c);
     const float4 b = *reinterpret_cast<const float4*>(ln.beta + c);
     const float4 sm = *reinterpret_cast<const float4*>(ln.smooth + c);
@@ -568,13 +570,13 @@ __global__ __launch_bounds__(256, 3) void gemm_ln_rows_kernel(GemmArgs p, LnArgs
     amax = nanless_max(amax, fabsf(ys[i].z));
     amax = nanless_max(amax, fabsf(ys[i].w));
   }
-  amax = lanes8_max(amax);  // amax is never NaN: fmaxf is nanless_max here
+  amax = kLpr == 16 ? row16_max(amax) : lanes8_max(amax);  // amax is never NaN: fmaxf is nanless_max here
   const float max_abs = nanless_max(1e-8f, amax);
   const float inv_scale = 127.0f / max_abs;
   if (valid) {
 #pragma unroll
-    for (int i = 0; i < 12; i++) {
-      const int c = (sub + 8 * i) * 4;
+    for (int i = 0; i < kF4; i++) {
+      const int c = (sub + kLpr * i) * 4;
       *reinterpret_cast<uint32_t*>(ln.q + (size_t)row * 384 + c) =
           pack4(qround(ys[i].x * inv_scale), qround(ys[i].y * inv_scale), qround(ys[i].z * inv_scale),
                 qround(ys[i].w * inv_scale));
@@ -1127,9 +1129,9 @@ static bool int8_rows16(const GemmArgs& p) {
 // two in-order sums of 384), and gemm_ln_rows_kernel's 32-row workgroups of 4
 // waves take twice as long for theirs on half the compute units: in passes of
 // 1,280, 2,844 and 4,096 rows it took 7.5, 7.2 and 6.7 us more per layer (771 ->
-// 689, 1,111 -> 1,032, 1,701 -> 1,627 us per pass).  With more rows the second
-// workgroup per CU waits for registers: 5,200 rows 1,023 -> 1,029, 8,000 rows
-// 1,789 -> 1,781.
+// 689, 1,111 -> 1,032, 1,701 -> 1,627 us per pass).  With more rows a second
+// workgroup per CU waits for registers: 5,200 rows 1,029 us against 1,023 in
+// 32-row workgroups of 4 waves, which take 8 there now.
 static bool ln_rows16(const GemmArgs& p) { return small_gemm(p) || (p.M + 15) / 16 <= device_cu_count(); }
 
 // ln != null: N = 384, kEpiF32, K <= kSmallMaxK, ln_rows16(p); the epilogue
@@ -1226,7 +1228,16 @@ void launch_gemm_ln(const GemmArgs& p, int amode, const LnArgs& ln, hipStream_t 
     return;
   }
   if (!ln_rows16(p)) {  // many rows: kAF32QSmooth, N = K = 384, with residual
-    hipLaunchKernelGGL(gemm_ln_rows_kernel, dim3((p.M + kLrRows - 1) / kLrRows), dim3(256), 0, st, p, ln);
+    // 8 waves (114 VGPRs, two workgroups per CU) halve every phase but the in-order
+    // sums, 4 waves (165, three per CU) hide one another's latency in several
+    // rounds: 8 while they run in one round, 16,384 rows.  Passes with 4 / 8 waves:
+    // 4,500 rows 942 / 891 us, 8,190 rows 1,094 / 1,041, 16,380 rows 1,629 / 1,586,
+    // 24,000 rows 2,294 / 2,351, 33,000 rows 3,572 / 3,534, 66,000 rows 6,163 / 6,168.
+    const int wgs = (p.M + kLrRows - 1) / kLrRows;
+    if (wgs <= 2 * device_cu_count())
+      hipLaunchKernelGGL(gemm_ln_rows_kernel<8>, dim3(wgs), dim3(512), 0, st, p, ln);
+    else
+      hipLaunchKernelGGL(gemm_ln_rows_kernel<4>, dim3(wgs), dim3(256), 0, st, p, ln);
     return;
   }
   if (amode == kAI8) launch_variant<kAI8, kEpiF32>(p, st, &ln);

@@ -217,10 +217,11 @@ def test_gemm_then_layernorm_bit_exact(torch_gpu, m):
     assert np.array_equal(bits(sc_d.cpu().numpy()), bits(rsc))
 
 
-@pytest.mark.parametrize("m", [1025, 4095, 4096, 4097])
+@pytest.mark.parametrize("m", [1025, 4095, 4096, 4097, 16384, 16385])
 def test_gemm_then_layernorm_tile_heights(torch_gpu, m):
-    """The same on both sides of the rule for the tile height (16 rows while one workgroup per
-    compute unit covers them, 32 beyond), with partial last tiles, the output in the residual's place."""
+    """The same on both sides of the rules for the tile height (16 rows while one workgroup per
+    compute unit covers them, 32 beyond, with 8 waves up to two per compute unit, then with 4), with
+    partial last tiles, the output in the residual's place."""
     torch = torch_gpu
     n = k = 384
     w, ws, b, s = linear_inputs(n, k, 12)
