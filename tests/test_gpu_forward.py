@@ -397,8 +397,8 @@ def test_layer_prefix_state_few_row_column_splits(engine, oracle_model, total):
 @pytest.mark.parametrize("n,lo,hi,layers", [(8, 300, 512, 1), (10, 400, 512, 2)], ids=["T~3k", "T~4.6k"])
 def test_layer_prefix_state_many_rows(engine, oracle_model, n, lo, hi, layers):
     """The many-row kernels (past the few-row path's 1,024 rows): the attention output GEMM fused
-    with LN1, the A-stationary or column-tiled QKV, the two-kernel FFN below 4,096 rows and the
-    fused FFN block above; state after `layers` layers bit-exact against the oracle."""
+    with LN1, the A-stationary or tiled QKV, the FFN block with LN2 in its kernel up to 4,096 rows
+    and behind it above; state after `layers` layers bit-exact against the oracle."""
     seqs = ragged_batch(n, lo, hi, 23 + n)
     T = sum(len(s) for s in seqs)
     assert T > 1024

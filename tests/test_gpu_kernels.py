@@ -179,8 +179,8 @@ def test_gemm_quantize_on_load_bit_exact(torch_gpu, smooth, n, k):
 
 @pytest.mark.parametrize("m", [37, 1500, 2000])
 def test_gemm_then_layernorm_bit_exact(torch_gpu, m):
-    """The attention output GEMM and LN1 in one kernel (the few-row form at 37 rows, the 32-row
-    many-row form at 1,500 and 2,000 with a partial last tile): f32 LN rows, int8 rows and scales
+    """The attention output GEMM and LN1 in one kernel (16-row workgroups, at 1,500 rows with a
+    partial last tile): f32 LN rows, int8 rows and scales
     bit for bit against the oracle's smooth_quantize -> gemm_scalar_fused(residual) ->
     layernorm_smooth_quantize.  Rows include a zero ctx row, a residual row whose mean and variance
     depend on the summation order (+-1e8 against small values) and a constant output row."""
