@@ -331,6 +331,10 @@ int ae_debug_mfma_products(const float* a_dev, const float* b_dev, float* out_de
  * tiled and register-row kernels only, 2 the latency form only.  Every form
  * gives the same bits.  AE_ERR_INVALID_ARG for another value. */
 int ae_debug_set_attention_form(int form);
+/* Whether ae_gemm_w8a8 of m > 1024 rows, with or without a residual, takes the
+ * 16-row workgroups on a GPU of `cus` compute units (a test hook, no reference
+ * counterpart, no device access): 1 or 0.  Either form gives the same bits. */
+int ae_debug_gemm_int8_rows16(int m, int n, int k, int residual, int cus);
 /* Token rows per workgroup of the fused FFN kernel, process-wide (a test hook,
  * no reference counterpart): 0 by the batch's size (the default), 32 or 64, or
  * -m (m a multiple of 64): the first m rows in 64-row workgroups and the rest

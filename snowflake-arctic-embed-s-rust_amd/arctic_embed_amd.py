@@ -78,6 +78,7 @@ _SIGS = {
     "ae_debug_gelu_map": (_i32, [_vp, _vp, _sz, _vp]),
     "ae_debug_mfma_products": (_i32, [_vp, _vp, _vp, ctypes.c_int, _vp]),
     "ae_debug_set_attention_form": (_i32, [ctypes.c_int]),
+    "ae_debug_gemm_int8_rows16": (_i32, [ctypes.c_int] * 5),
     "ae_debug_set_ffn_rows": (_i32, [ctypes.c_int]),
     "ae_debug_set_ffn_exact_gelu": (_i32, [ctypes.c_int]),
     "ae_debug_gelu_fast_certify": (_i32, [ctypes.POINTER(ctypes.c_uint64)]),
@@ -487,6 +488,12 @@ def set_attention_form(form):
     """Exact-attention kernels to launch from now on: 0 by the batch (default),
     1 tiled / register rows only, 2 the latency form only (a test hook)."""
     _check(_lib.ae_debug_set_attention_form(int(form)))
+
+
+def gemm_int8_rows16(m, n, k, residual, cus=256):
+    """Whether Linear.gemm of m > 1024 rows takes its 16-row workgroups on a GPU of cus compute
+    units (a test hook, no device access)."""
+    return bool(_lib.ae_debug_gemm_int8_rows16(int(m), int(n), int(k), 1 if residual else 0, int(cus)))
 
 
 def set_ffn_rows(rows):

@@ -1592,6 +1592,11 @@ int ae_debug_set_attention_form(int form) {
   return AE_OK;
 }
 
+// test hook: the rule that keeps the 16-row workgroups of the int8 GEMM (no device access)
+int ae_debug_gemm_int8_rows16(int m, int n, int k, int residual, int cus) {
+  return aek::gemm_int8_rows16(m, n, k, residual != 0, cus) ? 1 : 0;
+}
+
 // test hook: the FFN kernel's workgroup height
 int ae_debug_set_ffn_rows(int rows) {
   if (rows != 0 && rows != 32 && rows != 64 && !(rows < 0 && rows % 64 == 0))

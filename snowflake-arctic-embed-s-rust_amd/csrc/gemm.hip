@@ -1114,13 +1114,23 @@ constexpr int kSplitMinK = 1024;
 // gemm_w8a8_kernel's K loop is a chain of 6 or 24 steps of 64 behind a barrier
 // each on a few 64 x 192 tiles.  K = 384: one round of them, three per compute
 // unit (N = 1152: 1,280 rows 6.6 -> 5.2 us, 2,048 rows 7.1 -> 6.4, but 2,843 rows
-// 8.2 -> 8.9; N = 1536: 1,536 rows 7.0 -> 6.4, 2,048 rows 7.5 -> 8.1).  K = 1536:
-// four rounds (N = 384: 1,280 rows 17.9 -> 6.8 us, 2,843 rows 18.0 -> 11.8, 5,500
-// rows 21.4 -> 18.6, but 8,192 rows 22.3 -> 26.0).
-static bool int8_rows16(const GemmArgs& p) {
-  const long mt = (p.M + 15) / 16, cus = device_cu_count();
-  if (p.K == 384) return mt * (p.N / 192) <= 3 * cus;
-  return p.K >= kSplitMinK && p.K <= kSmallMaxK && p.K % 512 == 0 && mt * (p.N / 48) <= 4 * 3 * cus;
+// 8.2 -> 8.9; N = 1536: 1,536 rows 7.0 -> 6.4, 2,048 rows 7.5 -> 8.1).  K of 1,024
+// and 1,536 (us per call, 64 x 192 tiles / 16-row workgroups; a round is three
+// workgroups per compute unit):
+//  * no residual: two rounds (N = 384, K = 1536: 3,072 rows 13.6 / 11.0, 4,096 rows
+//    14.0 / 13.7, 6,144 rows 14.6 / 18.4; K = 1024: 3,072 rows 10.5 / 9.1, 4,096 rows
+//    10.7 / 11.3; N = 1536, K = 1024: 1,040 rows 11.1 / 12.1, 1,536 rows 11.5 / 16.3);
+//  * a residual, which costs the 64 x 192 tiles 1.5 to 6 us (by where the buffers
+//    lie): four rounds at K = 1536 up to N = 768 (N = 384: 1,280 rows 17.7 / 6.8,
+//    6,144 rows 20.8 / 18.9, 8,192 rows 22.3 / 26.0; N = 768: 3,072 rows 21.9 / 20.1),
+//    else less than three (K = 1024: N = 384, 4,096 rows 13.6 / 11.6, 6,144 rows 14.9
+//    to 17.6 / 15.6 to 16.9; N = 1152, 1,280 rows 15.1 / 11.6, 1,536 rows 12.9 / 13.1).
+bool gemm_int8_rows16(int m, int n, int k, bool res, int cus) {
+  const long mt = (m + 15) / 16;
+  if (k == 384) return mt * (n / 192) <= 3L * cus;
+  if (k < kSplitMinK || k > kSmallMaxK || k % 512 != 0) return false;
+  const long wgs = mt * (n / 48);
+  return !res ? wgs <= 6L * cus : k == 1536 && n <= 768 ? wgs <= 12L * cus : wgs < 9L * cus;
 }
 
 // The attention output GEMM with LN1 (kAF32QSmooth, N = K = 384) takes
@@ -1143,7 +1153,8 @@ static void launch_variant(GemmArgs p, hipStream_t st, const LnArgs* ln = nullpt
     hipLaunchKernelGGL((gemm_small_kernel<AM, kEpiF32, true, 1>), dim3(mt16), dim3(512), 0, st, p, *ln, PreArgs{});
     return;
   }
-  if (small_gemm(p) || (AM == kAI8 && EM == kEpiF32 && int8_rows16(p))) {
+  if (small_gemm(p) ||
+      (AM == kAI8 && EM == kEpiF32 && gemm_int8_rows16(p.M, p.N, p.K, p.res != nullptr, device_cu_count()))) {
     if (EM == kEpiF32 && p.K >= kSplitMinK && p.K % 512 == 0) {
       if (AM != kAI8 && mt16 * (p.N / 48) < 256)  // 8-row tiles: half the f32 A per workgroup, twice the workgroups
         hipLaunchKernelGGL((gemm_small_kernel<AM, kEpiF32, false, 8, 8>), dim3(((p.M + 7) / 8) * (p.N / 48)),

@@ -167,6 +167,9 @@ struct PreArgs {
 void launch_gemm_pre_ln(const GemmArgs& p, const PreArgs& pre, const LnArgs& ln, hipStream_t st);
 // whether launch_gemm takes the few-rows kernels for m rows (and the prologue form applies)
 bool gemm_small_path(int m);
+// whether an int8-A GEMM (kEpiF32, m rows beyond the few-rows path, K = k) keeps the
+// 16-row workgroups on a GPU of cus compute units
+bool gemm_int8_rows16(int m, int n, int k, bool res, int cus);
 
 void launch_row_quant(int m, int n, float* x, const float* smooth, int8_t* q, float* scale, bool gelu,
                       hipStream_t st);

@@ -51,6 +51,24 @@ def test_noalloc_attention_refuses_before_any_device_work():
     assert call(3, 2, 64) == ae.AE_ERR_INVALID_ARG  # fewer tokens than segments
 
 
+@pytest.mark.parametrize("m,n,k,residual,rows16", [
+    # K = 1024 and 1536 without a residual: two rounds of workgroups (slower beyond: 1.06 to 1.42 times)
+    (3072, 384, 1536, False, True), (4096, 384, 1024, False, False), (6144, 384, 1536, False, False),
+    (2048, 768, 1024, False, False), (1536, 1152, 1024, False, False), (1040, 1536, 1024, False, False),
+    # with one: four rounds at K = 1536 up to N = 768, else less than three
+    (6144, 384, 1536, True, True), (6145, 384, 1536, True, False), (3072, 768, 1536, True, True),
+    (4096, 384, 1024, True, True), (5120, 384, 1024, True, False), (2048, 768, 1024, True, True),
+    (1280, 1152, 1024, True, True), (1536, 1152, 1024, True, False), (1536, 1536, 1536, True, False),
+    # K = 384: one round, with or without
+    (6144, 384, 384, False, True), (2048, 1152, 384, True, True), (2049, 1152, 384, True, False),
+    # no K split
+    (1025, 384, 768, False, False)])
+def test_gemm_tile_height_rule(m, n, k, residual, rows16):
+    """Which int8 GEMMs beyond 1,024 rows keep the 16-row workgroups (256 compute units): those for
+    which these measured faster than the 64 x 192 tiles."""
+    assert ae.gemm_int8_rows16(m, n, k, residual) == rows16
+
+
 def test_version_and_default_dir(monkeypatch):
     assert "gfx950" in ae.version()
     monkeypatch.setenv("ARCTIC_EMBED_MODEL_DIR", "/some/dir")
