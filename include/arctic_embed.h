@@ -331,6 +331,12 @@ int ae_debug_mfma_products(const float* a_dev, const float* b_dev, float* out_de
  * tiled and register-row kernels only, 2 the latency form only.  Every form
  * gives the same bits.  AE_ERR_INVALID_ARG for another value. */
 int ae_debug_set_attention_form(int form);
+/* The kernels of the exact attention for a batch of n_seqs segments, total_tokens
+ * tokens and rows of at most max_seq_len on a GPU of `cus` compute units (a test
+ * hook, no reference counterpart, no device access): 0 tiles of 32 queries (rows
+ * in registers up to 64 keys), 1 tiles of 16 queries, 2 the kernel of batches so
+ * small that each of its workgroups has a compute unit to itself. */
+int ae_debug_attention_choice(int n_seqs, int total_tokens, int max_seq_len, int cus);
 /* Whether ae_gemm_w8a8 of m > 1024 rows, with or without a residual, takes the
  * 16-row workgroups on a GPU of `cus` compute units (a test hook, no reference
  * counterpart, no device access): 1 or 0.  Either form gives the same bits. */

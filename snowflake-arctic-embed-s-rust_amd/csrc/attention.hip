@@ -689,33 +689,35 @@ __global__ __launch_bounds__(64 * kWaves) void attention_kernel(AttnArgs p, int 
 }
 
 // ---------------------------------------------------------------------------
-// One sequence of at most kLatL tokens (the latency entry points): one workgroup
-// of 8 waves per (8 queries, head), with the arithmetic of attention_kernel<true>
-// in the same order, laid out for a short critical path rather than for
-// throughput (128 keys 6.6 us, attention_kernel's 16-query tiles 7.4; two rows
-// of 128: 11 / 7.6):
+// A few tokens (single sequences above all): one workgroup of 8 waves per
+// (sequence, 8 queries, head), with the arithmetic of attention_kernel<true> in
+// the same order, laid out for a short critical path rather than for throughput,
+// and taken while its workgroups fit the compute units one to one
+// (attention_choice).  kB = 1 or 2: sequences of at most 128 kB tokens.
 //  * every global load (the Q operands, the K operands of the wave's key
-//    block, the head's V rows into LDS) is issued at the start;
-//  * scores: wave w takes the 16-key block w: MFMA products and in-order adds
-//    exactly as attention_kernel<true>'s phase 1;
+//    blocks, the head's V rows into LDS) is issued at the start;
+//  * scores: wave w takes the 16-key blocks w and w + 8: MFMA products and
+//    in-order adds exactly as attention_kernel<true>'s phase 1;
 //  * exp and the in-order denominator as there;
 //  * p_t = e_t * inv in place (the reference's `s[i] * inv`), then PV on the
 //    VALU, one output (query, dim) per thread: p_t * v_t,d rounded, added in
 //    key order from LDS.
 // ---------------------------------------------------------------------------
-constexpr int kLatL = 128;  // keys: one 16-key block per wave
 constexpr int kLatQ = 8;  // queries per workgroup (MFMA rows 8-15 repeat a query and are not used)
 
-__global__ __launch_bounds__(512) void attention_lat_kernel(AttnArgs p) {
+template <int kB>
+__global__ __launch_bounds__(512) void attention_lat_kernel(AttnArgs p, int tiles_per_seq) {
+  constexpr int kLatL = 128 * kB;  // keys: kB 16-key blocks per wave
   __shared__ float s_maxw[8][kLatQ];
   __shared__ float s_max[kLatQ], s_inv[kLatQ];
   __shared__ uint64_t s_tab[32];
   constexpr int pitch = kLatL + 4;
   __shared__ __attribute__((aligned(16))) float S[kLatQ * pitch];  // scores -> exps -> probabilities
   __shared__ __attribute__((aligned(16))) float sV[kLatL * 32];
-  const int h = blockIdx.x % 12, q0 = blockIdx.x / 12 * kLatQ;
+  const int h = blockIdx.x % 12, bt = blockIdx.x / 12, b = bt / tiles_per_seq;
+  const int q0 = (bt - b * tiles_per_seq) * kLatQ;
   // bounds that the host knows (p.len1 > 0): no cu_seqlens load
-  const int s0 = p.len1 > 0 ? 0 : p.cu[0], L = min(p.len1 > 0 ? p.len1 : p.cu[1] - s0, min(p.s_pitch - 4, kLatL));
+  const int s0 = p.len1 > 0 ? 0 : p.cu[b], L = min(p.len1 > 0 ? p.len1 : p.cu[b + 1] - s0, min(p.s_pitch - 4, kLatL));
   if (q0 >= L) return;  // workgroup-uniform
   const int nq = min(kLatQ, L - q0);
   const int tid = threadIdx.x, lane = tid & 63;
@@ -753,8 +755,9 @@ __global__ __launch_bounds__(512) void attention_lat_kernel(AttnArgs p) {
   }
   float qf[8];  // query q0 + lr (rows past the segment, and lr >= kLatQ, clamped)
   load_dims(qkv + (size_t)min(q0 + min(lr, kLatQ - 1), L - 1) * HQKV, qf);
-  float kf[8];
-  load_dims(qkv + H + (size_t)min(16 * wave + lr, L - 1) * HQKV, kf);
+  float kf[kB][8];
+#pragma unroll
+  for (int j = 0; j < kB; j++) load_dims(qkv + H + (size_t)min(16 * (wave + 8 * j) + lr, L - 1) * HQKV, kf[j]);
   __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
   for (int i = 0; i < kVF; i++)  // lanes past the segment rewrite its last float4
@@ -763,29 +766,33 @@ __global__ __launch_bounds__(512) void attention_lat_kernel(AttnArgs p) {
   // scores of query lr for keys 16kb + 4lg + i (dot32_f32 order) and the row max;
   // keys >= L repeat key L - 1 (clamped rows) and cannot change the max
   float m = -INFINITY;
-  if (16 * wave < L) {  // wave-uniform
-    float acc[4];
 #pragma unroll
-    for (int c = 0; c < 2; c++) {
-      v16f pr[4];
+  for (int j = 0; j < kB; j++) {
+    const int kb = wave + 8 * j;
+    if (16 * kb < L) {  // wave-uniform
+      float acc[4];
 #pragma unroll
-      for (int u = 0; u < 4; u++) pr[u] = mfma_products(kf[4 * c + u], qf[4 * c + u]);
+      for (int c = 0; c < 2; c++) {
+        v16f pr[4];
 #pragma unroll
-      for (int blk = 0; blk < 4; blk++)  // dims 16c + 4blk + u, in order
+        for (int u = 0; u < 4; u++) pr[u] = mfma_products(kf[j][4 * c + u], qf[4 * c + u]);
 #pragma unroll
-        for (int u = 0; u < 4; u++)
+        for (int blk = 0; blk < 4; blk++)  // dims 16c + 4blk + u, in order
 #pragma unroll
-          for (int i = 0; i < 4; i++)
-            acc[i] = (c == 0 && blk == 0 && u == 0) ? pr[0][i] : acc[i] + pr[u][4 * blk + i];
-    }
-    float4 sc;
-    sc.x = acc[0] * kInvSqrtD;
-    sc.y = acc[1] * kInvSqrtD;
-    sc.z = acc[2] * kInvSqrtD;
-    sc.w = acc[3] * kInvSqrtD;
-    if (lr < kLatQ) {
-      *reinterpret_cast<float4*>(&S[lr * pitch + 16 * wave + 4 * lg]) = sc;
-      m = fmaxf(fmaxf(m, fmaxf(sc.x, sc.y)), fmaxf(sc.z, sc.w));
+          for (int u = 0; u < 4; u++)
+#pragma unroll
+            for (int i = 0; i < 4; i++)
+              acc[i] = (c == 0 && blk == 0 && u == 0) ? pr[0][i] : acc[i] + pr[u][4 * blk + i];
+      }
+      float4 sc;
+      sc.x = acc[0] * kInvSqrtD;
+      sc.y = acc[1] * kInvSqrtD;
+      sc.z = acc[2] * kInvSqrtD;
+      sc.w = acc[3] * kInvSqrtD;
+      if (lr < kLatQ) {
+        *reinterpret_cast<float4*>(&S[lr * pitch + 16 * kb + 4 * lg]) = sc;
+        m = fmaxf(fmaxf(m, fmaxf(sc.x, sc.y)), fmaxf(sc.z, sc.w));
+      }
     }
   }
   m = fmaxf(m, __shfl_xor(m, 16, 64));
@@ -805,7 +812,8 @@ __global__ __launch_bounds__(512) void attention_lat_kernel(AttnArgs p) {
     const int cols4 = (L + 3) >> 2;
     const float rcols = 1.0f / (float)cols4;  // q = floor((u + 0.5) / cols4): exact for u < 2^13
     const int units = nq * cols4;
-    if (64 * wave < units) {  // wave-uniform (expf_libm needs all lanes); one float4 per lane
+    static_assert(kLatQ * kLatL / 4 <= 512, "one float4 per thread");
+    if (64 * wave < units) {  // wave-uniform (expf_libm needs all lanes)
       const int u = min(tid, units - 1);
       const int q = (int)(((float)u + 0.5f) * rcols);
       float* e = &S[q * pitch + 4 * (u - q * cols4)];
@@ -1185,15 +1193,35 @@ static int g_attention_form = 0;  // 0 by the batch, 1 tiled (32 queries) / regi
 void set_attention_form(int form) { g_attention_form = form; }
 int attention_form() { return g_attention_form; }
 
+// attention_lat_kernel's workgroups run one to a compute unit: a batch of at most
+// this many 32-query tiles (the longest row's for every row, which bounds the
+// surplus workgroups) takes it while those with a query, at most 12 per (T + 7 B)
+// / 8, fit in one round.  Kernel times in us against attention_kernel's 16-query
+// tiles: one row of 128 keys 6.6 / 7.4, two of 128 (two rounds) 11 / 7.6.  Passes:
+// one row of 129 427 / 444, 168: 445 / 461; 2 x 66: 414 / 431; 140 + 16: 432 / 448;
+// 80 + 3 x 20: 414 / 429.
+constexpr int kLatMaxTiles = 16;
+
+int attention_choice(int B, int T, int max_len, int cus) {
+  if (max_len <= 64) return kAttnTiles32;
+  if (B * (long)((max_len + 31) / 32) <= kLatMaxTiles && 12 * ((T + 7 * B) / 8) <= cus && T <= 256) return kAttnLat;
+  const bool mixed = 2 * (size_t)max_len * B > 3 * (size_t)T;  // the longest row over 1.5 times the mean
+  return T <= (mixed ? kHalfMaxMixedT : kHalfMaxT) ? kAttnTiles16 : kAttnTiles32;
+}
+
 void launch_attention(const AttnArgs& p, int T, hipStream_t st, bool plan) {
   if (T <= 0 || p.B <= 0) return;
   const int max_len = p.s_pitch - 4;  // round16 of the longest sequence
-  const bool mixed = 2 * (size_t)max_len * p.B > 3 * (size_t)T;  // the longest row over 1.5 times the mean
-  const bool half = g_attention_form == 2 || (g_attention_form == 0 && max_len > 64 && T <= (mixed ? kHalfMaxMixedT : kHalfMaxT));
+  const int choice = attention_choice(p.B, T, max_len, device_cu_count());
+  const bool lat = g_attention_form != 1 && choice == kAttnLat;
+  const bool half = g_attention_form == 2 || (g_attention_form == 0 && choice == kAttnTiles16);
   const int max_tiles = attention_max_tiles(p.B, T);
   const int records = (int)attention_plan_list_records(p.B, T);
-  if (g_attention_form != 1 && p.B == 1 && max_len > 64 && max_len <= kLatL) {
-    hipLaunchKernelGGL(attention_lat_kernel, dim3(12 * ((max_len + kLatQ - 1) / kLatQ)), dim3(512), 0, st, p);
+  if (lat) {
+    const int tps = (min(max_len, T) + kLatQ - 1) / kLatQ;  // (no segment exceeds the batch's tokens)
+    const dim3 grid(p.B * tps * 12);
+    if (min(max_len, T) <= 128) hipLaunchKernelGGL(attention_lat_kernel<1>, grid, dim3(512), 0, st, p, tps);
+    else hipLaunchKernelGGL(attention_lat_kernel<2>, grid, dim3(512), 0, st, p, tps);
     return;
   }
   if (half) {

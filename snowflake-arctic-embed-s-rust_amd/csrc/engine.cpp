@@ -1592,6 +1592,11 @@ int ae_debug_set_attention_form(int form) {
   return AE_OK;
 }
 
+// test hook: the exact attention's kernels by the batch (no device access)
+int ae_debug_attention_choice(int n_seqs, int total_tokens, int max_seq_len, int cus) {
+  return aek::attention_choice(n_seqs, total_tokens, aek::attention_pitch(max_seq_len) - 4, cus);
+}
+
 // test hook: the rule that keeps the 16-row workgroups of the int8 GEMM (no device access)
 int ae_debug_gemm_int8_rows16(int m, int n, int k, int residual, int cus) {
   return aek::gemm_int8_rows16(m, n, k, residual != 0, cus) ? 1 : 0;

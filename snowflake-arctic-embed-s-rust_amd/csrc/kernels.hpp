@@ -212,6 +212,11 @@ hipError_t noalloc_plan_scratch(int** plan);
 // T = total tokens of the batch; plan = false reuses the plan already in p.plan
 // (launch_attention_plan, which depends only on cu, B and s_pitch)
 void launch_attention(const AttnArgs& p, int T, hipStream_t st, bool plan = true);
+// the exact attention's kernels for B segments, T tokens and rows of at most max_len
+// keys on a GPU of cus compute units: 32-query tiles (register rows up to 64 keys),
+// 16-query tiles, or attention_lat_kernel.  Every choice gives the same bits.
+enum AttnChoice { kAttnTiles32 = 0, kAttnTiles16 = 1, kAttnLat = 2 };
+int attention_choice(int B, int T, int max_len, int cus);
 // split = 1: rows of more than 384 keys in the plan's second list
 void launch_attention_plan(const AttnArgs& p, hipStream_t st, int split, int max_tiles);
 // exact-attention kernel choice for later launches: 0 by the batch, 1 tiled (32 queries) /

@@ -51,6 +51,17 @@ def test_noalloc_attention_refuses_before_any_device_work():
     assert call(3, 2, 64) == ae.AE_ERR_INVALID_ARG  # fewer tokens than segments
 
 
+@pytest.mark.parametrize("lens,choice", [
+    # a workgroup per compute unit: single sequences up to 168 tokens, a few short ones
+    ([65], 2), ([128], 2), ([129], 2), ([160], 2), ([168], 2), ([169], 1), ([509], 1),
+    ([66, 66], 2), ([80, 80], 2), ([140, 16], 2), ([80, 20, 20, 20], 2), ([112, 20, 20], 2),
+    ([128, 128], 1), ([88, 90], 1), ([100, 60, 20], 1), ([70] + [8] * 9, 1),
+    ([64], 0), ([128] * 12, 0)])
+def test_attention_choice(lens, choice):
+    """Which kernels the exact attention takes by the batch (256 compute units)."""
+    assert ae.attention_choice(len(lens), sum(lens), max(lens)) == choice
+
+
 @pytest.mark.parametrize("m,n,k,residual,rows16", [
     # K = 1024 and 1536 without a residual: two rounds of workgroups (slower beyond: 1.06 to 1.42 times)
     (3072, 384, 1536, False, True), (4096, 384, 1024, False, False), (6144, 384, 1536, False, False),

@@ -614,9 +614,13 @@ def test_attention_bit_exact(torch_gpu, attention_form, lens):
 
 # the latency form's choices: up to 16 segments its workgroups find their items (up to
 # 42 tiles of 16 queries with eight waves, up to 80 all resident at once, else longest
-# first), from 17 on the plan's, one row of up to 128 has a kernel of its own; by the batch up to 1,024 tokens, or 9,000 where the longest row is over
-# 1.5 times the mean.  Each set takes the latency form and the 32-query tiles.
-LATENCY_LENS = {"one_65": [65], "one_129": [129], "one_497": [497],
+# first), from 17 on the plan's; one row of up to 168 tokens, or a few short ones of
+# about as many in all, have a kernel of their own (up to 128 and up to 256 keys); by the
+# batch up to 1,024 tokens, or 9,000 where the longest row is over 1.5 times the mean.
+# Each set takes the latency form and the 32-query tiles.
+LATENCY_LENS = {"one_65": [65], "one_128": [128], "one_129": [129], "one_161": [161], "one_168": [168],
+                "one_169": [169], "one_497": [497], "few_66_66": [66, 66], "few_140_16": [140, 16],
+                "few_80_20_20_20": [80, 20, 20, 20], "few_129_1_30": [129, 1, 30], "few_88_90": [88, 90],
                 "two": [81, 17], "tiles_42": [336, 335], "tiles_44": [337, 340],
                 "resident_80_tiles": [256, 241, 255, 250, 242],
                 "longest_first": [16, 257, 1, 512, 512, 15, 31, 33, 48, 512, 49, 500, 2, 64, 65],
