@@ -120,7 +120,8 @@ int ae_embed_batch_tokens(const ae_engine* e, ae_workspace* ws, const uint16_t* 
 /* PackedModel::forward_ragged_cls (src/model.rs:521-914) with device-resident
  * inputs: ids_dev[total_tokens] u16, cu_seqlens_dev[n_seqs+1] i32 (each sequence
  * 1..max_seq_len tokens; max_seq_len <= 512, 0 means 512), out_dev[n_seqs*384]
- * f32.  Asynchronous on `stream`; no host copies.  Used when the caller keeps
+ * f32.  A max_seq_len below 512 is taken for the batch's longest length where the
+ * attention kernels are chosen (the same bits by any).  Asynchronous on `stream`; no host copies.  Used when the caller keeps
  * token ids in HBM.  The device checks cu_seqlens (cu[0] = 0, cu[n_seqs] =
  * total_tokens, every segment 1..max_seq_len tokens); a batch that fails is
  * reported as AE_ERR_INVALID_ARG by the next ae_workspace_synchronize.  Its
@@ -332,11 +333,12 @@ int ae_debug_mfma_products(const float* a_dev, const float* b_dev, float* out_de
  * gives the same bits.  AE_ERR_INVALID_ARG for another value. */
 int ae_debug_set_attention_form(int form);
 /* The kernels of the exact attention for a batch of n_seqs segments, total_tokens
- * tokens and rows of at most max_seq_len on a GPU of `cus` compute units (a test
- * hook, no reference counterpart, no device access): 0 tiles of 32 queries (rows
+ * tokens and rows of at most max_seq_len, the longest of them of `longest` tokens
+ * (0: not known), on a GPU of `cus` compute units (a test hook, no reference
+ * counterpart, no device access): 0 tiles of 32 queries (rows
  * in registers up to 64 keys), 1 tiles of 16 queries, 2 the kernel of batches so
  * small that each of its workgroups has a compute unit to itself. */
-int ae_debug_attention_choice(int n_seqs, int total_tokens, int max_seq_len, int cus);
+int ae_debug_attention_choice(int n_seqs, int total_tokens, int max_seq_len, int longest, int cus);
 /* Whether ae_gemm_w8a8 of m > 1024 rows, with or without a residual, takes the
  * 16-row workgroups on a GPU of `cus` compute units (a test hook, no reference
  * counterpart, no device access): 1 or 0.  Either form gives the same bits. */

@@ -78,7 +78,7 @@ _SIGS = {
     "ae_debug_gelu_map": (_i32, [_vp, _vp, _sz, _vp]),
     "ae_debug_mfma_products": (_i32, [_vp, _vp, _vp, ctypes.c_int, _vp]),
     "ae_debug_set_attention_form": (_i32, [ctypes.c_int]),
-    "ae_debug_attention_choice": (_i32, [ctypes.c_int] * 4),
+    "ae_debug_attention_choice": (_i32, [ctypes.c_int] * 5),
     "ae_debug_gemm_int8_rows16": (_i32, [ctypes.c_int] * 5),
     "ae_debug_set_ffn_rows": (_i32, [ctypes.c_int]),
     "ae_debug_set_ffn_exact_gelu": (_i32, [ctypes.c_int]),
@@ -491,10 +491,11 @@ def set_attention_form(form):
     _check(_lib.ae_debug_set_attention_form(int(form)))
 
 
-def attention_choice(n_seqs, total_tokens, max_seq_len, cus=256):
-    """The exact attention's kernels for a batch: 0 tiles of 32 queries, 1 of 16, 2 the smallest
-    batches' kernel (a test hook, no device access)."""
-    return _lib.ae_debug_attention_choice(int(n_seqs), int(total_tokens), int(max_seq_len), int(cus))
+def attention_choice(n_seqs, total_tokens, max_seq_len, longest=0, cus=256):
+    """The exact attention's kernels for a batch (longest: its longest row, 0 if only the bound
+    max_seq_len is known): 0 tiles of 32 queries, 1 of 16, 2 the smallest batches' kernel (a test
+    hook, no device access)."""
+    return _lib.ae_debug_attention_choice(int(n_seqs), int(total_tokens), int(max_seq_len), int(longest), int(cus))
 
 
 def gemm_int8_rows16(m, n, k, residual, cus=256):

@@ -1173,16 +1173,31 @@ void launch_attention_plan(const AttnArgs& p, hipStream_t st, int split, int max
 }
 
 // Batches whose 32-query tiles leave CUs idle or end on a long critical path take
-// the latency form's 16-query tiles.  Kernel times in us, 16-query against
-// 32-query tiles (against the two launches by length where those apply; these
-// need the plan kernel's 12 to 19 us first, once per pass): one row of 256
-// keys 11.0 / 14.2, 512: 22.6 / 24.8; 2 x 512: 29.3 / 31.1, 8 x 128: 12.0 / 12.2,
-// 12 x 128: 16.4 / 14.9, 3 x 384: 26.9 / 25.9, 16 x 96: 14.7 / 12.7, so up to kHalfMaxT
-// tokens.  Batches of mixed lengths (16 to 512 keys), whose long rows are the
-// critical path: 1,782 tokens 31.5 / 45.7, 2,843: 44 / 60.6, 5,470: 84 / 91,
-// 9,420: 146 / 146, 13,773: 217 / 210; 128 rows of 64 with one of 512 (8,704) 50 /
-// 54, so up to kHalfMaxMixedT tokens.
-constexpr int kHalfMaxT = 1024, kHalfMaxMixedT = 9000;
+// the latency form's 16-query tiles; a full chip runs them 7 to 13 % slower than
+// 32-query tiles.  Kernel times in us, 16-query against 32-query tiles (these need
+// the plan kernel's 12 to 19 us first, once per pass): one row of 256 keys 11.0 /
+// 14.2, 512: 22.6 / 24.8; 2 x 512: 29.3 / 31.1, 8 x 128: 12.0 / 12.2, 12 x 128: 16.4 /
+// 14.9, 3 x 384: 26.9 / 25.9, 16 x 96: 14.7 / 12.7, so up to kHalfMaxT tokens.
+//
+// Beyond, up to kHalfMaxMixedT tokens, only batches whose longest row is over 1.5
+// times the mean.  Up to kHalfMaxSegs segments they need no plan, and the bound of
+// the lengths stands for the longest row: 1,782 tokens of 16 to 512 keys 31.5 / 45.7,
+// 2,843: 44 / 60.6, 8 rows of 260 behind a bound of 512 39 / 55 per operator call.
+// With more (times per operator call, plan included; the 32-query tiles run rows
+// over kAttnLongL keys in a second launch, the 16-query tiles all rows in one):
+//  * a row of more than kAttnLongL keys among others: 4,353 tokens of 16 to 512 0.88
+//    of the time, 5,138: 0.87, 6,166: 0.91, 7,486: 120.0 / 120.2, 8,126: 127.6 / 126.3,
+//    a pass of 8,985 2,665 / 2,705.  Where only a bound of the lengths is known,
+//    it may be far above them: with rows of up to 300 keys behind a bound of 512,
+//    3,400 tokens 56.7 / 52.9, 8,320: 125 / 112, so up to kHalfMaxBoundT tokens then;
+//  * mostly rows too short for the wide variant: 130 of 8 to 40 and one of 512 0.76
+//    of the time, 130 of 16 to 64 behind a bound of 512 0.84; without a row over
+//    kAttnLongL less far: rows of 8 to 40 and one of 100, 2,553 tokens 29.4 / 30.7,
+//    4,804: 44.1 / 43.5, 7,101: 61.6 / 58.6 (in a pass, whose plan serves all layers,
+//    2,215 tokens 785 / 767);
+//  * else never: 24 rows of 16 to 128 (1,669 tokens) 28.2 / 27.0, 40 of 60 to 260
+//    (6,265) 79 / 71, 32 of 100 to 400 (7,963) 119 / 105.
+constexpr int kHalfMaxT = 1024, kHalfMaxMixedT = 9000, kHalfMaxBoundT = 2500, kHalfMaxShortT = 4000;
 // 16-query tiles (counting the longest row's for every row) whose workgroups, 12
 // per tile, are resident at once at 4 per CU
 constexpr int kHalfResidentTiles = 80;
@@ -1200,19 +1215,26 @@ int attention_form() { return g_attention_form; }
 // tiles: one row of 128 keys 6.6 / 7.4, two of 128 (two rounds) 11 / 7.6.  Passes:
 // one row of 129 427 / 444, 168: 445 / 461; 2 x 66: 414 / 431; 140 + 16: 432 / 448;
 // 80 + 3 x 20: 414 / 429.
-constexpr int kLatMaxTiles = 16;
+constexpr int kLatMaxTiles = 16, kLatMaxT = 256;
 
-int attention_choice(int B, int T, int max_len, int cus) {
+int attention_choice(int B, int T, int max_len, int longest, int cus) {
   if (max_len <= 64) return kAttnTiles32;
-  if (B * (long)((max_len + 31) / 32) <= kLatMaxTiles && 12 * ((T + 7 * B) / 8) <= cus && T <= 256) return kAttnLat;
-  const bool mixed = 2 * (size_t)max_len * B > 3 * (size_t)T;  // the longest row over 1.5 times the mean
-  return T <= (mixed ? kHalfMaxMixedT : kHalfMaxT) ? kAttnTiles16 : kAttnTiles32;
+  if (B * (long)((max_len + 31) / 32) <= kLatMaxTiles && 12 * ((T + 7 * B) / 8) <= cus && T <= kLatMaxT) return kAttnLat;
+  if (T <= kHalfMaxT) return kAttnTiles16;
+  const long top = longest > 0 && B > kHalfMaxSegs ? longest : max_len;
+  const bool is_short = T <= kWideMinMeanLen * (long)B;
+  int most = kHalfMaxMixedT;
+  if (2 * top * B <= 3L * T) most = 0;
+  else if (B > kHalfMaxSegs && top <= kAttnLongL) most = is_short ? kHalfMaxShortT : 0;
+  else if (B > kHalfMaxSegs && longest <= 0 && !is_short) most = kHalfMaxBoundT;
+  return T <= most ? kAttnTiles16 : kAttnTiles32;
 }
 
 void launch_attention(const AttnArgs& p, int T, hipStream_t st, bool plan) {
   if (T <= 0 || p.B <= 0) return;
-  const int max_len = p.s_pitch - 4;  // round16 of the longest sequence
-  const int choice = attention_choice(p.B, T, max_len, device_cu_count());
+  const int max_len = p.s_pitch - 4;  // round16 of the bound of the lengths
+  const int cus = max_len > 64 && T <= kLatMaxT ? device_cu_count() : 0;  // (asked for only where it counts)
+  const int choice = attention_choice(p.B, T, max_len, p.longest, cus);
   const bool lat = g_attention_form != 1 && choice == kAttnLat;
   const bool half = g_attention_form == 2 || (g_attention_form == 0 && choice == kAttnTiles16);
   const int max_tiles = attention_max_tiles(p.B, T);

@@ -226,11 +226,11 @@ struct ae_workspace {
     const void *ids, *cu, *out;
     hipStream_t st;
     int B, T, max_len;
-    int attention_mode;
+    int attention_mode, attention_choice;
     int attention_form, ffn_rows, ffn_exact_gelu;
     bool operator==(const GraphKey& o) const {
       return ids == o.ids && cu == o.cu && out == o.out && st == o.st && B == o.B && T == o.T && max_len == o.max_len &&
-             attention_mode == o.attention_mode && attention_form == o.attention_form && ffn_rows == o.ffn_rows &&
+             attention_mode == o.attention_mode && attention_choice == o.attention_choice && attention_form == o.attention_form && ffn_rows == o.ffn_rows &&
              ffn_exact_gelu == o.ffn_exact_gelu;
     }
   };
@@ -365,11 +365,12 @@ static aek::FfnArgs ffn_args(const ae_linear& up, const ae_linear& down, int m, 
 // one forward pass over a token-packed batch already resident on the device
 // (PackedModel::forward_ragged_cls, src/model.rs:521-914, without its 64-sequence /
 // 512-token limits).  ids/cu may be the workspace's or the caller's buffers;
-// max_len bounds every sequence length (it sizes the attention score rows).
+// max_len bounds every sequence length (it sizes the attention score rows);
+// longest is the longest of them, where it is known (0: not), and chooses kernels.
 // stop_layers >= 0 stops after the embedding and that many encoder layers
 // (a test hook that leaves hidden / act_q / act_scale in the workspace).
-int run_forward(ae_workspace* ws, const uint16_t* ids, const int* cu, int B, int T, int max_len, float* out,
-                hipStream_t st, int stop_layers = -1) {
+int run_forward(ae_workspace* ws, const uint16_t* ids, const int* cu, int B, int T, int max_len, int longest,
+                float* out, hipStream_t st, int stop_layers = -1) {
   const ae_engine* E = ws->e;
   using namespace aek;
   if (ws->timing && ws->ev_used + 2 * 80 > ws->ev_pool.size()) {
@@ -502,6 +503,7 @@ int run_forward(ae_workspace* ws, const uint16_t* ids, const int* cu, int B, int
       AttnArgs a{ws->qkv, cu, B, ws->attn_plan, ws->ctx, D.attn_out.inv_smooth, ws->rowmax_ctx, s_pitch};
       // one sequence: its only segment is [0, T) (a cu_seqlens saying otherwise sets the error word)
       if (B == 1) a.len1 = T;
+      a.longest = longest;
       if (sme) {
         launch_attention_sme(a, sme_args, T, st, /*plan=*/l == 0);
         launch_attention_short(a, st);
@@ -640,13 +642,17 @@ int run_forward(ae_workspace* ws, const uint16_t* ids, const int* cu, int B, int
 // run_forward through the workspace's graph cache: the same launch parameters a
 // second time are captured into a hipGraph, later calls replay it (one launch
 // instead of ~90).  Eager when timing is on or the stream is already capturing.
-int run_forward_replay(ae_workspace* ws, const uint16_t* ids, const int* cu, int B, int T, int max_len, float* out,
-                       hipStream_t st) {
-  if (!ws->graphs || ws->timing) return run_forward(ws, ids, cu, B, T, max_len, out, st);
+int run_forward_replay(ae_workspace* ws, const uint16_t* ids, const int* cu, int B, int T, int max_len, int longest,
+                       float* out, hipStream_t st) {
+  if (!ws->graphs || ws->timing) return run_forward(ws, ids, cu, B, T, max_len, longest, out, st);
   hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
   if (hipStreamIsCapturing(st, &cs) != hipSuccess || cs != hipStreamCaptureStatusNone)
-    return run_forward(ws, ids, cu, B, T, max_len, out, st);
-  const ae_workspace::GraphKey key{ids, cu, out, st, B, T, max_len, ws->attention_mode, aek::attention_form(),
+    return run_forward(ws, ids, cu, B, T, max_len, longest, out, st);
+  // (of longest, a graph holds only the attention kernels that it chose)
+  const int choice = ws->attention_mode == AE_ATTENTION_EXACT
+                         ? aek::attention_choice(B, T, aek::attention_pitch(max_len) - 4, longest, aek::device_cu_count())
+                         : 0;
+  const ae_workspace::GraphKey key{ids, cu, out, st, B, T, max_len, ws->attention_mode, choice, aek::attention_form(),
                                    aek::ffn_rows(), aek::ffn_exact_gelu() ? 1 : 0};
   ws->graph_tick++;
   ae_workspace::GraphEntry* hit = nullptr;
@@ -668,12 +674,12 @@ int run_forward_replay(ae_workspace* ws, const uint16_t* ids, const int* cu, int
       ws->graph_cache.erase(lru);
     }
     ws->graph_cache.push_back({key, nullptr, ws->graph_tick});
-    return run_forward(ws, ids, cu, B, T, max_len, out, st);
+    return run_forward(ws, ids, cu, B, T, max_len, longest, out, st);
   }
   // second use: capture, instantiate, launch
   DevLock lock(g_dev_mu);
   HIP_TRY(hipStreamBeginCapture(st, hipStreamCaptureModeThreadLocal));
-  const int rc = run_forward(ws, ids, cu, B, T, max_len, out, st);
+  const int rc = run_forward(ws, ids, cu, B, T, max_len, longest, out, st);
   hipGraph_t graph = nullptr;
   const hipError_t end = hipStreamEndCapture(st, &graph);
   if (rc != AE_OK) {
@@ -733,6 +739,7 @@ struct DevBatch {
   size_t first;      // first sequence (in length order)
   int B, T;          // real sequences and tokens
   int Bp, Tp, Lp;    // the launched shape (bucketed, or the real one)
+  int longest;       // its longest sequence, the dummies of a bucketed shape included
   size_t ids_off, cu_off;
 };
 
@@ -778,6 +785,8 @@ int run_sequences(const ae_engine* e, ae_workspace* ws, const std::vector<const 
       d.Tp = d.T;
       d.Lp = max_len;
     }
+    const int D = d.Bp - d.B;
+    d.longest = D ? std::max(max_len, (d.Tp - d.T + D - 1) / D) : max_len;
     d.ids_off = ids_total;
     d.cu_off = cu_total;
     ids_total += size_t(d.Tp);
@@ -808,7 +817,8 @@ int run_sequences(const ae_engine* e, ae_workspace* ws, const std::vector<const 
     std::memset(bi + d.T, 0, size_t(P) * sizeof(uint16_t));
     HIP_TRY(hipMemcpyAsync(ws->ids, bi, size_t(d.Tp) * sizeof(uint16_t), hipMemcpyHostToDevice, ws->stream));
     HIP_TRY(hipMemcpyAsync(ws->cu, bc, size_t(d.Bp + 1) * sizeof(int), hipMemcpyHostToDevice, ws->stream));
-    if (int rc = run_forward_replay(ws, ws->ids, ws->cu, d.Bp, d.Tp, d.Lp, ws->out_c, ws->stream)) return rc;
+    if (int rc = run_forward_replay(ws, ws->ids, ws->cu, d.Bp, d.Tp, d.Lp, d.longest, ws->out_c, ws->stream))
+      return rc;
     HIP_TRY(hipMemcpyAsync(h_out + d.first * ae::kHidden, ws->out_c, size_t(d.B) * ae::kHidden * sizeof(float),
                            hipMemcpyDeviceToHost, ws->stream));
   }
@@ -823,6 +833,10 @@ int check_ids(const uint16_t* ids, size_t n) {
     if (ids[i] >= ae::kVocab) return fail(AE_ERR_INVALID_ARG, "token id " + std::to_string(ids[i]) + " >= vocab size");
   return AE_OK;
 }
+
+// the longest sequence by the max_seq_len that a caller states: a program that
+// gives the model's limit says nothing about its batch
+int stated_longest(int max_seq_len) { return max_seq_len < ae::kMaxPos ? max_seq_len : 0; }
 
 hipStream_t as_stream(void* s) { return reinterpret_cast<hipStream_t>(s); }
 
@@ -1123,7 +1137,7 @@ int ae_forward_packed_device(const ae_engine* e, ae_workspace* ws, const uint16_
     return fail(AE_ERR_CAPACITY, "packed batch exceeds workspace capacity");
   hipStream_t st = stream ? as_stream(stream) : ws->stream;
   return run_forward_replay(ws, ids_dev, cu_seqlens_dev, n_seqs, total_tokens,
-                            max_seq_len ? max_seq_len : ae::kMaxPos, out_dev, st);
+                            max_seq_len ? max_seq_len : ae::kMaxPos, stated_longest(max_seq_len), out_dev, st);
 }
 
 float ae_cosine_similarity(const float* a, const float* b) {  // src/lib.rs:265-271
@@ -1291,6 +1305,7 @@ static int attention_varlen(const float* qkv_dev, const int32_t* cu_seqlens_dev,
     aek::init_attention_sme_kernels();
     aek::launch_attention_sme(a, sa, total_tokens, as_stream(stream));
   } else {
+    a.longest = std::min(max_len, ae::kMaxPos);
     aek::launch_attention(a, total_tokens, as_stream(stream));
   }
   const hipError_t err = hipStreamSynchronize(as_stream(stream));
@@ -1324,6 +1339,7 @@ int ae_attention_varlen_noalloc(const float* qkv_dev, const int32_t* cu_seqlens_
   // max_seq_len gives unspecified values, never an access outside the rows
   aek::launch_sanitize_segments(cu_seqlens_dev, n_seqs, total_tokens, max_seq_len, /*strict=*/false, nullptr, cs, st);
   aek::AttnArgs a{qkv_dev, cs, n_seqs, plan, ctx_dev, nullptr, nullptr, aek::attention_pitch(max_seq_len)};
+  a.longest = stated_longest(max_seq_len);
   aek::launch_attention(a, total_tokens, st);
   HIP_TRY(hipGetLastError());
   return AE_OK;
@@ -1349,6 +1365,7 @@ static int workspace_attention(ae_workspace* ws, const float* qkv_dev, const int
   aek::launch_sanitize_segments(cu_dev, n_seqs, total_tokens, max_seq_len, /*strict=*/true, ws->err, ws->cu_safe, st);
   aek::AttnArgs a{qkv_dev, ws->cu_safe, n_seqs, ws->attn_plan, ctx_dev, nullptr, nullptr,
                   aek::attention_pitch(max_seq_len)};
+  a.longest = stated_longest(max_seq_len);
   if (quantized) aek::launch_attention_sme(a, ws->sme, total_tokens, st);  // per_seq = 0: the batch's V scales
   else aek::launch_attention(a, total_tokens, st);
   HIP_TRY(hipGetLastError());
@@ -1570,7 +1587,7 @@ int ae_debug_forward_prefix(const ae_engine* e, ae_workspace* ws, const uint16_t
   std::memcpy(h_ids, ids, size_t(T) * sizeof(uint16_t));
   HIP_TRY(hipMemcpyAsync(ws->ids, h_ids, size_t(T) * sizeof(uint16_t), hipMemcpyHostToDevice, ws->stream));
   HIP_TRY(hipMemcpyAsync(ws->cu, h_cu, (n + 1) * sizeof(int), hipMemcpyHostToDevice, ws->stream));
-  if (int rc = run_forward(ws, ws->ids, ws->cu, int(n), T, max_len, nullptr, ws->stream, layers)) return rc;
+  if (int rc = run_forward(ws, ws->ids, ws->cu, int(n), T, max_len, max_len, nullptr, ws->stream, layers)) return rc;
   HIP_TRY(hipMemcpyAsync(hidden, ws->hidden, size_t(T) * 384 * 4, hipMemcpyDeviceToHost, ws->stream));
   HIP_TRY(hipMemcpyAsync(act_q, ws->act_q, size_t(T) * 384, hipMemcpyDeviceToHost, ws->stream));
   HIP_TRY(hipMemcpyAsync(act_scale, ws->act_scale, size_t(T) * 4, hipMemcpyDeviceToHost, ws->stream));
@@ -1593,8 +1610,8 @@ int ae_debug_set_attention_form(int form) {
 }
 
 // test hook: the exact attention's kernels by the batch (no device access)
-int ae_debug_attention_choice(int n_seqs, int total_tokens, int max_seq_len, int cus) {
-  return aek::attention_choice(n_seqs, total_tokens, aek::attention_pitch(max_seq_len) - 4, cus);
+int ae_debug_attention_choice(int n_seqs, int total_tokens, int max_seq_len, int longest, int cus) {
+  return aek::attention_choice(n_seqs, total_tokens, aek::attention_pitch(max_seq_len) - 4, longest, cus);
 }
 
 // test hook: the rule that keeps the 16-row workgroups of the int8 GEMM (no device access)

@@ -182,9 +182,10 @@ struct AttnArgs {
   float* ctx;              // [T,384]
   const float* smooth;     // attn_out inv_smooth [384] or null
   uint32_t* rowmax;        // [T] or null
-  int s_pitch;             // score row pitch: attention_pitch(max sequence length)
+  int s_pitch;             // score row pitch: attention_pitch(bound of the sequence lengths)
   int skip_from = 0;       // attention_rows_kernel: segments of at least this many tokens are left out (0: none)
   int len1 = 0;            // B == 1 and cu_seqlens = {0, len1} known on the host: the latency form needs no load
+  int longest = 0;         // the longest segment, where the host knows it (it chooses the kernels; 0: not known)
 };
 int attention_pitch(int max_len);
 size_t attention_lds_bytes(int s_pitch);
@@ -213,10 +214,11 @@ hipError_t noalloc_plan_scratch(int** plan);
 // (launch_attention_plan, which depends only on cu, B and s_pitch)
 void launch_attention(const AttnArgs& p, int T, hipStream_t st, bool plan = true);
 // the exact attention's kernels for B segments, T tokens and rows of at most max_len
-// keys on a GPU of cus compute units: 32-query tiles (register rows up to 64 keys),
-// 16-query tiles, or attention_lat_kernel.  Every choice gives the same bits.
+// keys, the longest of them of `longest` (0: not known), on a GPU of cus compute units:
+// 32-query tiles (register rows up to 64 keys), 16-query tiles, or
+// attention_lat_kernel.  Every choice gives the same bits.
 enum AttnChoice { kAttnTiles32 = 0, kAttnTiles16 = 1, kAttnLat = 2 };
-int attention_choice(int B, int T, int max_len, int cus);
+int attention_choice(int B, int T, int max_len, int longest, int cus);
 // split = 1: rows of more than 384 keys in the plan's second list
 void launch_attention_plan(const AttnArgs& p, hipStream_t st, int split, int max_tiles);
 // exact-attention kernel choice for later launches: 0 by the batch, 1 tiled (32 queries) /

@@ -59,7 +59,25 @@ def test_noalloc_attention_refuses_before_any_device_work():
     ([64], 0), ([128] * 12, 0)])
 def test_attention_choice(lens, choice):
     """Which kernels the exact attention takes by the batch (256 compute units)."""
-    assert ae.attention_choice(len(lens), sum(lens), max(lens)) == choice
+    assert ae.attention_choice(len(lens), sum(lens), max(lens), max(lens)) == choice
+
+
+@pytest.mark.parametrize("n_seqs,tokens,bound,longest,choice", [
+    # 16-query tiles beyond 1,024 tokens: the longest row over 1.5 times the mean; as launched by
+    # embed_batch (bound: the longest up to a power of two)
+    (32, 8192, 512, 260, 0), (104, 7168, 128, 66, 0), (64, 8192, 256, 130, 0), (24, 7168, 512, 300, 0),
+    # up to 16 segments, by the bound
+    (12, 2843, 512, 506, 1), (16, 4040, 400, 398, 1), (16, 9001, 512, 512, 0), (8, 2048, 512, 260, 1),
+    # more, with rows over 400 keys: further where the longest row is known
+    (17, 4353, 502, 502, 1), (30, 8985, 496, 496, 1), (30, 9001, 496, 496, 0),
+    (20, 2490, 512, 0, 1), (20, 2501, 512, 0, 0), (20, 5138, 512, 0, 0),
+    # more, up to 400 keys: not unless the rows are mostly short
+    (24, 1669, 127, 127, 0), (40, 6265, 260, 260, 0), (32, 7963, 385, 385, 0), (17, 4420, 400, 0, 0),
+    (64, 1578, 100, 100, 1), (200, 4000, 100, 100, 1), (200, 4774, 100, 100, 0), (60, 1024, 512, 0, 1),
+    # mostly short rows behind a long one, or behind a bound of 512
+    (130, 3764, 512, 512, 1), (130, 5087, 512, 0, 1), (200, 9000, 512, 0, 1), (200, 9001, 512, 0, 0)])
+def test_attention_choice_by_the_longest_row(n_seqs, tokens, bound, longest, choice):
+    assert ae.attention_choice(n_seqs, tokens, bound, longest) == choice
 
 
 @pytest.mark.parametrize("m,n,k,residual,rows16", [

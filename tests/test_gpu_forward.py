@@ -461,6 +461,21 @@ def test_graph_replay_matches_eager(engine, oracle_model, torch_gpu):
     ws.close()
 
 
+def test_graphs_of_one_shape_with_other_longest_rows(engine, oracle_model):
+    """Two batches that pad to one shape (24 sequences, 1,536 tokens, bound 512) but whose longest
+    rows choose other attention kernels: in turn, each through its own captured graph, bit-exact."""
+    rng = np.random.default_rng(43)
+    row = lambda n: np.concatenate([[101], rng.integers(1000, 30522, n - 2), [102]]).astype(np.uint16)
+    batches = [[row(257)] + [row(60) for _ in range(19)], [row(500)] + [row(47) for _ in range(19)]]
+    assert [ae.attention_choice(24, 1536, 512, n) for n in (257, 500)] == [0, 1]
+    refs = [np.stack([oracle_model.forward_cls(s) for s in b]) for b in batches]
+    w = engine.workspace(2048, 40)
+    for rep in range(4):  # 1st call eager, 2nd captures, then replays
+        for k, (b, ref) in enumerate(zip(batches, refs)):
+            assert np.array_equal(engine.embed_batch_tokens(w, b).view(np.uint32), ref.view(np.uint32)), (rep, k)
+    w.close()
+
+
 @pytest.fixture(scope="module")
 def ws_quant(engine):
     w = engine.workspace(8192, 64)

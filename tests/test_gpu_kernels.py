@@ -616,8 +616,9 @@ def test_attention_bit_exact(torch_gpu, attention_form, lens):
 # 42 tiles of 16 queries with eight waves, up to 80 all resident at once, else longest
 # first), from 17 on the plan's; one row of up to 168 tokens, or a few short ones of
 # about as many in all, have a kernel of their own (up to 128 and up to 256 keys); by the
-# batch up to 1,024 tokens, or 9,000 where the longest row is over 1.5 times the mean.
-# Each set takes the latency form and the 32-query tiles.
+# batch up to 1,024 tokens, or, where the longest row is over 1.5 times the mean, up to
+# 9,000 with 16 segments or with a row over 400 (2,500 where the longest row is not known
+# and the rows are not mostly short).  Each set takes the latency form and the 32-query tiles.
 LATENCY_LENS = {"one_65": [65], "one_128": [128], "one_129": [129], "one_161": [161], "one_168": [168],
                 "one_169": [169], "one_497": [497], "few_66_66": [66, 66], "few_140_16": [140, 16],
                 "few_80_20_20_20": [80, 20, 20, 20], "few_129_1_30": [129, 1, 30], "few_88_90": [88, 90],
@@ -627,6 +628,8 @@ LATENCY_LENS = {"one_65": [65], "one_128": [128], "one_129": [129], "one_161": [
                 "segments_16": [96, 95, 97] + [15, 16, 17, 31, 32, 33, 47, 48, 49, 63, 64, 65, 1],
                 "segments_17": [96, 95, 97] + [15, 16, 17, 31, 32, 33, 47, 48, 49, 63, 64, 65, 1, 2],
                 "even_1024": [128] * 8, "even_1025": [128] * 7 + [129],
+                "bound_2500": [130] * 18 + [160], "bound_2501": [130] * 18 + [161],
+                "short_4000": [100] + [20] * 195, "short_4001": [100] + [20] * 194 + [21],
                 "mixed_9000": [512] * 4 + [200] * 34 + [152], "mixed_9001": [512] * 4 + [200] * 34 + [153],
                 **{k: v for k, v in ATTN_LENS.items() if k.startswith("tiled")}}
 
