@@ -554,12 +554,10 @@ int run_forward(ae_workspace* ws, const uint16_t* ids, const int* cu, int B, int
       if (!(stop_layers >= 0 && l + 1 == stop_layers)) ln2.dst = nullptr;
     }
     const FfnArgs ffn = ffn_args(D.ffn_inter, D.ffn_out, T, ws->act_q, ws->act_scale, ws->hidden, ws->tmp);
-    const bool ffn_ln = ffn_fuses_ln(ffn);
     {  // FFN-up, GELU, quantize and FFN-down in one kernel (up to 4,096 rows, LN2 too)
       KernelTimer kt(ws, st, AE_KERNEL_GEMM_FFN_UP);
-      launch_ffn(ffn, st, ws->side, ws->fork_ev, ws->join_ev, ffn_ln ? &ln2 : nullptr);
+      if (launch_ffn(ffn, st, ws->side, ws->fork_ev, ws->join_ev, &ln2)) continue;
     }
-    if (ffn_ln) continue;
     KernelTimer kt(ws, st, AE_KERNEL_LN2);
     launch_ln_quant(ln2, kLnSrcF32, st);
   }

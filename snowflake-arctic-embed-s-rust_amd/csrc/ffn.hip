@@ -679,21 +679,17 @@ static FfnPlan ffn_plan(const FfnArgs& p) {
   return {tile, m64, tail};
 }
 
-// in one round of 16-row workgroups, which all end on the LayerNorm's in-order sums together
-bool ffn_fuses_ln(const FfnArgs& p) {
-  const FfnPlan plan = ffn_plan(p);
-  return p.M > 0 && plan.m64 == 0 && plan.tile == 16;
-}
-
-void launch_ffn(const FfnArgs& p, hipStream_t st, hipStream_t side, hipEvent_t fork, hipEvent_t join, const LnArgs* ln) {
-  if (p.M <= 0) return;
+bool launch_ffn(const FfnArgs& p, hipStream_t st, hipStream_t side, hipEvent_t fork, hipEvent_t join, const LnArgs* ln) {
+  if (p.M <= 0) return false;
   const FfnPlan plan = ffn_plan(p);
   const long m64 = plan.m64;
   const int tail = plan.tail;
   if (m64 == 0) {
-    if (ln && plan.tile == 16) launch_ffn_rows<1, 1, true>(p, st, *ln);
+    // 16-row workgroups run in one round (ffn_plan), so all end on the LayerNorm's in-order sums together
+    const bool fused = ln && plan.tile == 16;
+    if (fused) launch_ffn_rows<1, 1, true>(p, st, *ln);
     else launch_ffn_tile(p, plan.tile, st);
-    return;
+    return fused;
   }
   FfnArgs a = p, b = p;
   a.M = (int)m64;
@@ -713,6 +709,7 @@ void launch_ffn(const FfnArgs& p, hipStream_t st, hipStream_t side, hipEvent_t f
     launch_ffn_tile(a, 64, st);
     launch_ffn_tile(b, tail, st);
   }
+  return false;
 }
 
 }  // namespace aek

@@ -70,14 +70,14 @@ struct FfnArgs {
 // work queued on st, joined before st continues), so its partial round of
 // workgroups fills CUs as the 64-row rounds free them instead of running alone
 // at the end
-// ln (only when ffn_fuses_ln(p)): the LayerNorm + SmoothQuant of the output rows
-// in the same kernel (ln->src is ignored, ln->rowmax_init2 not written; ln->q may
-// be p.A, ln->scale p.a_scale and ln->dst p.res: a workgroup has read its rows
-// before it writes them)
+// ln (optional): the LayerNorm + SmoothQuant of the output rows in the same kernel
+// where its workgroups are 16 rows high (ln->src is ignored, ln->rowmax_init2 not
+// written; ln->q may be p.A, ln->scale p.a_scale and ln->dst p.res: a workgroup has
+// read its rows before it writes them).  Returns whether the launch includes it;
+// if not, it is the caller's to launch.
 struct LnArgs;
-void launch_ffn(const FfnArgs& p, hipStream_t st, hipStream_t side = nullptr, hipEvent_t fork = nullptr,
+bool launch_ffn(const FfnArgs& p, hipStream_t st, hipStream_t side = nullptr, hipEvent_t fork = nullptr,
                 hipEvent_t join = nullptr, const LnArgs* ln = nullptr);
-bool ffn_fuses_ln(const FfnArgs& p);
 // test hooks: the exact-GELU kernel for every launch (process-wide); the fast
 // kernel's repair counters on the current device ([0] column tiles recomputed for
 // an undecided quantized value, [1] groups of 16 rows in which a row maximum was
