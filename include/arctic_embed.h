@@ -363,8 +363,9 @@ int ae_debug_set_ffn_exact_gelu(int exact);
 int ae_debug_ffn_repairs(uint64_t* tiles, uint64_t* rows, int reset);
 /* The certification of the fused FFN kernel's fast GELU (a test hook,
  * synchronous, a few seconds): evaluates it and the reference's GELU on all
- * 2^32 f32 inputs on the current device and writes 6 counters: [0] inputs
- * outside the certified bound, [1] NaN results for a non-NaN, finite input,
+ * 2^32 f32 inputs on the current device, both as the kernel does (the fast one
+ * on 4 and on 8 values at once), and writes 6 counters: [0] inputs outside the
+ * certified bound or whose two fast values differ, [1] NaN results for a non-NaN, finite input,
  * [2] / [3] inputs in the saturated ranges where the reference's GELU is not
  * exactly v / 0, [4] inputs outside the bound with half its absolute term (must
  * be nonzero: the check can fail), [5] inputs checked (2^32). */

@@ -258,26 +258,16 @@ constexpr float kGeluFastRel = 0x1p-21f;
 constexpr float kGeluFastAbs = 0x1.64p-24f;
 constexpr float kGeluSatPos = 0x1.563c42p+2f;   // the float after 5.34742737 (0x1.563c4p+2)
 constexpr float kGeluSatNeg = -0x1.62c12ep+2f;  // the float below -5.54304028 (-0x1.62c12cp+2)
-__device__ __forceinline__ float gelu_fast(float v) {
-  constexpr float kA1 = 0.5f * 0.254829592f, kA2 = 0.5f * -0.284496736f, kA3 = 0.5f * 1.421413741f,
-                  kA4 = 0.5f * -1.453152027f, kA5 = 0.5f * 1.061405429f;
-  const float y = __builtin_fmaf(fabsf(v), 0.3275911f * 0.70710677f, 1.0f);
-  const float t = __builtin_amdgcn_rcpf(y);
-  const float ph = t * __builtin_fmaf(__builtin_fmaf(__builtin_fmaf(__builtin_fmaf(kA5, t, kA4), t, kA3), t, kA2), t, kA1);
-  const float e = __builtin_amdgcn_exp2f(v * (v * (-0.5f * 1.44269504088896340736f)));
-  return __builtin_fmaf(-fabsf(v), ph * e, fmaxf(v, 0.0f));
-}
-
-// The same for N values at once, operation by operation (bit for bit gelu_fast):
-// a dependent VALU instruction issues about 10 cycles after its source, so a
-// wave beside one other on its SIMD needs several independent chains in flight;
-// the scheduling barriers keep the compiler from serializing them again (it
-// orders the values one after the other to save registers).
-// kc: 0.3275911f * 0.70710677f in a VGPR (its instruction takes |v|, so it cannot
-// hold the constant itself, and an f32 instruction that reads an SGPR issues at
-// half the rate).  The maximum by hand: fmaxf would canonicalize v first.
+constexpr float kGeluFastK = 0.3275911f * 0.70710677f;  // p / sqrt 2
+// N values at once: a dependent VALU instruction issues about 10 cycles after its
+// source, so a wave beside one other on its SIMD needs several independent chains
+// in flight; the scheduling barriers keep the compiler from serializing them again
+// (it orders the values one after the other to save registers).
+// kc: kGeluFastK in a VGPR (its instruction takes |v|, so it cannot hold the
+// constant itself, and an f32 instruction that reads an SGPR issues at half the
+// rate).  The maximum by hand: fmaxf would canonicalize v first.
 template <int N>
-__device__ __forceinline__ void gelu_fast_n(const float (&v)[N], float kc, float (&out)[N]) {
+__device__ __forceinline__ void gelu_fast(const float (&v)[N], float kc, float (&out)[N]) {
   constexpr float kA1 = 0.5f * 0.254829592f, kA2 = 0.5f * -0.284496736f, kA3 = 0.5f * 1.421413741f,
                   kA4 = 0.5f * -1.453152027f, kA5 = 0.5f * 1.061405429f;
   float t[N], a[N], ph[N], m[N];

@@ -202,7 +202,7 @@ __global__ __launch_bounds__(kThreads, 2) void ffn_kernel(FfnArgs p, LnArgs ln) 
   }
   const ExpTabLds tb{s_tab};
   // (constants that an f32 instruction would otherwise read from an SGPR, at half its rate)
-  float kc = 0.3275911f * 0.70710677f, kcap = kCapMul, kq = kQRel;
+  float kc = kGeluFastK, kcap = kCapMul, kq = kQRel;
   asm volatile("" : "+v"(kc), "+v"(kcap), "+v"(kq));
   // opaque per phase: addresses formed from them are not kept from one phase to the next (spills)
   auto opaque_ids = [&]() { asm volatile("" : "+v"(tid), "+v"(lane), "+v"(fr), "+v"(fq)); };
@@ -393,7 +393,7 @@ __global__ __launch_bounds__(kThreads, 2) void ffn_kernel(FfnArgs p, LnArgs ln) 
         float vv[N], x[N], t[N], d[N], gi[N];
 #pragma unroll
         for (int k = 0; k < N; k++) vv[k] = v[k >> 2][k & 3][j];
-        gelu_fast_n<N>(vv, kc, x);
+        gelu_fast<N>(vv, kc, x);
         auto each = [&](auto f) {
 #pragma unroll
           for (int k = 0; k < N; k++) f(k);
@@ -576,9 +576,11 @@ void set_ffn_exact_gelu(bool exact) { g_ffn_exact_gelu = exact; }
 bool ffn_exact_gelu() { return g_ffn_exact_gelu; }
 
 // The certification of gelu_fast (device_common.hpp) over all 2^32 f32 inputs
-// against gelu_exact, both as the kernels evaluate them.  Counters: [0] inputs
-// breaking the certified bound (G' NaN only for NaN / +-inf v, else gelu_exact
-// finite and |G - G'| <= kGeluFastRel |G'| + kGeluFastAbs, in f64), [1] NaN G'
+// against gelu_exact, both as ffn_kernel evaluates them (gelu_fast on 8 values at
+// once, its 32- and 64-row workgroups, and on 4, its 16-row ones).  Counters: [0]
+// inputs breaking the certified bound (G' NaN only for NaN / +-inf v, else
+// gelu_exact finite and |G - G'| <= kGeluFastRel |G'| + kGeluFastAbs, in f64) or
+// whose two G' differ in a bit, [1] NaN G'
 // for another v, [2] v >= kGeluSatPos with gelu_exact(v) != v, [3] finite
 // v <= kGeluSatNeg with gelu_exact(v) != 0, [4] inputs breaking the bound with
 // half its absolute term (a too-tight bound must fail: the check is not
@@ -587,9 +589,23 @@ __global__ __launch_bounds__(256) void gelu_fast_certify_kernel(unsigned long lo
   const ExpTab tb = exp_tab_regs();
   const uint32_t i0 = base + (blockIdx.x * 256u + threadIdx.x) * 16u;
   unsigned c[6] = {0, 0, 0, 0, 0, 0};
+  float kc = kGeluFastK;
+  asm volatile("" : "+v"(kc));
+  float v8[8], g8[8], v4[4], g4[4];
+#pragma unroll
   for (int u = 0; u < 16; u++) {
-    const float v = __uint_as_float(i0 + (uint32_t)u);
-    const float G = gelu_exact(v, tb), Gp = gelu_fast(v);
+    if (u % 8 == 0) {
+#pragma unroll
+      for (int k = 0; k < 8; k++) v8[k] = __uint_as_float(i0 + (uint32_t)(u + k));
+      gelu_fast<8>(v8, kc, g8);
+    }
+    if (u % 4 == 0) {
+#pragma unroll
+      for (int k = 0; k < 4; k++) v4[k] = __uint_as_float(i0 + (uint32_t)(u + k));
+      gelu_fast<4>(v4, kc, g4);
+    }
+    const float v = v8[u % 8], G = gelu_exact(v, tb), Gp = g8[u % 8];
+    if (__float_as_uint(g4[u % 4]) != __float_as_uint(Gp)) c[0]++;
     const bool special = __builtin_isnan(v) || __builtin_isinf(v);
     if (__builtin_isnan(Gp)) {
       if (!special) c[1]++;
