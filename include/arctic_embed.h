@@ -307,13 +307,20 @@ int ae_debug_gemm_ln(const ae_linear* l, int m, const float* x_dev, const uint32
  * rowmax[m] = max(rowmax[m], max_n |g|) on f32 bits (caller pre-sets rowmax). */
 int ae_debug_gemm_gelu(const ae_linear* l, int m, const int8_t* a_dev, const float* a_scale_dev,
                        const float* g_smooth_dev, float* out_dev, uint32_t* rowmax_dev, void* stream);
-/* The FFN block of src/model.rs:725-755 as the forward pass runs it at large
- * token counts (one kernel, no [m,1536] intermediate in memory):
+/* The FFN block of src/model.rs:725-755 as the forward pass runs it beyond 1,024
+ * tokens (one kernel, no [m,1536] intermediate in memory):
  * out = gemm_int8_fused(ffn_out, gelu_smooth_quantize(gemm_int8_fused(ffn_inter, a)), res).
  * up: 384 -> 1536 linear, down: 1536 -> 384 linear (its inv_smooth smooths the
  * GELU output).  out may equal res. */
 int ae_debug_ffn(const ae_linear* up, const ae_linear* down, int m, const int8_t* a_dev, const float* a_scale_dev,
                  const float* res_dev, float* out_dev, void* stream);
+/* ae_debug_ffn with the LayerNorm + SmoothQuant of its output rows in the same
+ * kernel (src/model.rs:756-767), as a pass of 1,025 to 4,096 tokens runs it:
+ * dst = LayerNorm(out), q / scale its int8 rows.  AE_ERR_INVALID_ARG if m rows are
+ * more than one round of 16-row workgroups (4,096 on 256 compute units). */
+int ae_debug_ffn_ln(const ae_linear* up, const ae_linear* down, int m, const int8_t* a_dev, const float* a_scale_dev,
+                    const float* res_dev, float* out_dev, const float* gamma_dev, const float* beta_dev,
+                    const float* ln_smooth_dev, float* dst_dev, int8_t* q_dev, float* scale_dev, void* stream);
 /* Embedding + the first `layers` (0..11) encoder layers over one packed batch of n
  * sequences (given order, each 1..512 ids); copies back hidden [T,384] f32,
  * act_q [T,384] int8 and act_scale [T] (T = offsets[n]), the state that
@@ -344,8 +351,8 @@ int ae_debug_attention_choice(int n_seqs, int total_tokens, int max_seq_len, int
  * counterpart, no device access): 1 or 0.  Either form gives the same bits. */
 int ae_debug_gemm_int8_rows16(int m, int n, int k, int residual, int cus);
 /* Token rows per workgroup of the fused FFN kernel, process-wide (a test hook,
- * no reference counterpart): 0 by the batch's size (the default), 32 or 64, or
- * -m (m a multiple of 64): the first m rows in 64-row workgroups and the rest
+ * no reference counterpart): 0 by the batch's size (the default), 16, 32 or 64,
+ * or -m (m a multiple of 64): the first m rows in 64-row workgroups and the rest
  * in a second launch of 32-row ones.  Every plan gives the same bits.
  * AE_ERR_INVALID_ARG for another value. */
 int ae_debug_set_ffn_rows(int rows);
@@ -357,9 +364,9 @@ int ae_debug_set_ffn_rows(int rows);
  * element.  Both give the same bits. */
 int ae_debug_set_ffn_exact_gelu(int exact);
 /* Counters of the fast FFN kernel's exact recomputations on the current device
- * (a test hook): *tiles = 16-column tiles of 4 rows recomputed for an undecided
- * quantized value, *rows = groups of 16 rows in which a row maximum was settled
- * among several exactly evaluated elements; reset != 0 clears them after reading. */
+ * (a test hook): *tiles = tiles of 16 rows x 16 columns recomputed for an undecided
+ * quantized value, *rows = the 16-row groups (one or two) of each pass that
+ * evaluated more candidates for its row maxima than it has rows; reset != 0 clears them after reading. */
 int ae_debug_ffn_repairs(uint64_t* tiles, uint64_t* rows, int reset);
 /* The certification of the fused FFN kernel's fast GELU (a test hook,
  * synchronous, a few seconds): evaluates it and the reference's GELU on all

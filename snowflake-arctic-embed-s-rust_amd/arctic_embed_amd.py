@@ -93,6 +93,7 @@ _SIGS = {
     "ae_debug_gemm_gelu": (_i32, [_vp, _i32, _vp, _vp, _vp, _vp, _vp, _vp]),
     "ae_debug_gemm_ln": (_i32, [_vp, _i32, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp]),
     "ae_debug_ffn": (_i32, [_vp, _vp, _i32, _vp, _vp, _vp, _vp, _vp]),
+    "ae_debug_ffn_ln": (_i32, [_vp, _vp, _i32] + [_vp] * 11),
     "ae_parallel_context_create": (_i32, [_vp, _i32, _c.POINTER(_vp)]),
     "ae_parallel_context_destroy": (None, [_vp]),
     "ae_parallel_context_threads": (_i32, [_vp]),
@@ -436,6 +437,13 @@ class Linear:
         (384 -> 1536) and `down` as FFN-down (1536 -> 384); out may equal res."""
         _check(_lib.ae_debug_ffn(self._h, down._h, int(m), a_ptr, a_scale_ptr, res_ptr, out_ptr, stream))
 
+    def ffn_ln(self, down, m, a_ptr, a_scale_ptr, res_ptr, out_ptr, gamma_ptr, beta_ptr, ln_smooth_ptr, dst_ptr, q_ptr,
+               scale_ptr, stream=None):
+        """ffn and the LayerNorm + SmoothQuant of its rows in one kernel (up to one round of 16-row
+        workgroups)."""
+        _check(_lib.ae_debug_ffn_ln(self._h, down._h, int(m), a_ptr, a_scale_ptr, res_ptr, out_ptr, gamma_ptr, beta_ptr,
+                                    ln_smooth_ptr, dst_ptr, q_ptr, scale_ptr, stream))
+
     def close(self):
         if self._h:
             _lib.ae_linear_destroy(self._h)
@@ -506,7 +514,7 @@ def gemm_int8_rows16(m, n, k, residual, cus=256):
 
 def set_ffn_rows(rows):
     """Token rows per workgroup of the fused FFN kernel from now on: 0 by the
-    batch (default), 32 or 64, or -m: the first m rows (a multiple of 64) in 64-row
+    batch (default), 16, 32 or 64, or -m: the first m rows (a multiple of 64) in 64-row
     workgroups, the rest in 32-row ones (a test hook)."""
     _check(_lib.ae_debug_set_ffn_rows(int(rows)))
 
@@ -526,8 +534,8 @@ def gelu_fast_certify():
 
 def ffn_repairs(reset=False):
     """(tiles, rows): the fast FFN kernel's exact recomputations on the current device since the
-    last reset: 16-column tiles recomputed for an undecided quantized value, and groups of 16 rows in
-    which a row maximum was settled among several exactly evaluated elements (a test hook)."""
+    last reset: 16 x 16 tiles recomputed for an undecided quantized value, and the 16-row groups of
+    the passes with more candidates for the row maxima than rows (a test hook)."""
     t, r = ctypes.c_uint64(0), ctypes.c_uint64(0)
     _check(_lib.ae_debug_ffn_repairs(ctypes.byref(t), ctypes.byref(r), 1 if reset else 0))
     return int(t.value), int(r.value)

@@ -1563,6 +1563,30 @@ int ae_debug_ffn(const ae_linear* up, const ae_linear* down, int m, const int8_t
   return AE_OK;
 }
 
+// test hook: the FFN with the LayerNorm + SmoothQuant of its rows in the same kernel (16-row workgroups)
+int ae_debug_ffn_ln(const ae_linear* up, const ae_linear* down, int m, const int8_t* a_dev, const float* a_scale_dev,
+                    const float* res_dev, float* out_dev, const float* gamma_dev, const float* beta_dev,
+                    const float* ln_smooth_dev, float* dst_dev, int8_t* q_dev, float* scale_dev, void* stream) {
+  if (!up || !down || m <= 0 || !a_dev || !a_scale_dev || !res_dev || !out_dev || !gamma_dev || !beta_dev ||
+      !ln_smooth_dev || !dst_dev || !q_dev || !scale_dev)
+    return fail(AE_ERR_INVALID_ARG, "bad arguments");
+  if (up->k != ae::kHidden || up->n != ae::kInter || down->k != ae::kInter || down->n != ae::kHidden)
+    return fail(AE_ERR_INVALID_ARG, "ffn: expects a 384->1536 and a 1536->384 linear");
+  aek::LnArgs ln{};
+  ln.T = m;
+  ln.gamma = gamma_dev;
+  ln.beta = beta_dev;
+  ln.smooth = ln_smooth_dev;
+  ln.dst = dst_dev;
+  ln.q = q_dev;
+  ln.scale = scale_dev;
+  const bool fused = aek::launch_ffn(ffn_args(*up, *down, m, a_dev, a_scale_dev, res_dev, out_dev),
+                                     as_stream(stream), nullptr, nullptr, nullptr, &ln);
+  HIP_TRY(hipGetLastError());
+  if (!fused) return fail(AE_ERR_INVALID_ARG, "ae_debug_ffn_ln: more rows than one round of 16-row workgroups");
+  return AE_OK;
+}
+
 // test hook: embedding + the first `layers` encoder layers over one packed batch
 // (in the given order); copies hidden [T,384], act_q [T,384], act_scale [T] back
 int ae_debug_forward_prefix(const ae_engine* e, ae_workspace* ws, const uint16_t* ids, const uint32_t* offsets,
@@ -1619,8 +1643,8 @@ int ae_debug_gemm_int8_rows16(int m, int n, int k, int residual, int cus) {
 
 // test hook: the FFN kernel's workgroup height
 int ae_debug_set_ffn_rows(int rows) {
-  if (rows != 0 && rows != 32 && rows != 64 && !(rows < 0 && rows % 64 == 0))
-    return fail(AE_ERR_INVALID_ARG, "FFN rows must be 0, 32, 64 or a negative multiple of 64");
+  if (rows != 0 && rows != 16 && rows != 32 && rows != 64 && !(rows < 0 && rows % 64 == 0))
+    return fail(AE_ERR_INVALID_ARG, "FFN rows must be 0, 16, 32, 64 or a negative multiple of 64");
   aek::set_ffn_rows(rows);
   return AE_OK;
 }

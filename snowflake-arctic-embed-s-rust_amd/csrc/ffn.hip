@@ -107,8 +107,8 @@ constexpr float kCapMul = 1.0854f, kCapSub = 0.2158f, kCapMin = 0.44f;
 constexpr float kCandShare = 0.92f;
 
 // repair counters (test hook ae_debug_ffn_repairs): [0] 16-row x 16-column tiles
-// recomputed exactly because a quantized value was undecided, [1] groups of 16
-// rows in which a row maximum was settled among several exact values
+// recomputed exactly because a quantized value was undecided, [1] the NR 16-row
+// groups of each pass whose first scan had more candidates than the pass has rows
 __device__ unsigned long long g_ffn_repairs[2];
 
 // kFast: the GELU is gelu_fast with exact repair (the same bits as the exact
@@ -568,7 +568,7 @@ __global__ __launch_bounds__(kThreads, 2) void ffn_kernel(FfnArgs p, LnArgs ln) 
   }
 }
 
-static int g_ffn_rows = 0;  // 0 by the batch, 32, 64, or -m: the mixed plan with m rows first (test hook)
+static int g_ffn_rows = 0;  // 0 by the batch, 16, 32, 64, or -m: the mixed plan with m rows first (test hook)
 void set_ffn_rows(int rows) { g_ffn_rows = rows; }
 int ffn_rows() { return g_ffn_rows; }
 static bool g_ffn_exact_gelu = false;  // test hook: the exact-GELU kernel for every launch

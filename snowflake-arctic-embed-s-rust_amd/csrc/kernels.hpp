@@ -79,9 +79,9 @@ struct LnArgs;
 bool launch_ffn(const FfnArgs& p, hipStream_t st, hipStream_t side = nullptr, hipEvent_t fork = nullptr,
                 hipEvent_t join = nullptr, const LnArgs* ln = nullptr);
 // test hooks: the exact-GELU kernel for every launch (process-wide); the fast
-// kernel's repair counters on the current device ([0] column tiles recomputed for
-// an undecided quantized value, [1] groups of 16 rows in which a row maximum was
-// settled among several exact values), optionally reset
+// kernel's repair counters on the current device ([0] 16 x 16 tiles recomputed for
+// an undecided quantized value, [1] the 16-row groups of passes with more candidates
+// for the row maxima than rows), optionally reset
 void set_ffn_exact_gelu(bool exact);
 bool ffn_exact_gelu();
 hipError_t ffn_repair_counts(unsigned long long counts[2], bool reset);

@@ -178,10 +178,10 @@ def test_gemm_quantize_on_load_bit_exact(torch_gpu, smooth, n, k):
     assert np.array_equal(bits(out_d.cpu().numpy()), bits(ref))
 
 
-@pytest.mark.parametrize("m", [37, 1500, 2000])
+@pytest.mark.parametrize("m", [37, 1500, 2000, 4101, 16387])
 def test_gemm_then_layernorm_bit_exact(torch_gpu, m):
-    """The attention output GEMM and LN1 in one kernel (16-row workgroups, at 1,500 rows with a
-    partial last tile): f32 LN rows, int8 rows and scales
+    """The attention output GEMM and LN1 in one kernel (16-row workgroups up to 4,096 rows, 32-row ones
+    of 8 waves up to 16,384, then of 4, with partial last tiles): f32 LN rows, int8 rows and scales
     bit for bit against the oracle's smooth_quantize -> gemm_scalar_fused(residual) ->
     layernorm_smooth_quantize.  Rows include a zero ctx row, a residual row whose mean and variance
     depend on the summation order (+-1e8 against small values) and a constant output row."""
@@ -271,11 +271,11 @@ def test_gemm_gelu_epilogue_bit_exact(torch_gpu, m):
     assert np.array_equal(rowmax / f32(127), sc)
 
 
-@pytest.fixture(params=[32, 64, -64], ids=["rows32", "rows64", "mixed64"])
+@pytest.fixture(params=[16, 32, 64, -64], ids=["rows16", "rows32", "rows64", "mixed64"])
 def ffn_rows(request, torch_gpu):
-    """Every fused-FFN test runs with 32-row and with 64-row workgroups, and with
-    the first 64 rows in a 64-row workgroup and the rest in a second launch of
-    32-row ones."""
+    """Every fused-FFN test runs with 16-, 32- and 64-row workgroups, and with the
+    first 64 rows in a 64-row workgroup and the rest in a second launch of 32-row
+    ones."""
     ae.set_ffn_rows(request.param)
     yield request.param
     ae.set_ffn_rows(0)
@@ -369,7 +369,7 @@ def test_ffn_fast_gelu_repairs_are_exact(torch_gpu, ffn_rows):
     saturated), a tie the kernel settles by recomputing every element that can reach it; (2)
     zero-weight columns whose GELU * inv_smooth lands exactly on k + 0.5 or one ulp either side of
     it (and a negative inv_smooth), so that x = g * (127 / 127) is undecided and the tile is
-    recomputed from its int32 dot products.  Bit-exact with the oracle, the repair counters move,
+    recomputed from its pre-activations.  Bit-exact with the oracle, the repair counters move,
     and the exact-GELU kernel gives the same bits."""
     torch = torch_gpu
     w1, ws1, b1, s1 = linear_inputs(1536, 384, 31)
@@ -407,11 +407,11 @@ def test_ffn_fast_gelu_repairs_are_exact(torch_gpu, ffn_rows):
             torch.cuda.synchronize()
             outs.append(out_d.cpu().numpy())
             tiles, rows = ae.ffn_repairs()
-            print("exact" if exact else "fast", "repairs: tiles", tiles, "row passes", rows, flush=True)
+            print("exact" if exact else "fast", "repairs: tiles", tiles, "16-row groups", rows, flush=True)
             if exact:
                 assert tiles == 0 and rows == 0
             else:
-                assert tiles >= len(cols) and rows >= (m + 31) // 32, (tiles, rows)
+                assert tiles >= len(cols) * ((m + 15) // 16) and rows >= (m + 15) // 16, (tiles, rows)
     finally:
         ae.set_ffn_exact_gelu(False)
     for o in outs:
@@ -419,13 +419,14 @@ def test_ffn_fast_gelu_repairs_are_exact(torch_gpu, ffn_rows):
 
 
 def test_ffn_fast_and_exact_gelu_kernels_agree(torch_gpu):
-    """The fast-GELU and exact-GELU fused FFN kernels give the same bits on a large random batch
-    (both 32- and 64-row workgroups by the launch's plan), and equal the oracle; the fast kernel's
-    repair count is reported."""
+    """The fast-GELU and exact-GELU fused FFN kernels give the same bits on a large random batch (by
+    the launch's plan 16,384 rows in 64-row workgroups, the rest in a second launch of 16-row ones),
+    and equal the oracle at the first rows, across that line and at the last, partial workgroup; the
+    fast kernel's repair count is reported."""
     torch = torch_gpu
     w1, ws1, b1, s1 = linear_inputs(1536, 384, 41)
     w2, ws2, b2, s2 = linear_inputs(384, 1536, 42)
-    m = 20000
+    m = 19999
     rng = np.random.default_rng(43)
     a = rng.integers(-127, 128, (m, 384), dtype=np.int8)
     sa = rng.uniform(0.01, 0.1, m).astype(f32)
@@ -441,12 +442,13 @@ def test_ffn_fast_and_exact_gelu_kernels_agree(torch_gpu):
             up.ffn(down, m, a_d.data_ptr(), sa_d.data_ptr(), res_d.data_ptr(), out_d.data_ptr())
             torch.cuda.synchronize()
             outs.append(out_d.cpu().numpy())
-            print("exact" if exact else "fast", "repairs (tiles, row passes):", ae.ffn_repairs(), flush=True)
+            print("exact" if exact else "fast", "repairs (tiles, 16-row groups):", ae.ffn_repairs(), flush=True)
     finally:
         ae.set_ffn_exact_gelu(False)
     assert np.array_equal(bits(outs[0]), bits(outs[1]))
-    ref = _ffn_ref(a[:300], sa[:300], w1, ws1, b1, w2, ws2, b2, s2, res[:300])
-    assert np.array_equal(bits(outs[0][:300]), bits(ref))
+    for r in (slice(0, 300), slice(16384 - 80, 16384 + 80), slice(m - 72, m)):
+        ref = _ffn_ref(a[r], sa[r], w1, ws1, b1, w2, ws2, b2, s2, res[r])
+        assert np.array_equal(bits(outs[0][r]), bits(ref)), r
 
 
 @pytest.mark.parametrize("m", [1, 15, 16, 17, 47, 1025, 4096, 4097, 8193])
@@ -499,6 +501,52 @@ def test_ffn_row_maximum_candidates(torch_gpu, ffn_rows, m):
         nan = np.isnan(ref)
         assert np.array_equal(nan, np.isnan(got))
         assert np.array_equal(bits(got)[~nan], bits(ref)[~nan])
+
+
+@pytest.mark.parametrize("exact", [False, True], ids=["fast", "exact"])
+def test_ffn_with_layernorm_special_rows(torch_gpu, exact):
+    """The FFN kernel with LN2 in its epilogue on rows that its repairs and its in-order sums decide:
+    tied row maxima and values on a half-integer in every row, zero, infinite and NaN row scales, a
+    residual row whose mean and variance depend on the order of summation (+-1e8 against small
+    values) and a constant one in the last, partial workgroup; in place of the inputs as in a pass.
+    f32 rows, LN rows, int8 rows and scales bit for bit (NaN for NaN) against the oracle's steps."""
+    torch = torch_gpu
+    w1, ws1, b1, s1 = linear_inputs(1536, 384, 71)
+    w2, ws2, b2, s2 = linear_inputs(384, 1536, 72)
+    m = 75
+    for c in (0, 16):  # the row maximum 127, twice
+        w1[c], b1[c], s2[c] = 0, 63.5, 2.0
+    for c, t in ((37, 10.5), (200, 20.5), (399, np.nextafter(f32(6.5), f32(0))), (1535, 100.5)):
+        w1[c], b1[c], s2[c] = 0, t, 1.0
+    rng = np.random.default_rng(73)
+    a = rng.integers(-127, 128, (m, 384), dtype=np.int8)
+    sa = rng.uniform(0.001, 0.02, m).astype(f32)
+    sa[1], sa[2], sa[33] = np.inf, np.nan, 0.0
+    res = rng.normal(0, 1, (m, 384)).astype(f32)
+    res[5, :] = rng.normal(0, 1e-3, 384).astype(f32)
+    res[5, 0], res[5, 1] = f32(1e8), f32(-1e8)
+    res[m - 1], a[m - 1] = f32(2.5), 0
+    gamma, beta = (1 + rng.normal(0, 0.05, 384)).astype(f32), rng.normal(0, 0.02, 384).astype(f32)
+    ln_s = (rng.uniform(0.5, 2.0, 384) ** -1).astype(f32)
+    up, down = ae.Linear(w1, ws1, b1, s1), ae.Linear(w2, ws2, b2, s2)
+    a_d, sa_d, res_d = dev(torch, a), dev(torch, sa), dev(torch, res)
+    g_d, b_d, ls_d = dev(torch, gamma), dev(torch, beta), dev(torch, ln_s)
+    out_d = torch.zeros((m, 384), dtype=torch.float32, device="cuda")
+    ae.set_ffn_exact_gelu(exact)
+    try:
+        up.ffn_ln(down, m, a_d.data_ptr(), sa_d.data_ptr(), res_d.data_ptr(), out_d.data_ptr(), g_d.data_ptr(),
+                  b_d.data_ptr(), ls_d.data_ptr(), res_d.data_ptr(), a_d.data_ptr(), sa_d.data_ptr())
+        torch.cuda.synchronize()
+    finally:
+        ae.set_ffn_exact_gelu(False)
+    ref = _ffn_ref(a, sa, w1, ws1, b1, w2, ws2, b2, s2, res)
+    ry, rq, rsc = orc.ln_quant_rows(ref, gamma, beta, ln_s)
+    for got, want in ((out_d, ref), (res_d, ry), (sa_d, rsc)):
+        got = got.cpu().numpy()
+        nan = np.isnan(want)
+        assert np.array_equal(nan, np.isnan(got))
+        assert np.array_equal(bits(got)[~nan], bits(want)[~nan])
+    assert np.array_equal(a_d.cpu().numpy(), rq)
 
 
 @pytest.mark.parametrize("m", [1, 31, 33, 100])
