@@ -266,7 +266,7 @@ int ae_write_synthetic_ae8(const char* path, uint64_t seed);
 #define AE_KERNEL_GEMM_QKV 1
 #define AE_KERNEL_ATTENTION 2
 #define AE_KERNEL_GEMM_ATTN_OUT 3
-#define AE_KERNEL_LN1 4
+#define AE_KERNEL_LN1 4 /* unused (count 0): LN1 runs in the kernel of GEMM_ATTN_OUT or GEMM_FFN_UP */
 #define AE_KERNEL_GEMM_FFN_UP 5 /* the whole fused FFN block when a pass has more than 1024 tokens (with LN2 while its
                                   16-row workgroups run in one round, 4096 tokens) */
 #define AE_KERNEL_GEMM_FFN_DOWN 6 /* unused (count 0) when the FFN block is fused */

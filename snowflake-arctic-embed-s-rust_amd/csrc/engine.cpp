@@ -185,8 +185,8 @@ struct ae_engine {
 struct ae_workspace {
   const ae_engine* e = nullptr;
   hipStream_t stream = nullptr;
-  // a second stream and its fork / join events: the fused FFN's 32-row launch of
-  // a mixed plan runs there beside the 64-row one (aek::launch_ffn)
+  // a second stream and its fork / join events: the fused FFN's launch of short
+  // workgroups in a mixed plan runs there beside the 64-row one (aek::launch_ffn)
   hipStream_t side = nullptr;
   hipEvent_t fork_ev = nullptr, join_ev = nullptr;
   int max_tokens = 0, max_seqs = 0;
@@ -199,7 +199,8 @@ struct ae_workspace {
   int attention_mode = AE_ATTENTION_EXACT;
   aek::SmeArgs sme{};
   int* err = nullptr;        // device error word: bit 0 = a packed batch with a bad segment (ae_workspace_synchronize)
-  float *hidden = nullptr, *tmp = nullptr, *qkv = nullptr, *ctx = nullptr, *g = nullptr;
+  float *hidden = nullptr, *tmp = nullptr, *qkv = nullptr, *ctx = nullptr;
+  float* g = nullptr;        // [min(max_tokens, kSmallM), 1536]: the FFN's intermediate of the few-row path (and rowmax_g)
   int8_t* act_q = nullptr;
   float* act_scale = nullptr;
   uint32_t *rowmax_ctx = nullptr, *rowmax_g = nullptr;
@@ -542,7 +543,7 @@ int run_forward(ae_workspace* ws, const uint16_t* ids, const int* cu, int B, int
         g.res_beta = E->layers[l - 1].ln2_b;
       }
       KernelTimer kt(ws, st, AE_KERNEL_GEMM_ATTN_OUT);  // and LN1, in the same kernel
-      launch_gemm_ln(g, kAF32QSmooth,
+      launch_gemm_ln(g,
                      ln_args(ws->tmp, ws->hidden, D.ln1_w, D.ln1_b, D.ffn_inter.inv_smooth, ws->act_q, ws->act_scale,
                              nullptr, T),
                      st);
@@ -624,7 +625,7 @@ int run_forward(ae_workspace* ws, const uint16_t* ids, const int* cu, int B, int
                                    ws->hidden_c, ws->tmp_c, nullptr, nullptr);
       const LnArgs l = ln_args(ws->tmp_c, ws->tmp_c, D.ln1_w, D.ln1_b, D.ffn_inter.inv_smooth, ws->act_q_c,
                                ws->act_scale_c, ws->rowmax_g_c, B);
-      launch_gemm_ln(g, kAF32QSmooth, l, st);
+      launch_gemm_ln(g, l, st);
     }
     gemm(D.ffn_inter, B, ws->act_q_c, kAI8, ws->act_scale_c, nullptr, nullptr, nullptr, ws->g_c, kEpiGelu,
          D.ffn_out.inv_smooth, ws->rowmax_g_c);
@@ -698,7 +699,7 @@ int run_forward_replay(ae_workspace* ws, const uint16_t* ids, const int* cu, int
 int grow_workspace(ae_workspace* ws, size_t T, size_t B);
 
 // An embedding call grows the workspace (once) so that the whole request runs in
-// as few device batches as these bounds allow (16 KB of device memory per token).
+// as few device batches as these bounds allow (10 KB of device memory per token).
 constexpr size_t kGrowTokens = size_t(1) << 18;
 constexpr size_t kGrowSeqs = 8192;
 // Batches of at most this many tokens are padded to a bucketed shape (below),
@@ -884,12 +885,13 @@ int alloc_capacity(ae_workspace* ws, size_t T, size_t B) {
     if (rc == AE_OK) ws->dev.push_back(*p);
     return rc;
   };
+  const size_t Ts = std::min(T, size_t(aek::kSmallM));  // only the few-row path holds the FFN's intermediate
   int rc;
   if ((rc = A(&ws->ids, T)) || (rc = A(&ws->cu, B + 1)) || (rc = A(&ws->cu_safe, B + 1)) ||
       (rc = A(&ws->err, size_t(1))) || (rc = A(&ws->attn_plan, aek::attention_plan_ints(int(B), int(T)))) ||
       (rc = A(&ws->hidden, T * 384)) || (rc = A(&ws->tmp, T * 384)) || (rc = A(&ws->qkv, T * 1152)) ||
-      (rc = A(&ws->ctx, T * 384)) || (rc = A(&ws->g, T * 1536)) || (rc = A(&ws->act_q, T * 384)) ||
-      (rc = A(&ws->act_scale, T)) || (rc = A(&ws->rowmax_ctx, T)) || (rc = A(&ws->rowmax_g, T)) ||
+      (rc = A(&ws->ctx, T * 384)) || (rc = A(&ws->g, Ts * 1536)) || (rc = A(&ws->act_q, T * 384)) ||
+      (rc = A(&ws->act_scale, T)) || (rc = A(&ws->rowmax_ctx, T)) || (rc = A(&ws->rowmax_g, Ts)) ||
       (rc = A(&ws->ln2_stats, T)) ||
       (rc = A(&ws->hidden_c, B * 384)) || (rc = A(&ws->tmp_c, B * 384)) ||
       (rc = A(&ws->ctx_c, B * 384)) || (rc = A(&ws->g_c, B * 1536)) || (rc = A(&ws->out_c, B * 384)) ||
@@ -1517,7 +1519,6 @@ int ae_debug_gemm_ln(const ae_linear* l, int m, const float* x_dev, const uint32
   p.w_scale = l->w_scale;
   p.bias = l->bias;
   p.res = res_dev;
-  if (!aek::gemm_fuses_ln(p, aek::kAF32QSmooth)) return fail(AE_ERR_INVALID_ARG, "ae_debug_gemm_ln: not fused");
   aek::LnArgs ln{};
   ln.T = m;
   ln.gamma = gamma_dev;
@@ -1526,7 +1527,7 @@ int ae_debug_gemm_ln(const ae_linear* l, int m, const float* x_dev, const uint32
   ln.dst = dst_dev;
   ln.q = q_dev;
   ln.scale = scale_dev;
-  aek::launch_gemm_ln(p, aek::kAF32QSmooth, ln, as_stream(stream));
+  aek::launch_gemm_ln(p, ln, as_stream(stream));
   HIP_TRY(hipGetLastError());
   return AE_OK;
 }

@@ -1084,7 +1084,6 @@ __global__ __launch_bounds__(512) void gemm_small_kernel(GemmArgs p, LnArgs ln, 
 }
 
 // Up to this many rows (and K <= kSmallMaxK) the GEMMs take gemm_small_kernel.
-constexpr int kSmallM = 1024;
 
 // compute units of the current device (cached per device; 256 on MI355X)
 int device_cu_count() {
@@ -1144,15 +1143,9 @@ bool gemm_int8_rows16(int m, int n, int k, bool res, int cus) {
 // 32-row workgroups of 4 waves, which take 8 there now.
 static bool ln_rows16(const GemmArgs& p) { return small_gemm(p) || (p.M + 15) / 16 <= device_cu_count(); }
 
-// ln != null: N = 384, kEpiF32, K <= kSmallMaxK, ln_rows16(p); the epilogue
-// applies *ln to each output row and p.out is not written
 template <int AM, int EM>
-static void launch_variant(GemmArgs p, hipStream_t st, const LnArgs* ln = nullptr) {
+static void launch_variant(GemmArgs p, hipStream_t st) {
   const int mt16 = (p.M + 15) / 16;
-  if (ln) {
-    hipLaunchKernelGGL((gemm_small_kernel<AM, kEpiF32, true, 1>), dim3(mt16), dim3(512), 0, st, p, *ln, PreArgs{});
-    return;
-  }
   if (small_gemm(p) ||
       (AM == kAI8 && EM == kEpiF32 && gemm_int8_rows16(p.M, p.N, p.K, p.res != nullptr, device_cu_count()))) {
     if (EM == kEpiF32 && p.K >= kSplitMinK && p.K % 512 == 0) {
@@ -1186,14 +1179,6 @@ static void launch_variant(GemmArgs p, hipStream_t st, const LnArgs* ln = nullpt
   const int nbase = ((p.M + 63) / 64) * (p.N / 192);
   hipLaunchKernelGGL((gemm_w8a8_kernel<AM, EM, 48>), dim3(nbase), dim3(256), 0, st, p);
 }
-
-// the GEMM and the LayerNorm of its output in one kernel: few rows (any A mode,
-// N = 384), or many rows of the attention output GEMM (kAF32QSmooth, N = K = 384)
-bool gemm_fuses_ln(const GemmArgs& p, int amode) {
-  return p.M > 0 && p.N == 384 && (small_gemm(p) || (amode == kAF32QSmooth && p.K == 384 && p.res));
-}
-
-bool gemm_small_path(int m) { return m > 0 && m <= kSmallM; }
 
 // A workgroup with a LayerNorm in front (up to 216 VGPRs, 8 waves) has a compute
 // unit to itself, and most of its time is that LayerNorm, whatever its columns.
@@ -1229,31 +1214,23 @@ void launch_gemm_pre_ln(const GemmArgs& p, const PreArgs& pre, const LnArgs& ln,
                        ln, pre);
 }
 
-void launch_gemm_ln(const GemmArgs& p, int amode, const LnArgs& ln, hipStream_t st) {
-  if (p.M <= 0) return;
-  if (!gemm_fuses_ln(p, amode)) {  // the GEMM, then the LayerNorm kernel over its output
-    launch_gemm(p, amode, kEpiF32, st);
-    LnArgs l = ln;
-    l.src = p.out;
-    launch_ln_quant(l, kLnSrcF32, st);
+void launch_gemm_ln(const GemmArgs& p, const LnArgs& ln, hipStream_t st) {
+  if (p.M <= 0 || p.N != 384 || p.K != 384 || !p.res) return;
+  if (ln_rows16(p)) {
+    hipLaunchKernelGGL((gemm_small_kernel<kAF32QSmooth, kEpiF32, true, 1>), dim3((p.M + 15) / 16), dim3(512), 0, st, p,
+                       ln, PreArgs{});
     return;
   }
-  if (!ln_rows16(p)) {  // many rows: kAF32QSmooth, N = K = 384, with residual
-    // 8 waves (114 VGPRs, two workgroups per CU) halve every phase but the in-order
-    // sums, 4 waves (165, three per CU) hide one another's latency in several
-    // rounds: 8 while they run in one round, 16,384 rows.  Passes with 4 / 8 waves:
-    // 4,500 rows 942 / 891 us, 8,190 rows 1,094 / 1,041, 16,380 rows 1,629 / 1,586,
-    // 24,000 rows 2,294 / 2,351, 33,000 rows 3,572 / 3,534, 66,000 rows 6,163 / 6,168.
-    const int wgs = (p.M + kLrRows - 1) / kLrRows;
-    if (wgs <= 2 * device_cu_count())
-      hipLaunchKernelGGL(gemm_ln_rows_kernel<8>, dim3(wgs), dim3(512), 0, st, p, ln);
-    else
-      hipLaunchKernelGGL(gemm_ln_rows_kernel<4>, dim3(wgs), dim3(256), 0, st, p, ln);
-    return;
-  }
-  if (amode == kAI8) launch_variant<kAI8, kEpiF32>(p, st, &ln);
-  else if (amode == kAF32Q) launch_variant<kAF32Q, kEpiF32>(p, st, &ln);
-  else if (amode == kAF32QSmooth) launch_variant<kAF32QSmooth, kEpiF32>(p, st, &ln);
+  // 8 waves (114 VGPRs, two workgroups per CU) halve every phase but the in-order
+  // sums, 4 waves (165, three per CU) hide one another's latency in several
+  // rounds: 8 while they run in one round, 16,384 rows.  Passes with 4 / 8 waves:
+  // 4,500 rows 942 / 891 us, 8,190 rows 1,094 / 1,041, 16,380 rows 1,629 / 1,586,
+  // 24,000 rows 2,294 / 2,351, 33,000 rows 3,572 / 3,534, 66,000 rows 6,163 / 6,168.
+  const int wgs = (p.M + kLrRows - 1) / kLrRows;
+  if (wgs <= 2 * device_cu_count())
+    hipLaunchKernelGGL(gemm_ln_rows_kernel<8>, dim3(wgs), dim3(512), 0, st, p, ln);
+  else
+    hipLaunchKernelGGL(gemm_ln_rows_kernel<4>, dim3(wgs), dim3(256), 0, st, p, ln);
 }
 
 void launch_gemm(const GemmArgs& p, int amode, int emode, hipStream_t st) {

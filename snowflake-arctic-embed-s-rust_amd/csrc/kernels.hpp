@@ -32,8 +32,7 @@ struct GemmArgs {
   const float* g_smooth;      // kEpiGelu: next layer inv_smooth [N]
   uint32_t* g_rowmax;         // kEpiGelu: [M], pre-set to bits(1e-8f)
   int col_fast;               // set by launch_gemm: workgroup order (column tile fastest)
-  // launch_gemm_ln only, in a call that gemm_fuses_ln holds for: res holds a LayerNorm's input rows, and the residual is
-  // that LayerNorm's output, recomputed as ((res - mean) * rstd) * res_gamma +
+  // launch_gemm_ln only: res holds a LayerNorm's input rows, and the residual is that LayerNorm's output, recomputed as ((res - mean) * rstd) * res_gamma +
   // res_beta from its (mean, rstd) per row
   const float2* res_stats = nullptr;
   const float* res_gamma = nullptr;
@@ -87,7 +86,7 @@ bool ffn_exact_gelu();
 hipError_t ffn_repair_counts(unsigned long long counts[2], bool reset);
 // the exhaustive check of gelu_fast against gelu_exact (6 counters at out_dev, device memory)
 hipError_t gelu_fast_certify(unsigned long long* out_dev, hipStream_t st);
-// token rows per FFN workgroup, process-wide (a test hook): 0 by the batch (default), 32 or 64
+// token rows per FFN workgroup, process-wide (a test hook): 0 by the batch (default), 16, 32, 64 or -m
 void set_ffn_rows(int rows);
 int ffn_rows();  // the current setting
 // compute units of the current device (cached per device)
@@ -136,13 +135,10 @@ void launch_ln_quant(const LnArgs& p, int src_mode, hipStream_t st);
 // given cs index rows inside [0, T) whatever cu held.
 void launch_sanitize_segments(const int* cu, int B, int T, int max_len, bool strict, int* err, int* cs,
                               hipStream_t st);
-// An N = 384 GEMM (kEpiF32) followed by the LayerNorm + SmoothQuant of its
-// output rows (ln.src is ignored: the GEMM output).  When gemm_fuses_ln(p, amode)
-// (few rows, or the many-row attention output GEMM: kAF32QSmooth, K = 384, with
-// residual) the LayerNorm runs in the GEMM's kernel and p.out is not written;
-// otherwise the GEMM writes p.out and launch_ln_quant reads it.
-void launch_gemm_ln(const GemmArgs& p, int amode, const LnArgs& ln, hipStream_t st);
-bool gemm_fuses_ln(const GemmArgs& p, int amode);
+// The attention output GEMM (kAF32QSmooth, N = K = 384, with residual) and the
+// LayerNorm + SmoothQuant of its output rows in one kernel (ln.src is ignored, p.out
+// is not written).
+void launch_gemm_ln(const GemmArgs& p, const LnArgs& ln, hipStream_t st);
 // Few rows (gemm_small_path): a GEMM whose A operand is the LayerNorm + SmoothQuant
 // of the f32 rows p.A (K = 384) under `ln` (gamma, beta, smooth), applied in each
 // workgroup's prologue; the workgroups of the first column tile also store the
@@ -166,7 +162,8 @@ struct PreArgs {
 // FFN-up GEMM): one kernel instead of two.  ln.dst must not alias pre.res or pre.A.
 void launch_gemm_pre_ln(const GemmArgs& p, const PreArgs& pre, const LnArgs& ln, hipStream_t st);
 // whether launch_gemm takes the few-rows kernels for m rows (and the prologue form applies)
-bool gemm_small_path(int m);
+constexpr int kSmallM = 1024;
+inline bool gemm_small_path(int m) { return m > 0 && m <= kSmallM; }
 // whether an int8-A GEMM (kEpiF32, m rows beyond the few-rows path, K = k) keeps the
 // 16-row workgroups on a GPU of cus compute units
 bool gemm_int8_rows16(int m, int n, int k, bool res, int cus);
