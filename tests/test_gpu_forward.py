@@ -1,7 +1,7 @@
 """End-to-end parity of the device forward pass (through the C ABI) against the
 oracle's restatement of forward_cls / embed_batch.
 
-Bar (BASELINE north_star): per embedding cosine >= 0.99999 and max |diff| <= 1e-4
+Bar: per embedding cosine >= 0.99999 and max |diff| <= 1e-4
 against the oracle.  Every kernel reproduces the reference's scalar evaluation
 order (test_gpu_kernels.py), so the device forward is in fact bit-identical to
 the oracle, and these tests assert that too.  Bit-exactness is also what the
@@ -346,7 +346,7 @@ def oracle_threads():
 
 @pytest.mark.parametrize("cfg", ["c3", "c4", "c5"])
 def test_full_size_configs(engine, oracle_model, cfg):
-    """BASELINE configs[2..4] at full size in one packed device batch each: every row of C3
+    """The large workloads at full size in one packed device batch each: every row of C3
     (256 x 16-512) and C4 (64 x 512), and 512 random rows of C5 (8192 x 8-64), bit-identical to
     the oracle (its embed_batch over the host's cores); unit norm and finite on every row."""
     seqs = {"c3": lambda: ragged_batch(256, 16, 512, 3), "c4": lambda: ragged_batch(64, 512, 512, 4),
@@ -568,8 +568,16 @@ _BAD_CU = {
 }
 
 
+@pytest.fixture(params=[0, 1], ids=["by_shape", "tiles32"])
+def attention_form(request, torch_gpu):
+    """The attention kernels that a small batch's shape selects, and the planned 32-query tiles."""
+    ae.set_attention_form(request.param)
+    yield request.param
+    ae.set_attention_form(0)
+
+
 @pytest.mark.parametrize("quantized", [False, True], ids=["exact", "quantized"])
-def test_device_batch_out_of_range_cu_seqlens(engine, oracle_model, torch_gpu, quantized):
+def test_device_batch_out_of_range_cu_seqlens(engine, oracle_model, torch_gpu, quantized, attention_form):
     """A device-resident cu_seqlens outside [0, total_tokens], non-monotone, with an empty or an
     over-long segment: the first kernel of the pass checks it and every later kernel reads the
     checked copy (B one-token segments after a bad one), so the pass stays inside the workspace's
@@ -606,7 +614,7 @@ def test_device_batch_out_of_range_cu_seqlens(engine, oracle_model, torch_gpu, q
     w.close()
 
 
-def test_attention_operators_out_of_range_cu_seqlens(engine, torch_gpu):
+def test_attention_operators_out_of_range_cu_seqlens(engine, torch_gpu, attention_form):
     """The workspace attention operators report a bad cu_seqlens at the next synchronize and the
     no-allocation operator returns (values unspecified); neither reads or writes outside the
     batch's rows: a guard region after qkv and ctx keeps its bits, and a good call afterwards

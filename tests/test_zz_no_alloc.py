@@ -15,20 +15,29 @@ def _call(lib, qkv, cu, n, t, max_len, ctx):
                                            ctypes.c_void_p(ctx), None)
 
 
-def test_noalloc_attention_matches_allocating_operator(torch_gpu):
+@pytest.fixture(params=[0, 1], ids=["by_shape", "tiles32"])
+def form(request, torch_gpu):
+    """By their shapes all but the last set take kernels without a plan; forced, the 32-query tiles."""
+    ae.set_attention_form(request.param)
+    yield request.param
+    ae.set_attention_form(0)
+
+
+def test_noalloc_attention_matches_allocating_operator(torch_gpu, form):
     """Bit-identical to ae_attention_varlen on consecutive calls through every kernel form.  The
-    static plan keeps the last call's records, so each call must rewrite what it reads: after the
-    first (tiled, split into two lists) set come the latency form and the short-row kernels, then
+    static plan keeps the last call's records, so each call must rewrite what it reads: with the
+    tiles forced, after the first (split into two lists) set come the short-row kernels, then
     smaller tiled sets with fewer segments and tiles, a split set and a non-split set after it."""
     torch = torch_gpu
     lib = ae.lib()
     rng = np.random.default_rng(7)
     for lens in ([130, 512, 7, 64, 1, 300, 33, 257],  # tiled, split (max > 400, mean <= 448): 46 tiles
-                 [100, 3, 70, 9],  # 16 tiles: latency form
+                 [100, 3, 70, 9],  # 8 tiles
                  [40, 2, 17],  # max_len <= 64: short-row kernel
                  [200, 90, 150, 77, 120],  # tiled, one list: 22 tiles
                  [450, 20, 66],  # tiled, split: 19 tiles
-                 [300, 250, 100]):  # tiled, one list after a split call
+                 [300, 250, 100],  # tiled, one list after a split call
+                 [96] * 3 + [15] * 14):  # 17 segments: the plan for 16-query tiles too
         cu = np.concatenate([[0], np.cumsum(lens)]).astype(np.int32)
         T = int(cu[-1])
         print("noalloc attention lens", lens, flush=True)
