@@ -1,13 +1,13 @@
 """Benchmark of the MI355X W8A8 arctic-embed-s forward pass (one GPU).
 
-A step is one device forward pass over one token-packed batch of BASELINE
-configs[2] (256 sequences, lengths U{16..512} with [CLS]/[SEP], ids U[1000,30522),
-seed 3) on the seeded synthetic model.  Inputs are resident in HBM
+A step is one device forward pass over one token-packed batch (256 sequences,
+lengths U{16..512} with [CLS]/[SEP], ids U[1000,30522), seed 3) on the seeded
+synthetic model.  Inputs are resident in HBM
 before the timed region; `value` is embeddings/s over exactly --steps passes.
 
 Also reported: per-kernel device time (HIP events on the workspace stream over
-the timed region) and the roofline of the dominant kernel, ms/seq at 128 tokens
-(configs[0]), the end-to-end roofline (the sum over launches of each kernel's
+the timed region) and the roofline of the dominant kernel, ms/seq at 128 tokens,
+the end-to-end roofline (the sum over launches of each kernel's
 ideal time against the measured pass), and the CPU baseline: the oracle's
 restatement of the reference's best x86 backend (AVX-VNNI, else AVX2) under the
 reference's embed_batch policy on the host's cores.
@@ -25,7 +25,7 @@ import numpy as np
 ROOT = os.path.dirname(os.path.abspath(__file__))
 sys.path.insert(0, os.path.join(ROOT, "snowflake-arctic-embed-s-rust_amd"))
 
-METRIC = json.load(open(os.path.join(ROOT, "BASELINE.json")))["metric"]
+METRIC = "embeddings/sec @ ragged 16\u2013512-tok batch; int8 MFMA % of peak; ms/seq @128"
 MODEL_SEED = 0xAE85EED
 PEAK_INT8_TOPS = 5000.0    # MI355X dense int8 MFMA
 PEAK_FP32_TFLOPS = 157.3   # MI355X dense fp32 MFMA
@@ -133,7 +133,7 @@ def host_cpu():
 
 
 def gemm_microbench(ae, torch, iters):
-    """standalone W8A8 GEMM, f32 output + bias, through the C ABI."""
+    """The standalone W8A8 GEMM, f32 output + bias, through the C ABI."""
     rng = np.random.default_rng(2)
     rows = []
     for (k, n) in [(384, 1152), (384, 384), (384, 1536), (1536, 384)]:
@@ -195,12 +195,12 @@ def main():
     ap.add_argument("--no-c1", action="store_true", help="skip the 128-token latency measurement")
     ap.add_argument("--no-quantized", action="store_true", help="skip the quantized-attention mode pass")
     ap.add_argument("--no-embed-batch", action="store_true", help="skip the host-to-host embed_batch measurement")
-    ap.add_argument("--gemm", action="store_true", help="run only the configs[1] GEMM microbench")
+    ap.add_argument("--gemm", action="store_true", help="run only the standalone GEMM microbench")
     ap.add_argument("--calib-copy-mib", type=int, default=0,
                     help="run one plain device copy of this many MiB first (calibrates rocprofv3 byte counters)")
     args = ap.parse_args()
     if args.gpus != 1:
-        print("bench.py: this build runs on exactly one GPU (the forward pass is data-parallel over sequences "
+        print("bench.py: runs on exactly one GPU (the forward pass is data-parallel over sequences "
               "with no cross-GPU exchange; --gpus %d is not supported)" % args.gpus, file=sys.stderr)
         sys.exit(2)
 
@@ -288,7 +288,7 @@ def main():
     e2e = {"t_roof_ms": round(sum(roof.values()), 4), "t_measured_ms": round(ms_per_step, 4),
            "frac": round(sum(roof.values()) / ms_per_step, 4),
            "per_kernel_frac": {k: round(roof[k] / kernel_ms[k], 4) for k in roof if kernel_ms.get(k)}}
-    # the FFN GEMMs' fraction of dense int8 MFMA peak (BASELINE metric, part 2)
+    # the FFN GEMMs' fraction of dense int8 MFMA peak (the metric's second part)
     ffn = {}
     for k in (("ffn_fused",) if ffn_fused else ("gemm_ffn_up", "gemm_ffn_down")):
         u, a, _, p = kernel_work(k, T, B, lens)
@@ -348,7 +348,7 @@ def main():
               "path": "host ids -> ae_embed_batch_tokens(engine, NULL workspace) -> host embeddings; "
                       "fresh lengths each step; wall clock"}
 
-    # ms/seq @ 128 tokens (BASELINE metric, part 3): single-sequence latency, device-resident input
+    # ms/seq @ 128 tokens (the metric's third part): single-sequence latency, device-resident input
     c1_ms = None
     if not args.no_c1:
         c1 = make_batch(1, 128, 128, 1)[0]
@@ -406,7 +406,7 @@ def main():
         run(sample[:32], threads)
         ref = run(sample, threads)
         cpu_s = median_s(lambda: run(sample, threads), 5)
-        # ms/seq at 128 tokens (configs[0]'s sequence): one thread, and all threads (the reference's
+        # ms/seq at 128 tokens: one thread, and all threads (the reference's
         # embed_batch gives one sequence to one thread, so more threads cannot shorten it); median of 5
         c1seq = make_batch(1, 128, 128, 1)
         run(c1seq, 1)

@@ -253,7 +253,7 @@ int ae_workspace_attention_varlen_quantized(ae_workspace* ws, const float* qkv_d
                                             void* stream);
 
 /* ---- tools and test hooks (no counterpart in the reference) -------------- */
-/* Writes a seeded synthetic model in `.ae8` layout (BASELINE configs[0]: fp32
+/* Writes a seeded synthetic model in `.ae8` layout (fp32
  * N(0,0.02) embeddings stored per-row int8, int8 weights U{-127..127}, scales
  * 0.05/127*U(0.5,1.5), SmoothQuant 1/U(0.5,2), biases N(0,0.02), LN gamma
  * 1+N(0,0.05), beta N(0,0.02); layer 11 carries the Q / KV split).  Host only. */

@@ -135,7 +135,7 @@ def version():
 
 
 def write_synthetic_ae8(path, seed):
-    """Seeded synthetic model in .ae8 layout (BASELINE configs[0])."""
+    """Seeded synthetic model in .ae8 layout."""
     _check(_lib.ae_write_synthetic_ae8(str(path).encode(), int(seed)))
 
 

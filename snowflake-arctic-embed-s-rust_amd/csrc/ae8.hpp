@@ -56,7 +56,7 @@ int load_ae8(const std::string& path, ModelRaw& out, std::string& err);
 // unwraps of layer 11's split, src/model.rs:403-404).
 int validate_model(const ModelRaw& m, std::string& err);
 
-// Seeded synthetic model in `.ae8` layout (BASELINE configs[0]): xoshiro256**
+// Seeded synthetic model in `.ae8` layout: xoshiro256**
 // seeded by SplitMix64, Box-Muller normals in double precision.
 int write_synthetic_ae8(const std::string& path, uint64_t seed, std::string& err);
 

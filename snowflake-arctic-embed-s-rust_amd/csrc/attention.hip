@@ -284,7 +284,7 @@ __device__ __forceinline__ bool half_item(const AttnArgs& p, int tps, int& h, in
 //
 // kWide: operands in float4 groups with four MFMA results live at a time (one
 // float4 load of K per 16 dims, one float4 LDS read of P per 16 keys, and four
-// back-to-back MFMAs before their adds), 160 VGPRs.  Otherwise one MFMA result
+// back-to-back MFMAs before their adds), 156 VGPRs.  Otherwise one MFMA result
 // at a time with scalar operands, 92 VGPRs: for short rows, where the score
 // tile leaves room for more waves than the wide variant's registers do.
 //

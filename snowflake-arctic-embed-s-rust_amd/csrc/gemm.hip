@@ -1180,8 +1180,8 @@ static void launch_variant(GemmArgs p, hipStream_t st) {
   hipLaunchKernelGGL((gemm_w8a8_kernel<AM, EM, 48>), dim3(nbase), dim3(256), 0, st, p);
 }
 
-// A workgroup with a LayerNorm in front (up to 216 VGPRs, 8 waves) has a compute
-// unit to itself, and most of its time is that LayerNorm, whatever its columns.
+// A workgroup with a LayerNorm in front (174 to 182 VGPRs, with 384 columns 224;
+// FFN-up behind attn_out 216 and 242; 8 waves) has a compute unit to itself, and most of its time is that LayerNorm, whatever its columns.
 // So the K split is the largest whose workgroups still run in one round: 48
 // columns each up to 160 rows (N = 1152), 96 up to 336, 192 up to 672, then 384.
 // Passes with 48 / 96 / 192 / 384 columns: 128 rows 411 / 412 / 416 / 427 us,

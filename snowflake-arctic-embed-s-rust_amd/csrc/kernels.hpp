@@ -216,7 +216,7 @@ void launch_attention(const AttnArgs& p, int T, hipStream_t st, bool plan = true
 // attention_lat_kernel.  Every choice gives the same bits.
 enum AttnChoice { kAttnTiles32 = 0, kAttnTiles16 = 1, kAttnLat = 2 };
 int attention_choice(int B, int T, int max_len, int longest, int cus);
-// split = 1: rows of more than 384 keys in the plan's second list
+// split = 1: rows of more than 400 keys in the plan's second list
 void launch_attention_plan(const AttnArgs& p, hipStream_t st, int split, int max_tiles);
 // exact-attention kernel choice for later launches: 0 by the batch, 1 tiled (32 queries) /
 // register rows only, 2 the latency form only (a test hook; same bits)

@@ -39,7 +39,7 @@ def oracle_model(model_dir):
 
 
 def c1_ids():
-    """BASELINE configs[0]: [CLS] + 126 ids U[1000,30522) + [SEP], seed 1."""
+    """[CLS] + 126 ids U[1000,30522) + [SEP], seed 1."""
     rng = np.random.default_rng(1)
     return np.concatenate([[101], rng.integers(1000, 30522, 126), [102]]).astype(np.uint16)
 

@@ -58,7 +58,7 @@ def test_gemm_bit_exact(torch_gpu, n, k, m, with_res):
 @pytest.mark.parametrize("k,n", [(384, 1152), (384, 384), (384, 1536), (1536, 384)])
 @pytest.mark.parametrize("m", [128, 4096, 32768])
 def test_gemm_configs1_microbench_shapes(torch_gpu, m, k, n):
-    """BASELINE configs[1] (the standalone W8A8 GEMM microbench that bench.py --gemm times) at its
+    """The standalone W8A8 GEMM microbench that bench.py --gemm times, at its
     own sizes and distributions: A int8 U[-127,127] with row scales U(0.01,0.1), W [K x N] int8
     U[-127,127] (stored [N,K]) with column scales U(0.0002,0.0006), bias N(0,0.02), f32 out.
     GEMM rows are independent, so every row at M = 128 and 64 rows otherwise (the first and
