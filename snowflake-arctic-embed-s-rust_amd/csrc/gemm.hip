@@ -1114,22 +1114,20 @@ constexpr int kSplitMinK = 1024;
 // each on a few 64 x 192 tiles.  K = 384: one round of them, three per compute
 // unit (N = 1152: 1,280 rows 6.6 -> 5.2 us, 2,048 rows 7.1 -> 6.4, but 2,843 rows
 // 8.2 -> 8.9; N = 1536: 1,536 rows 7.0 -> 6.4, 2,048 rows 7.5 -> 8.1).  K of 1,024
-// and 1,536 (us per call, 64 x 192 tiles / 16-row workgroups; a round is three
-// workgroups per compute unit):
-//  * no residual: two rounds (N = 384, K = 1536: 3,072 rows 13.6 / 11.0, 4,096 rows
-//    14.0 / 13.7, 6,144 rows 14.6 / 18.4; K = 1024: 3,072 rows 10.5 / 9.1, 4,096 rows
-//    10.7 / 11.3; N = 1536, K = 1024: 1,040 rows 11.1 / 12.1, 1,536 rows 11.5 / 16.3);
-//  * a residual, which costs the 64 x 192 tiles 1.5 to 6 us (by where the buffers
-//    lie): four rounds at K = 1536 up to N = 768 (N = 384: 1,280 rows 17.7 / 6.8,
-//    6,144 rows 20.8 / 18.9, 8,192 rows 22.3 / 26.0; N = 768: 3,072 rows 21.9 / 20.1),
-//    else less than three (K = 1024: N = 384, 4,096 rows 13.6 / 11.6, 6,144 rows 14.9
-//    to 17.6 / 15.6 to 16.9; N = 1152, 1,280 rows 15.1 / 11.6, 1,536 rows 12.9 / 13.1).
+// and 1,536, by the workgroups per compute unit (three run at once; medians over 10
+// to 16 placements of the buffers in us, 64 x 192 tiles / 16-row workgroups):
+//  * no residual: up to 7 (K = 1024) or 8 (K = 1536).  N = 384: K = 1024, 3,584 rows
+//    10.4 / 9.9, 3,840 rows 10.5 / 10.8; K = 1536, 4,096 rows 13.6 / 13.1, 4,352 rows
+//    13.9 / 14.2.  N = 1152: K = 1024, 1,184 rows 10.5 / 9.7, 1,280 rows 10.5 / 10.8;
+//  * a residual, which costs the 64 x 192 tiles 2.5 to 9 us (by where the buffers
+//    lie): up to 12.  N = 384: K = 1024, 6,144 rows 17.3 / 15.4; K = 1536, 1,280 rows
+//    17.7 / 6.8, 6,144 rows 19.7 / 18.7, 8,192 rows 22.3 / 26.0.  N = 1152: K = 1024,
+//    1,536 rows 14.8 / 12.2, 2,048 rows 16.6 / 15.6.
 bool gemm_int8_rows16(int m, int n, int k, bool res, int cus) {
   const long mt = (m + 15) / 16;
   if (k == 384) return mt * (n / 192) <= 3L * cus;
   if (k < kSplitMinK || k > kSmallMaxK || k % 512 != 0) return false;
-  const long wgs = mt * (n / 48);
-  return !res ? wgs <= 6L * cus : k == 1536 && n <= 768 ? wgs <= 12L * cus : wgs < 9L * cus;
+  return mt * (n / 48) <= (res ? 12L : k == 1024 ? 7L : 8L) * cus;
 }
 
 // The attention output GEMM with LN1 (kAF32QSmooth, N = K = 384) takes

@@ -81,13 +81,13 @@ def test_attention_choice_by_the_longest_row(n_seqs, tokens, bound, longest, cho
 
 
 @pytest.mark.parametrize("m,n,k,residual,rows16", [
-    # K = 1024 and 1536 without a residual: two rounds of workgroups (slower beyond: 1.06 to 1.42 times)
-    (3072, 384, 1536, False, True), (4096, 384, 1024, False, False), (6144, 384, 1536, False, False),
-    (2048, 768, 1024, False, False), (1536, 1152, 1024, False, False), (1040, 1536, 1024, False, False),
-    # with one: four rounds at K = 1536 up to N = 768, else less than three
-    (6144, 384, 1536, True, True), (6145, 384, 1536, True, False), (3072, 768, 1536, True, True),
-    (4096, 384, 1024, True, True), (5120, 384, 1024, True, False), (2048, 768, 1024, True, True),
-    (1280, 1152, 1024, True, True), (1536, 1152, 1024, True, False), (1536, 1536, 1536, True, False),
+    # K = 1024 and 1536 without a residual: 7 and 8 workgroups per compute unit (slower beyond: up to 1.42 times)
+    (3584, 384, 1024, False, True), (3585, 384, 1024, False, False), (4096, 384, 1536, False, True),
+    (4097, 384, 1536, False, False), (6144, 384, 1536, False, False), (2048, 768, 1024, False, False),
+    (1184, 1152, 1024, False, True), (1536, 1152, 1024, False, False), (1040, 1536, 1024, False, False),
+    # with one: 12
+    (6144, 384, 1536, True, True), (6145, 384, 1536, True, False), (3072, 768, 1024, True, True),
+    (6144, 384, 1024, True, True), (2048, 1152, 1024, True, True), (1537, 1536, 1536, True, False),
     # K = 384: one round, with or without
     (6144, 384, 384, False, True), (2048, 1152, 384, True, True), (2049, 1152, 384, True, False),
     # no K split

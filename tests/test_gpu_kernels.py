@@ -111,7 +111,7 @@ def test_gemm_row_stationary_tiles(torch_gpu, m, n):
 
 
 @pytest.mark.parametrize("m,n,k", [(1025, 384, 384), (2048, 1152, 384), (2049, 1152, 384), (1537, 1536, 384),
-                                   (1025, 384, 1536), (3072, 384, 1536), (3073, 384, 1536), (6144, 384, 1536),
+                                   (1025, 384, 1536), (4096, 384, 1536), (4097, 384, 1536), (6144, 384, 1536),
                                    (6145, 384, 1536), (1100, 768, 1024), (1536, 1152, 1024)])
 @pytest.mark.parametrize("with_res", [False, True])
 def test_gemm_int8_tile_heights(torch_gpu, m, n, k, with_res):
