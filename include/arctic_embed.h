@@ -218,7 +218,8 @@ int ae_attention_varlen_quantized(const float* qkv_dev, const int32_t* cu_seqlen
 /* No counterpart in the reference: ae_attention_varlen for callers that cannot
  * allocate device memory (code under HIP graph capture, tight serving loops,
  * harnesses that forbid hipMalloc).  It allocates nothing, copies nothing to the
- * host and does not synchronize: the caller states max_seq_len (1..512), and
+ * host and does not synchronize: the caller states max_seq_len (1..512; below 512
+ * taken for the longest segment where the kernels are chosen), and
  * cu_seqlens must lie in [0, total_tokens] with segments of 0..max_seq_len
  * tokens.  A cu_seqlens that breaks this gives unspecified values (the call
  * cannot report it) but no access outside the batch's rows: a checked copy of
@@ -238,7 +239,8 @@ int ae_attention_varlen_noalloc(const float* qkv_dev, const int32_t* cu_seqlens_
  * workspace's), no host copy, no synchronization, no allocation (the quantized
  * variant allocates its scratch on its first call, as
  * ae_workspace_set_attention_mode does).  The caller states max_seq_len
- * (1..512), the longest segment; n_seqs and total_tokens within the workspace
+ * (1..512), the longest segment (512 also where it is not known: kernels that need
+ * it are then not chosen); n_seqs and total_tokens within the workspace
  * capacity (AE_ERR_CAPACITY otherwise).  A cu_seqlens that is not an exact
  * prefix sum of segments of 1..max_seq_len tokens is reported by the next
  * ae_workspace_synchronize (its values are then unspecified; every access stays
